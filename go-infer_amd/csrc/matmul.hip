@@ -15,10 +15,14 @@
 //   16t.., columns 32kk..) is 512 elements in lane order, lane
 //   16 * ((c / 8) % 4) + r % 16 holding columns 8 ((c / 8) % 4) .. +7 of its
 //   row (op_index);
-//   activation halves: the same tiles, each row-major (x_index), which the
-//   direct loads permute into lane order;
-//   Q8_0  int8 codes in the same order (512 bytes per tile), fp16 block
-//         scales [cols/32][rows_pad];
+//   activation halves: the same tiles, in lane order (matmul_reg) or
+//   row-major (x_index; matmul_sk's direct loads permute them);
+//   Q8_0  int8 codes in the same order (512 bytes per tile), and per tile the
+//         fp16 block scales of its 16 rows (scale_index), so that a row tile's
+//         scales are one run: row-fastest over the whole matrix, each tile's
+//         32 bytes shared their lines with workgroups of other XCDs, whose
+//         L2s then each fetched them (Q4_0, 8192 x 8192, batch 1: 19.1 -> 17.9
+//         us);
 //   Q4_0  per tile and block, the 16 nibble bytes of each of the 16 rows
 //         (byte j holds elements j and j+16, quant.go:504), 256 bytes;
 //         scales as Q8_0;
@@ -27,25 +31,23 @@
 // Rows of weights are padded with zeros to multiples of 128 and those of
 // activations to multiples of 64, so the product loops need no bounds checks.
 //
-// Activations are split per batch row into fp16 hi + lo of x * 2^e[b], so the
-// products keep float32 accuracy.  The matrix cores then compute W * x^T on
-// 16x16x32 f16 tiles: quantised codes are exact fp16 values, and one 32-wide
-// k-step is exactly one quantisation block, so each k-step's partial product
-// is scaled by its block scale in float32 (DotVecQ8_0 / DotVecQ4_0 sum a
-// block, then multiply by d).  F32 weights take three products (hi*hi, hi*lo,
-// lo*hi).
+// Activations are split into fp16 hi + lo of x * 2^e, e per batch row and
+// range of k-steps, so the products keep float32 accuracy.  The matrix cores
+// then compute W * x^T on 16x16x32 f16 tiles: quantised codes are exact fp16
+// values, and one 32-wide k-step is exactly one quantisation block, so each
+// k-step's partial product is scaled by its block scale in float32
+// (DotVecQ8_0 / DotVecQ4_0 sum a block, then multiply by d).  F32 weights take
+// three products (hi*hi, hi*lo, lo*hi).
 //
-// Two forms of the product:
-//   * matmul_lds (quantised weights, and batches under 128): a workgroup owns
-//     a 64 x 64 (rows x batch) output tile.  Its four waves take every fourth
-//     k-step each, and each wave streams its k-steps through its own LDS
-//     stages by direct global->LDS loads, two steps ahead (one for F32, whose
-//     stages are twice as large).  Waves 1-3 then leave their partial tiles
-//     in LDS and wave 0 adds them to its own, so one launch covers the
-//     product with no global reduction.
-//   * matmul_sk (F16 and F32 weights, batches of 128 and more): 128 x 128
-//     tiles over slices of the k-steps, the slices' partial tiles added by
-//     reduce_splits (described at the kernel).
+// Three forms of the product, each described at its kernel:
+//   * matmul_vec (batches of up to 16): bound by the weights' bytes and by
+//     latency; one launch that splits x itself;
+//   * matmul_reg (larger batches): 16 .. 64 x 32 / 64 tiles, the k-steps
+//     divided over the waves of a workgroup, operands straight into registers;
+//     split_x runs first;
+//   * matmul_sk (F16 and F32 weights, large products): 128 x 128 tiles over
+//     slices of the k-steps through LDS, the slices' partial tiles added by
+//     reduce_splits; split_rows runs first.
 #include "../../include/goinfer_paged.h"
 #include "gi_common.h"
 #include "devbuf.h"
@@ -62,6 +64,7 @@
 namespace gi {
 namespace {
 
+typedef __attribute__((address_space(3))) void *lds_void;
 using mfma_ops::f4;
 using mfma_ops::h8;
 using mfma_ops::i8x8_to_h8;
@@ -86,13 +89,19 @@ __host__ __device__ __forceinline__ int64_t op_index(int64_t r, int c, int KS)
     return (((r >> 4) * KS + (c >> 5)) * 64 + 16 * ((c >> 3) & 3) + (r & 15)) * 8 + (c & 7);
 }
 
-// Element (b, c) of the activation halves: each 16 x 32 tile row-major
+// Element (b, c) of the split-K form's activation halves: each 16 x 32 tile row-major
 // (16 rows of 64 bytes), so that one batch row's k-step is one 64-byte run
 // when it is written.  The direct loads read a tile's 1 KiB whole and permute
 // it into lane order (operand order) on the way into LDS.
 __host__ __device__ __forceinline__ int64_t x_index(int64_t b, int c, int KS)
 {
     return (((b >> 4) * KS + (c >> 5)) * 16 + (b & 15)) * 32 + (c & 31);
+}
+
+// The scale of row r's quantisation block kk.
+__host__ __device__ __forceinline__ int64_t scale_index(int64_t r, int kk, int KS)
+{
+    return ((r >> 4) * KS + kk) * 16 + (r & 15);
 }
 
 // Byte i of row r's Q4_0 block kk.
@@ -117,7 +126,7 @@ __global__ __launch_bounds__(256) void convert_quant(const uint8_t *__restrict__
     const bool live = r < rows;
     const int bb = type == W_Q8_0 ? 34 : 18;
     const uint8_t *blk = raw + (live ? i : 0) * bb;
-    scales[(int64_t)kb * rows_pad + r] = live ? (uint16_t)(blk[0] | (blk[1] << 8)) : 0;
+    scales[scale_index(r, kb, nb)] = live ? (uint16_t)(blk[0] | (blk[1] << 8)) : 0;
     if (type == W_Q8_0) {
         for (int j = 0; j < 32; j++)
             codes[op_index(r, 32 * kb + j, nb)] = live ? blk[2 + j] : 0;
@@ -181,8 +190,9 @@ __global__ __launch_bounds__(256) void convert_f32(const float *__restrict__ raw
         row_scale[r] = ldexpf(1.0f, -e);
 }
 
-// ---- activations: x * 2^e split into hi + lo per batch row ---------------
+// ---- activations: x * 2^e split into hi + lo -----------------------------------
 
+// For the split-K form: one power of two per batch row.
 // One workgroup per padded batch row (rows past the batch are zeros); each
 // thread takes runs of 8 columns, so the halves go out as 16-byte stores,
 // four of them one 64-byte run of a tile (x_index).
@@ -256,6 +266,89 @@ __global__ __launch_bounds__(256) void split_rows(const float *__restrict__ x, i
         xscale[b] = ldexpf(1.0f, -e);
 }
 
+// For matmul_reg: each wave of a workgroup takes one contiguous segment of the
+// k-steps (seg_steps of them), and x is scaled per (batch row, segment), so
+// that a wave's sums carry one power of two per column.
+constexpr int kRegWaves = 8, kRegWorkgroups = 256;
+__host__ __device__ __forceinline__ int seg_steps(int KS) { return (KS + kRegWaves - 1) / kRegWaves; }
+
+// One workgroup per (16 batch rows, segment): the rows' largest magnitudes
+// over the segment, then the halves in operand order (op_index), whole tiles
+// at a time: lane r of 16 holds row r, so 16 lanes write one 256-byte run.
+// xscale[segment][batch_pad] = 2^-e.  Rows past the batch are zeros.
+__global__ __launch_bounds__(256) void split_x(const float *__restrict__ x, int batch, int batch_pad, int cols,
+                                              _Float16 *__restrict__ xh, _Float16 *__restrict__ xl,
+                                              float *__restrict__ xscale)
+{
+    __shared__ float s_max[4][16];
+    const int KS = cols / 32, per = seg_steps(KS), seg = blockIdx.y;
+    const int r = threadIdx.x & 15, q0 = threadIdx.x >> 4, b = blockIdx.x * 16 + r;
+    const int first = 4 * per * seg, runs = max(0, min(4 * per, cols / 8 - first)); // runs of 8 columns
+    const float *xr = x + (int64_t)min(b, batch - 1) * cols + 8 * (int64_t)first;
+    // a thread's first KEEP runs stay in registers between the two passes
+    // (all of them for rows up to 8192 columns)
+    constexpr int KEEP = 8;
+    f4 ku[KEEP], kv[KEEP];
+    float m = 0.0f;
+    auto top = [&](const f4 &u, const f4 &v) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            m = fmaxf(m, fmaxf(fabsf(u[i]), fabsf(v[i])));
+    };
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) {
+        const int q = q0 + 16 * k;
+        ku[k] = kv[k] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (q < runs && b < batch) {
+            ku[k] = *reinterpret_cast<const f4 *>(xr + 8 * q);
+            kv[k] = *reinterpret_cast<const f4 *>(xr + 8 * q + 4);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < KEEP; k++)
+        top(ku[k], kv[k]);
+    if (b < batch)
+        for (int q = q0 + 16 * KEEP; q < runs; q += 16)
+            top(*reinterpret_cast<const f4 *>(xr + 8 * q), *reinterpret_cast<const f4 *>(xr + 8 * q + 4));
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    if ((threadIdx.x & 48) == 0)
+        s_max[threadIdx.x >> 6][r] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(s_max[0][r], s_max[1][r]), fmaxf(s_max[2][r], s_max[3][r]));
+    const int e = pow2_exponent_for(m);
+    const float up = ldexpf(1.0f, e);
+    auto emit = [&](int q, const f4 &u, const f4 &v) __attribute__((always_inline)) {
+        h8 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const float t = (k < 4 ? u[k] : v[k - 4]) * up; // exact: a power of two
+            const _Float16 h = (_Float16)t;
+            hi[k] = h;
+            lo[k] = (_Float16)(t - (float)h);
+        }
+        const int64_t o = op_index(b, 8 * (first + q), KS);
+        *reinterpret_cast<h8 *>(xh + o) = hi;
+        *reinterpret_cast<h8 *>(xl + o) = lo;
+    };
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) {
+        const int q = q0 + 16 * k;
+        if (q < runs)
+            emit(q, ku[k], kv[k]);
+    }
+    for (int q = q0 + 16 * KEEP; q < runs; q += 16) {
+        f4 u = f4{0.0f, 0.0f, 0.0f, 0.0f}, v = u;
+        if (b < batch) {
+            u = *reinterpret_cast<const f4 *>(xr + 8 * q);
+            v = *reinterpret_cast<const f4 *>(xr + 8 * q + 4);
+        }
+        emit(q, u, v);
+    }
+    if (threadIdx.x < 16)
+        xscale[(int64_t)seg * batch_pad + b] = ldexpf(1.0f, -e);
+}
+
 // ---- the product -----------------------------------------------------------
 
 struct MatArgs {
@@ -264,205 +357,19 @@ struct MatArgs {
     int rows_pad;           // rows padded to a multiple of 128
     const uint8_t *a;      // F16 / F32-hi / Q8 codes / Q4 nibble bytes
     const uint8_t *a_lo;   // F32 lo
-    const uint16_t *scales; // Q8 / Q4 block scales [cols/32][rows_pad]
+    const uint16_t *scales; // Q8 / Q4 block scales (scale_index)
     const float *row_scale; // F32
     const _Float16 *xh, *xl;
     const float *xscale;
     float *y;
 };
 
-// One wave's operands of one k-step, as the direct loads lay them down: the
-// four batch tiles' hi and lo halves (1 KiB each), the four weight tiles
-// (F16 1 KiB, F32 hi then lo, Q8_0 512 B, Q4_0 256 B), and for Q8_0 / Q4_0
-// the 64 rows' block scales.
-template <int WT>
-struct MStage {
-    static constexpr int XB = 8 * 1024;
-    static constexpr int WB = WT == W_F32 ? 8192 : WT == W_F16 ? 4096 : WT == W_Q8_0 ? 2048 : 1024;
-    static constexpr int SB = (WT == W_Q8_0 || WT == W_Q4_0) ? 128 : 0;
-    static constexpr int BYTES = XB + WB + SB;
-    // direct loads per k-step: 8 activation tiles, the weight tiles, the scales
-    static constexpr int NL = 8 + (WT == W_F32 ? 8 : 4) + (SB ? 1 : 0);
-};
-
-typedef __attribute__((address_space(3))) void *lds_void;
-
-template <int WT, int NST>
-__global__ __launch_bounds__(256) void matmul_lds(MatArgs a)
+// Lane I of this lane's row of 16.
+template <int I>
+__device__ __forceinline__ uint32_t row_lane(uint32_t x)
 {
-    typedef MStage<WT> M;
-    constexpr int STAGE_ALL = 4 * NST * M::BYTES, ACC = 3 * 64 * 65 * 4;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[STAGE_ALL > ACC ? STAGE_ALL : ACC];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int j = lane & 15, g = lane >> 4;
-    const int b0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
-    const int C = a.cols, R = a.rows, KS = C / 32;
-    const int64_t rt0 = r0 / 16, bt0 = b0 / 16;
-    f4 acc[4][4];
-#pragma unroll
-    for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-        for (int bs = 0; bs < 4; bs++)
-            acc[rs][bs] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    uint8_t *mine = smem + w * NST * M::BYTES;
-    // This wave's k-steps are w, w + 4, ...: nk of them.
-    const int nk = w < KS ? (KS - w + 3) / 4 : 0;
-    // The NL direct loads of this wave's i-th k-step (clamped to its last,
-    // so every call issues the same number of loads) into stage st.
-    auto issue = [&](int i, int st) {
-        const int kk = w + 4 * min(i, nk - 1);
-        uint8_t *d = mine + st * M::BYTES;
-#pragma unroll
-        for (int bs = 0; bs < 4; bs++) {
-            // lane (j, g) fetches row j's k-elements 8g .. 8g+7 of the tile
-            const int64_t o = ((bt0 + bs) * KS + kk) * 512 + 32 * j + 8 * g;
-            __builtin_amdgcn_global_load_lds(a.xh + o, (lds_void)(d + 2048 * bs), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds(a.xl + o, (lds_void)(d + 2048 * bs + 1024), 16, 0, 0);
-        }
-        d += M::XB;
-#pragma unroll
-        for (int rs = 0; rs < 4; rs++) {
-            const int64_t t = (rt0 + rs) * KS + kk;
-            if (WT == W_F16 || WT == W_F32) {
-                __builtin_amdgcn_global_load_lds(a.a + t * 1024 + 16 * lane, (lds_void)(d + 1024 * rs), 16, 0, 0);
-                if (WT == W_F32)
-                    __builtin_amdgcn_global_load_lds(a.a_lo + t * 1024 + 16 * lane, (lds_void)(d + 4096 + 1024 * rs),
-                                                     16, 0, 0);
-            } else {
-                constexpr int TB = WT == W_Q8_0 ? 512 : 256; // bytes of one weight tile
-                if (lane < TB / 16)
-                    __builtin_amdgcn_global_load_lds(a.a + t * TB + 16 * lane, (lds_void)(d + TB * rs), 16, 0, 0);
-            }
-        }
-        if (M::SB && lane < 8)
-            __builtin_amdgcn_global_load_lds(a.scales + (int64_t)kk * a.rows_pad + r0 + 8 * lane,
-                                             (lds_void)(d + M::WB), 16, 0, 0);
-    };
-    if (nk > 0) {
-#pragma unroll
-        for (int i = 0; i < NST - 1; i++)
-            issue(i, i);
-        for (int i = 0; i < nk; i++) {
-            issue(i + NST - 1, (i + NST - 1) % NST);
-            // this k-step's loads are done once no more than the later
-            // stages' remain in flight
-            constexpr int VM = (NST - 1) * M::NL;
-            __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8));
-            const uint8_t *sp = mine + (i % NST) * M::BYTES;
-            h8 bh[4], bl[4];
-#pragma unroll
-            for (int bs = 0; bs < 4; bs++) {
-                bh[bs] = *reinterpret_cast<const h8 *>(sp + 2048 * bs + 16 * lane);
-                bl[bs] = *reinterpret_cast<const h8 *>(sp + 2048 * bs + 1024 + 16 * lane);
-            }
-            const uint8_t *wp = sp + M::XB;
-#pragma unroll
-            for (int rs = 0; rs < 4; rs++) {
-                if (WT == W_F16 || WT == W_F32) {
-                    const h8 ah = *reinterpret_cast<const h8 *>(wp + 1024 * rs + 16 * lane);
-                    h8 al = {};
-                    if (WT == W_F32)
-                        al = *reinterpret_cast<const h8 *>(wp + 4096 + 1024 * rs + 16 * lane);
-#pragma unroll
-                    for (int bs = 0; bs < 4; bs++) {
-                        acc[rs][bs] = mfma16(ah, bh[bs], acc[rs][bs]);
-                        acc[rs][bs] = mfma16(ah, bl[bs], acc[rs][bs]);
-                        if (WT == W_F32)
-                            acc[rs][bs] = mfma16(al, bh[bs], acc[rs][bs]);
-                    }
-                } else {
-                    const h8 aq = WT == W_Q8_0
-                                      ? i8x8_to_h8(*reinterpret_cast<const u2 *>(wp + 512 * rs + 8 * lane))
-                                      : u4x8_to_h8(*reinterpret_cast<const u2 *>(wp + 256 * rs + 16 * j + 8 * (g & 1)),
-                                                   (g & 2) ? 4 : 0);
-                    const u2 sw = *reinterpret_cast<const u2 *>(wp + M::WB + (16 * rs + 4 * g) * 2);
-                    const uint32_t s01 = sw.x, s23 = sw.y;
-                    float d[4];
-                    d[0] = (float)__builtin_bit_cast(_Float16, (uint16_t)(s01 & 0xFFFFu));
-                    d[1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(s01 >> 16));
-                    d[2] = (float)__builtin_bit_cast(_Float16, (uint16_t)(s23 & 0xFFFFu));
-                    d[3] = (float)__builtin_bit_cast(_Float16, (uint16_t)(s23 >> 16));
-#pragma unroll
-                    for (int bs = 0; bs < 4; bs++) {
-                        f4 z = mfma16(aq, bh[bs], f4{0.0f, 0.0f, 0.0f, 0.0f});
-                        z = mfma16(aq, bl[bs], z);
-#pragma unroll
-                        for (int r = 0; r < 4; r++)
-                            acc[rs][bs][r] = fmaf(z[r], d[r], acc[rs][bs][r]);
-                    }
-                }
-            }
-        }
-    }
-    // the trailing (unused) loads land before the staging area becomes the
-    // reduction buffer
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    float(*s_acc)[64][65] = reinterpret_cast<float(*)[64][65]>(smem);
-    if (w > 0) {
-#pragma unroll
-        for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-            for (int bs = 0; bs < 4; bs++)
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    s_acc[w - 1][16 * rs + 4 * g + i][16 * bs + j] = acc[rs][bs][i];
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-        for (int rs = 0; rs < 4; rs++)
-#pragma unroll
-            for (int bs = 0; bs < 4; bs++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int rl = 16 * rs + 4 * g + i, bl = 16 * bs + j;
-                    s_acc[0][rl][bl] = acc[rs][bs][i] + s_acc[0][rl][bl] + s_acc[1][rl][bl] + s_acc[2][rl][bl];
-                }
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int bl = e >> 6, rl = e & 63; // rows fastest: coalesced stores
-        const int b = b0 + bl, r = r0 + rl;
-        if (b >= a.batch || r >= R)
-            continue;
-        float v = s_acc[0][rl][bl];
-        v *= a.xscale[b];
-        if (WT == W_F32)
-            v *= a.row_scale[r];
-        a.y[(int64_t)b * R + r] = v;
-    }
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x150 + I, 0xF, 0xF, false); // row_newbcast
 }
-
-// ---- 16-bit weights, batches of 128 and more: split-K ------------------------
-//
-// A workgroup of four waves owns a 128 x 128 (rows x batch) output tile over
-// one of S slices of the k-steps, and two workgroups share a CU.  Wave w
-// takes batch rows 32w .. 32w + 31 of the tile and all 128 rows, so each
-// weight fragment read from LDS feeds four products (two batch tiles, hi and
-// lo) and each activation fragment eight (the row tiles).  Per k-step the
-// eight weight tiles (shared by the waves, each loading two) and every wave's
-// activation halves arrive by direct global->LDS loads two k-steps ahead,
-// through three stages; one barrier per k-step hands a stage from the loads
-// to the products.  The per-CU load volume is 24 KiB per 128 products against
-// 12 KiB per 32 in the 64 x 64 form.  With S > 1 the partial tiles go to a
-// workspace and reduce_splits adds them.  Quantised weights keep the 64 x 64
-// form: their per-block scale multiply-adds need 272 registers here (one
-// wave per SIMD), and measured slower (Q8_0 50.5 against 41.8 us per call
-// at 256 x 4096 x 4096).
-
-struct SKArgs {
-    MatArgs m;
-    int splits;   // S: slices of the k-steps
-    int ks_per;   // k-steps per slice (the last may have fewer)
-    float *part;  // S > 1: partial tiles [S][batch_pad][rows_pad]
-    int batch_pad;
-};
-
-// The split-K form serves batches of at least kSplitKMinBatch rows; its
-// k-step slices give about kSplitKWorkgroups workgroups, none shorter than
-// kMinSliceSteps k-steps.
-constexpr int kSplitKMinBatch = 128, kSplitKWorkgroups = 256, kMinSliceSteps = 4;
 
 template <int N>
 using ic = std::integral_constant<int, N>;
@@ -479,6 +386,254 @@ __device__ __forceinline__ void static_for(F &&f)
 {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
+
+// ---- batches over 16 ---------------------------------------------------------------
+//
+// A workgroup of 8 waves owns 16 RT rows x 16 CT batch columns; wave w takes
+// the w-th segment of the k-steps for the whole tile, its operands straight
+// from memory into registers in lane order, one k-step ahead.  No two waves
+// share an operand, so nothing goes through LDS and nothing synchronises
+// until the eight waves' sums meet at the end; a weight fragment feeds 2 CT
+// products (hi and lo), an activation pair RT.  Tiles are sized so that one
+// round of workgroups covers the CUs: each re-reads its operands from the L2
+// (30 TB/s measured for L2-resident runs of 1 KiB), and consecutive workgroups
+// of an XCD (blockIdx mod 8) take consecutive tiles of one eighth of the rows,
+// so an XCD reads an eighth of the weights.  What bounds it: 10 to 12 KiB of
+// operands per 32 products against a CU's 56 bytes per cycle from the L2, and
+// for quantised weights the scale multiply-adds beside the products.
+//
+// Per call with split_x, 4096 x 4096: batch 32 Q8_0 34.9 -> 15.4 us, F16 34.5
+// -> 17.1; batch 256 Q8_0 39.3 -> 31.5, F16 33.6 -> 31.5; 8192 x 8192, batch
+// 64, Q8_0: 62.8 -> 42.7.  (Before: 64 x 64 tiles staged through LDS by four
+// waves, one per SIMD, on rows / 64 workgroups; F16 at batch 256 matmul_sk.)
+// Weights four k-steps ahead instead of one (tiles of up to 32 rows): Q8_0,
+// batch 32: 17.0 -> 15.4.
+template <int WT, int RT, int CT>
+__global__ __launch_bounds__(64 * kRegWaves) void matmul_reg(MatArgs a, int batch_pad)
+{
+#if __HIP_DEVICE_COMPILE__ // (target builtins inside generic lambdas: not for the host pass)
+    constexpr bool QUANT = WT == W_Q8_0 || WT == W_Q4_0;
+    constexpr int COLS = 16 * CT;
+    __shared__ float red[kRegWaves][16 * RT][COLS + 1];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = lane & 15, g = lane >> 4;
+    // tile index: row tiles major, batch tiles minor; XCD x takes the x-th
+    // eighth of them
+    const int bts = (a.batch + COLS - 1) / COLS, tiles = (a.rows + 16 * RT - 1) / (16 * RT) * bts;
+    const int per_xcd = gridDim.x / 8;
+    const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (tile >= tiles)
+        return;
+    const int r0 = tile / bts * 16 * RT, b0 = tile % bts * COLS;
+    const int KS = a.cols / 32, per = seg_steps(KS);
+    const int k0 = w * per, k1 = min(KS, k0 + per);
+    const int64_t rt0 = r0 / 16, bt0 = b0 / 16;
+    f4 acc[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int c = 0; c < CT; c++)
+            acc[r][c] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    // the operands of one k-step; the weights of tiles of up to 32 rows are
+    // instead loaded four k-steps at a time (they come from memory, where one
+    // k-step's products do not cover the latency; a larger tile has no
+    // registers for it)
+    constexpr bool GROUP = RT <= 2;
+    struct Weights {
+        h8 wh[QUANT ? 1 : RT], wl[WT == W_F32 ? RT : 1];
+        u2 wq[QUANT ? RT : 1];
+    };
+    struct Step {
+        h8 xh[CT], xl[CT];
+        Weights W;
+    };
+    auto load_w = [&](int k, Weights &W) __attribute__((always_inline)) {
+        const int kk = min(k, k1 - 1);
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int64_t t = (rt0 + r) * KS + kk;
+            if constexpr (QUANT) {
+                W.wq[r] = *reinterpret_cast<const u2 *>(WT == W_Q8_0 ? a.a + t * 512 + 8 * lane
+                                                                     : a.a + t * 256 + 16 * j + 8 * (g & 1));
+            } else {
+                W.wh[r] = *reinterpret_cast<const h8 *>(a.a + t * 1024 + 16 * lane);
+                if constexpr (WT == W_F32)
+                    W.wl[r] = *reinterpret_cast<const h8 *>(a.a_lo + t * 1024 + 16 * lane);
+            }
+        }
+    };
+    auto load = [&](int k, Step &S) __attribute__((always_inline)) {
+        const int kk = min(k, k1 - 1);
+#pragma unroll
+        for (int c = 0; c < CT; c++) {
+            const int64_t o = ((bt0 + c) * KS + kk) * 512 + 8 * lane;
+            S.xh[c] = *reinterpret_cast<const h8 *>(a.xh + o);
+            S.xl[c] = *reinterpret_cast<const h8 *>(a.xl + o);
+        }
+        if constexpr (!GROUP)
+            load_w(k, S.W);
+    };
+    // scales of four k-steps from k: lane (j, g) holds rows 4g .. 4g + 3 of
+    // k-step k + (j & 3)
+    auto load_scales = [&](int k, u2 (&sw)[RT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+            sw[r] = *reinterpret_cast<const u2 *>(a.scales + ((rt0 + r) * KS + min(k + (j & 3), k1 - 1)) * 16 + 4 * g);
+    };
+    auto products = [&](auto ic_i, const Step &S, const Weights &W, const u2 (&sw)[RT]) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic_i)::value;
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            if constexpr (QUANT) {
+                const h8 aq = WT == W_Q8_0 ? i8x8_to_h8(W.wq[r]) : u4x8_to_h8(W.wq[r], (g & 2) ? 4 : 0);
+                const uint32_t s01 = row_lane<i>(sw[r].x), s23 = row_lane<i>(sw[r].y);
+                const _Float16 d[4] = {__builtin_bit_cast(_Float16, (uint16_t)(s01 & 0xFFFFu)),
+                                       __builtin_bit_cast(_Float16, (uint16_t)(s01 >> 16)),
+                                       __builtin_bit_cast(_Float16, (uint16_t)(s23 & 0xFFFFu)),
+                                       __builtin_bit_cast(_Float16, (uint16_t)(s23 >> 16))};
+#pragma unroll
+                for (int c = 0; c < CT; c++) {
+                    f4 z = mfma16(aq, S.xh[c], f4{0.0f, 0.0f, 0.0f, 0.0f});
+                    z = mfma16(aq, S.xl[c], z);
+#pragma unroll
+                    for (int q = 0; q < 4; q++)
+                        acc[r][c][q] = fmaf(z[q], (float)d[q], acc[r][c][q]);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < CT; c++) {
+                    acc[r][c] = mfma16(W.wh[r], S.xh[c], acc[r][c]);
+                    acc[r][c] = mfma16(W.wh[r], S.xl[c], acc[r][c]);
+                    if constexpr (WT == W_F32)
+                        acc[r][c] = mfma16(W.wl[r], S.xh[c], acc[r][c]);
+                }
+            }
+        }
+    };
+    if (k0 < k1) {
+        Step A, B;
+        Weights wc[GROUP ? 4 : 1], wn[GROUP ? 4 : 1]; // this group's and the next's
+        u2 sw[RT], sn[RT];
+        auto load_group = [&](int k) __attribute__((always_inline)) {
+            if constexpr (GROUP) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    load_w(k + i, wn[i]);
+            }
+            if constexpr (QUANT)
+                load_scales(k, sn);
+        };
+        load_group(k0);
+        load(k0, A);
+        for (int k = k0; k < k1; k += 4) {
+            if constexpr (GROUP) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    wc[i] = wn[i];
+            }
+            if constexpr (QUANT) {
+#pragma unroll
+                for (int r = 0; r < RT; r++)
+                    sw[r] = sn[r];
+            }
+            load_group(k + 4);
+            load(k + 1, B);
+            products(ic<0>{}, A, GROUP ? wc[0] : A.W, sw);
+            load(k + 2, A);
+            if (k + 1 < k1)
+                products(ic<1>{}, B, GROUP ? wc[GROUP ? 1 : 0] : B.W, sw);
+            load(k + 3, B);
+            if (k + 2 < k1)
+                products(ic<2>{}, A, GROUP ? wc[GROUP ? 2 : 0] : A.W, sw);
+            load(k + 4, A);
+            if (k + 3 < k1)
+                products(ic<3>{}, B, GROUP ? wc[GROUP ? 3 : 0] : B.W, sw);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CT; c++) {
+        const float down = a.xscale[(int64_t)w * batch_pad + b0 + 16 * c + j];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                red[w][16 * r + 4 * g + q][16 * c + j] = acc[r][c][q] * down;
+    }
+    __syncthreads();
+    // rows fastest: coalesced stores
+    for (int e = threadIdx.x; e < 16 * RT * COLS; e += 64 * kRegWaves) {
+        const int rl = e % (16 * RT), cl = e / (16 * RT), r = r0 + rl, b = b0 + cl;
+        if (b >= a.batch || r >= a.rows)
+            continue;
+        float v = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kRegWaves; q++)
+            v += red[q][rl][cl];
+        a.y[(int64_t)b * a.rows + r] = WT == W_F32 ? v * a.row_scale[r] : v;
+    }
+#endif
+}
+
+// Tile shapes: 32 columns to batch 32, else 64; as many rows (16, 32 or 64)
+// as leave about one workgroup per CU.
+template <int WT>
+void launch_reg(const MatArgs &a, int batch_pad, hipStream_t st)
+{
+    const int ct = a.batch <= 32 ? 2 : 4, bts = (a.batch + 16 * ct - 1) / (16 * ct);
+    auto tiles = [&](int rt) { return (a.rows + 16 * rt - 1) / (16 * rt) * bts; };
+    const int rt = tiles(4) >= kRegWorkgroups ? 4 : tiles(2) >= kRegWorkgroups ? 2 : 1;
+    const dim3 grid((unsigned)((tiles(rt) + 7) / 8 * 8)), block(64 * kRegWaves);
+#define GI_REG(RT, CT) hipLaunchKernelGGL((matmul_reg<WT, RT, CT>), grid, block, 0, st, a, batch_pad)
+    if (ct == 2) {
+        if (rt == 4)
+            GI_REG(4, 2);
+        else if (rt == 2)
+            GI_REG(2, 2);
+        else
+            GI_REG(1, 2);
+    } else {
+        if (rt == 4)
+            GI_REG(4, 4);
+        else if (rt == 2)
+            GI_REG(2, 4);
+        else
+            GI_REG(1, 4);
+    }
+#undef GI_REG
+}
+
+// ---- 16-bit weights, large products: split-K ---------------------------------
+//
+// A workgroup of four waves owns a 128 x 128 (rows x batch) output tile over
+// one of S slices of the k-steps, and two workgroups share a CU.  Wave w
+// takes batch rows 32w .. 32w + 31 of the tile and all 128 rows, so each
+// weight fragment read from LDS feeds four products (two batch tiles, hi and
+// lo) and each activation fragment eight (the row tiles).  Per k-step the
+// eight weight tiles (shared by the waves, each loading two) and every wave's
+// activation halves arrive by direct global->LDS loads two k-steps ahead,
+// through three stages; one barrier per k-step hands a stage from the loads
+// to the products.  The per-CU load volume is 24 KiB per 128 products against
+// 12 KiB per 32 in the 64 x 64 form.  With S > 1 the partial tiles go to a
+// workspace and reduce_splits adds them.  Quantised weights
+// do not take it: their per-block scale multiply-adds need 272 registers here
+// (one wave per SIMD).
+
+struct SKArgs {
+    MatArgs m;
+    int splits;   // S: slices of the k-steps
+    int ks_per;   // k-steps per slice (the last may have fewer)
+    float *part;  // S > 1: partial tiles [S][batch_pad][rows_pad]
+    int batch_pad;
+};
+
+// The k-step slices give about kSplitKWorkgroups workgroups, none shorter than kMinSliceSteps
+// k-steps.  The form is taken from kSplitKMinSteps (64 x 64
+// tiles times k-steps) up, where matmul_reg's operand volume per product
+// costs more than the reduction launch here (per call, this / matmul_reg):
+// 8192 x 8192, batch 256: F16 93 / 101 us, F32 123 / 142; batch 127: 57 / 58,
+// 81 / 88; 4096 x 4096, batch 512: 54 / 56, 69 / 72; batch 256 (below the
+// line): 33.6 / 31.5, 41.8 / 41.2.
+constexpr int kSplitKWorkgroups = 256, kMinSliceSteps = 4, kSplitKMinSteps = 65536;
 
 template <int WT>
 __global__ __launch_bounds__(256) void matmul_sk(SKArgs s)
@@ -675,6 +830,204 @@ __global__ __launch_bounds__(256) void reduce_splits(const float *__restrict__ p
     }
 }
 
+// ---- batches of up to 16: one launch, no workspace ---------------------------
+//
+// A workgroup of 16 waves owns 16 rows; wave w takes the w-th sixteenth of the
+// k-steps, CH at a time, for all BP (batch padded to a power of two) rows of
+// x.  Such a product is bound by reading the weights once, and its time by
+// latency: 256 workgroups at 4096 rows put every weight byte in flight in the
+// first instructions, before anything is waited for.  The x chunk (BP x 32 CH
+// columns) is loaded once per wave (64 / BP lanes share a row), scaled by the
+// chunk's own power of two per row, split into hi + lo halves and handed to
+// the operand lanes through the wave's own LDS, so nothing synchronises until
+// the sixteen waves' sums meet at the end.  Each x row's 64-byte k-steps are
+// XOR-swizzled by row, so that the operand reads of four rows fall on all 64
+// banks.
+//
+// Up to 8 batch rows share one 16-column operand: column b holds row b's hi
+// half, column 8 + b its lo half, and the two sums are added at the end.
+//
+// Batch 1, per call: 4096 x 4096 Q4_0 35.1 -> 5.2 us, F16 32.6 -> 7.6 (4.4 TB/s
+// of weights; an empty kernel called the same way takes 4.2); 8192 x 8192
+// Q4_0 63 -> 13.8, F16 59 -> 22.8 (5.9 TB/s).  Batch 16, 4096 x 4096: Q4_0
+// 35.4 -> 9.7, F32 41.8 -> 15.6.  (Before: x padded to 64 rows and split in a
+// launch of its own, then 64 x 64 tiles on 64 workgroups.)  Above 16 rows the
+// x each workgroup converts outweighs its weights.  Batch 1 over quantised
+// weights fits two workgroups on a CU (64 VGPRs), so that one's loads run
+// under the other's products where there are more than 256: 8192 x 8192 Q8_0
+// 17.4 -> 14.5 us.
+constexpr int kVecWaves = 16, kVecMaxBatch = 16;
+
+// Bytes of LDS per wave: hi and lo planes of BP rows of CH k-steps.
+template <int BP, int CH>
+constexpr int kVecStage = 2 * BP * CH * 64;
+
+template <int WT, int BP, int CH>
+__global__ __launch_bounds__(64 * kVecWaves, (WT == W_Q8_0 || WT == W_Q4_0) && BP == 1 ? 8 : 1) void matmul_vec(MatArgs a, const float *__restrict__ x)
+{
+    static_assert(BP >= 1 && BP <= 16 && (BP & (BP - 1)) == 0, "batch rows padded to a power of two");
+    static_assert(CH >= 4 && CH <= 16, "a lane of a 16-lane row per k-step's scales");
+#if __HIP_DEVICE_COMPILE__ // (target builtins inside generic lambdas, as in matmul_sk)
+    constexpr bool PACK = BP <= 8; // hi and lo columns in one operand
+    constexpr int LPR = 64 / BP;   // lanes per x row
+    constexpr int XI = CH * 32 / (4 * LPR) > 0 ? CH * 32 / (4 * LPR) : 1; // 16-byte loads per lane
+    constexpr int ROW = CH * 64;   // bytes of one row of a plane
+    constexpr int RED = kVecWaves * 16 * 17 * 4;
+    constexpr int STG = kVecWaves * kVecStage<BP, CH>;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[STG > RED ? STG : RED];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int j = lane & 15, g = lane >> 4;
+    const int r0 = blockIdx.x * 16, b0 = blockIdx.y * BP;
+    const int C = a.cols, KS = C / 32;
+    const int per = (KS + kVecWaves - 1) / kVecWaves;
+    const int k0 = w * per, k1 = min(KS, k0 + per);
+    uint8_t *mine = smem + w * kVecStage<BP, CH>;
+    // this lane's x row and first column within a chunk
+    const int xb = lane / LPR, xs = 4 * (lane % LPR);
+    const float *xr = x + (int64_t)min(b0 + xb, a.batch - 1) * C;
+    // the plane rows this lane's operand columns read
+    const int ob = PACK ? (j & 7) & (BP - 1) : j;
+    const uint8_t *op = mine + ob * ROW + 16 * g + (PACK && j >= 8 ? BP * ROW : 0);
+    const int64_t t0 = (int64_t)blockIdx.x * KS;
+
+    f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int kc = k0; kc < k1; kc += CH) {
+        const int nk = min(CH, k1 - kc);
+        // the chunk's weights (k-steps past the range repeat its last) ...
+        h8 wh[CH], wl[WT == W_F32 ? CH : 1];
+        u2 wq[CH], sw; // sw: lane (j, g) holds rows 4g .. 4g + 3's scales of k-step j
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            const int kk = min(kc + i, k1 - 1);
+            const int64_t t = t0 + kk;
+            if (WT == W_F16 || WT == W_F32) {
+                wh[i] = *reinterpret_cast<const h8 *>(a.a + t * 1024 + 16 * lane);
+                if (WT == W_F32)
+                    wl[i] = *reinterpret_cast<const h8 *>(a.a_lo + t * 1024 + 16 * lane);
+            } else {
+                wq[i] = *reinterpret_cast<const u2 *>(WT == W_Q8_0 ? a.a + t * 512 + 8 * lane
+                                                                   : a.a + t * 256 + 16 * j + 8 * (g & 1));
+            }
+        }
+        if (WT == W_Q8_0 || WT == W_Q4_0)
+            sw = *reinterpret_cast<const u2 *>(a.scales + (t0 + min(kc + (j & (CH - 1)), k1 - 1)) * 16 + 4 * g);
+        // ... and its x, the row's largest magnitude in the chunk, and the halves
+        f4 xv[XI];
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int c = xs + 4 * LPR * i;
+            xv[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (c < 32 * nk)
+                xv[i] = *reinterpret_cast<const f4 *>(xr + 32 * kc + c);
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                m = fmaxf(m, fabsf(xv[i][q]));
+        }
+#pragma unroll
+        for (int o = LPR / 2; o > 0; o >>= 1)
+            m = fmaxf(m, __shfl_xor(m, o));
+        const int e = pow2_exponent_for(m);
+        const float up = ldexpf(1.0f, e);
+        // the operand reads of the last chunk are done (they fed its products)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int c = xs + 4 * LPR * i;
+            typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+            h4 hi, lo;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const float t = xv[i][q] * up; // exact: a power of two
+                const _Float16 h = (_Float16)t;
+                hi[q] = h;
+                lo[q] = (_Float16)(t - (float)h);
+            }
+            uint8_t *d = mine + xb * ROW + 64 * ((c >> 5) ^ (xb & (CH - 1) & 3)) + 2 * (c & 31);
+            if (c < 32 * CH) {
+                *reinterpret_cast<h4 *>(d) = hi;
+                *reinterpret_cast<h4 *>(d + BP * ROW) = lo;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // 2^-e of the row of this lane's operand column
+        const float down = __shfl(ldexpf(1.0f, -e), ob * LPR);
+        f4 z = f4{0.0f, 0.0f, 0.0f, 0.0f}; // the chunk's sums, in units of 2^-e
+        static_for<CH>([&](auto ic_i) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic_i)::value;
+            if (i >= nk)
+                return;
+            const uint8_t *xp = op + 64 * (i ^ (ob & (CH - 1) & 3));
+            const h8 xh = *reinterpret_cast<const h8 *>(xp);
+            h8 xl = {};
+            if (!PACK)
+                xl = *reinterpret_cast<const h8 *>(xp + BP * ROW);
+            if (WT == W_F16 || WT == W_F32) {
+                z = mfma16(wh[i], xh, z);
+                if (!PACK)
+                    z = mfma16(wh[i], xl, z);
+                if (WT == W_F32)
+                    z = mfma16(wl[i], xh, z);
+            } else {
+                const h8 aq = WT == W_Q8_0 ? i8x8_to_h8(wq[i]) : u4x8_to_h8(wq[i], (g & 2) ? 4 : 0);
+                f4 p = mfma16(aq, xh, f4{0.0f, 0.0f, 0.0f, 0.0f});
+                if (!PACK)
+                    p = mfma16(aq, xl, p);
+                // k-step i's scales, from lane i of each row of 16 lanes
+                const uint32_t s01 = row_lane<i>(sw.x), s23 = row_lane<i>(sw.y);
+                z[0] = fmaf(p[0], (float)__builtin_bit_cast(_Float16, (uint16_t)(s01 & 0xFFFFu)), z[0]);
+                z[1] = fmaf(p[1], (float)__builtin_bit_cast(_Float16, (uint16_t)(s01 >> 16)), z[1]);
+                z[2] = fmaf(p[2], (float)__builtin_bit_cast(_Float16, (uint16_t)(s23 & 0xFFFFu)), z[2]);
+                z[3] = fmaf(p[3], (float)__builtin_bit_cast(_Float16, (uint16_t)(s23 >> 16)), z[3]);
+            }
+        });
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            acc[i] = fmaf(z[i], down, acc[i]);
+    }
+    // the sixteen waves' sums: [wave][column][row]
+    __syncthreads();
+    float(*red)[16][17] = reinterpret_cast<float(*)[16][17]>(smem);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        red[w][j][4 * g + i] = acc[i];
+    __syncthreads();
+    // lanes 16 q + r of wave b: row r of batch row b, waves 4 q .. 4 q + 3
+    if (w < BP && b0 + w < a.batch) {
+        float v = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kVecWaves / 4; q++) {
+            v += red[4 * g + q][w][j];
+            if (PACK)
+                v += red[4 * g + q][8 + w][j];
+        }
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+        const int r = r0 + j;
+        if (g == 0 && r < a.rows)
+            a.y[(int64_t)(b0 + w) * a.rows + r] = WT == W_F32 ? v * a.row_scale[r] : v;
+    }
+#endif
+}
+
+// Launches matmul_vec for a.batch <= kVecMaxBatch.
+template <int WT>
+void launch_vec(const MatArgs &a, const float *x, hipStream_t st)
+{
+    const dim3 grid((unsigned)((a.rows + 15) / 16)), block(64 * kVecWaves);
+    if (a.batch <= 1)
+        hipLaunchKernelGGL((matmul_vec<WT, 1, 8>), grid, block, 0, st, a, x);
+    else if (a.batch <= 2)
+        hipLaunchKernelGGL((matmul_vec<WT, 2, 8>), grid, block, 0, st, a, x);
+    else if (a.batch <= 4)
+        hipLaunchKernelGGL((matmul_vec<WT, 4, 8>), grid, block, 0, st, a, x);
+    else if (a.batch <= 8)
+        hipLaunchKernelGGL((matmul_vec<WT, 8, WT == W_F32 ? 4 : 8>), grid, block, 0, st, a, x);
+    else
+        hipLaunchKernelGGL((matmul_vec<WT, 16, 4>), grid, block, 0, st, a, x);
+}
+
 int hip_fail(hipError_t e, const char *what)
 {
     return set_error(GI_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
@@ -806,35 +1159,11 @@ int gi_matmul_batch(gi_weights *w, int batch, const float *x, float *y)
     if (batch == 0)
         return GI_OK;
     gi_paged *h = w->h;
-    const int batch_pad = (int)round_pad(batch); // activation rows, zero-padded
     const int rows_pad = (int)weight_rows_pad(w->rows);
     hipStream_t st = (hipStream_t)gi_paged_stream(h);
-    // the split-K form from two batch tiles of 64 up; its slices: enough for
-    // one workgroup per CU, each at least kMinSliceSteps k-steps long
-    const int KS = w->cols / 32;
-    const bool sk = batch_pad >= kSplitKMinBatch && (w->type == W_F16 || w->type == W_F32);
-    int splits = 1, ks_per = KS;
-    if (sk) {
-        const int tiles = (rows_pad / 128) * ((batch_pad + 127) / 128);
-        splits = std::max(1, std::min((kSplitKWorkgroups + tiles - 1) / tiles, KS / kMinSliceSteps));
-        ks_per = (KS + splits - 1) / splits;
-        splits = (KS + ks_per - 1) / ks_per;
-    }
-    // hi and lo halves [batch_pad][cols], the row scales, then the partial
-    // tiles [splits][batch_pad][rows_pad]
-    const size_t nx = (size_t)batch_pad * w->cols * 2;
-    const size_t part_off = (2 * nx + (size_t)batch_pad * 4 + 255) / 256 * 256;
-    const size_t need = part_off + (splits > 1 ? (size_t)splits * batch_pad * rows_pad * 4 : 0);
     hipError_t e = hipSetDevice(w->device);
     if (e != hipSuccess)
         return hip_fail(e, "gi_matmul_batch");
-    const int rc = devbuf_reserve(w->xsplit, need, st, "gi_matmul_batch");
-    if (rc != GI_OK)
-        return rc;
-    _Float16 *xh = (_Float16 *)w->xsplit.ptr;
-    _Float16 *xl = (_Float16 *)((uint8_t *)w->xsplit.ptr + nx);
-    float *xscale = (float *)((uint8_t *)w->xsplit.ptr + 2 * nx);
-    hipLaunchKernelGGL(split_rows, dim3((unsigned)batch_pad), dim3(256), 0, st, x, batch, w->cols, xh, xl, xscale);
     MatArgs a{};
     a.type = w->type;
     a.rows = w->rows;
@@ -845,11 +1174,48 @@ int gi_matmul_batch(gi_weights *w, int batch, const float *x, float *y)
     a.a_lo = w->a_lo;
     a.scales = w->scales;
     a.row_scale = w->row_scale;
+    a.y = y;
+    // matmul_vec writes rows of y while other workgroups still read x: buffers
+    // that overlap take the form that splits x first
+    const uintptr_t xa = (uintptr_t)x, ya = (uintptr_t)y;
+    const bool overlap = xa < ya + (uintptr_t)batch * w->rows * 4 && ya < xa + (uintptr_t)batch * w->cols * 4;
+    if (batch <= kVecMaxBatch && !overlap) {
+        switch (w->type) {
+        case W_F32: launch_vec<W_F32>(a, x, st); break;
+        case W_F16: launch_vec<W_F16>(a, x, st); break;
+        case W_Q8_0: launch_vec<W_Q8_0>(a, x, st); break;
+        default: launch_vec<W_Q4_0>(a, x, st); break;
+        }
+        e = hipGetLastError();
+        return e == hipSuccess ? GI_OK : hip_fail(e, "gi_matmul_batch");
+    }
+    // hi and lo halves [batch_pad][cols], their row scales (matmul_reg: per
+    // segment), then (split-K) the partial tiles [splits][batch_pad][rows_pad]
+    const int batch_pad = (int)round_pad(batch);
+    const size_t nx = (size_t)batch_pad * w->cols * 2;
+    const int KS = w->cols / 32;
+    const int64_t tiles64 = (int64_t)((w->rows + 63) / 64) * (batch_pad / 64);
+    const bool sk = (w->type == W_F16 || w->type == W_F32) && tiles64 * KS >= kSplitKMinSteps;
+    int splits = 1, ks_per = KS;
+    if (sk) {
+        const int tiles = (rows_pad / 128) * ((batch_pad + 127) / 128);
+        splits = std::max(1, std::min((kSplitKWorkgroups + tiles - 1) / tiles, KS / kMinSliceSteps));
+        ks_per = (KS + splits - 1) / splits;
+        splits = (KS + ks_per - 1) / ks_per;
+    }
+    const size_t part_off = (2 * nx + (size_t)kRegWaves * batch_pad * 4 + 255) / 256 * 256;
+    const size_t need = part_off + (splits > 1 ? (size_t)splits * batch_pad * rows_pad * 4 : 0);
+    const int rc = devbuf_reserve(w->xsplit, need, st, "gi_matmul_batch");
+    if (rc != GI_OK)
+        return rc;
+    _Float16 *xh = (_Float16 *)w->xsplit.ptr;
+    _Float16 *xl = (_Float16 *)((uint8_t *)w->xsplit.ptr + nx);
+    float *xscale = (float *)((uint8_t *)w->xsplit.ptr + 2 * nx);
     a.xh = xh;
     a.xl = xl;
     a.xscale = xscale;
-    a.y = y;
     if (sk) {
+        hipLaunchKernelGGL(split_rows, dim3((unsigned)batch_pad), dim3(256), 0, st, x, batch, w->cols, xh, xl, xscale);
         SKArgs k{};
         k.m = a;
         k.splits = splits;
@@ -868,12 +1234,13 @@ int gi_matmul_batch(gi_weights *w, int batch, const float *x, float *y)
                                w->type == W_F32 ? (const float *)w->row_scale : nullptr, y);
         }
     } else {
-        dim3 grid((unsigned)(batch_pad / 64), (unsigned)(a.rows_pad / 64));
+        hipLaunchKernelGGL(split_x, dim3((unsigned)(batch_pad / 16), kRegWaves), dim3(256), 0, st, x, batch,
+                           batch_pad, w->cols, xh, xl, xscale);
         switch (w->type) {
-        case W_F32: hipLaunchKernelGGL((matmul_lds<W_F32, 2>), grid, dim3(256), 0, st, a); break;
-        case W_F16: hipLaunchKernelGGL((matmul_lds<W_F16, 3>), grid, dim3(256), 0, st, a); break;
-        case W_Q8_0: hipLaunchKernelGGL((matmul_lds<W_Q8_0, 3>), grid, dim3(256), 0, st, a); break;
-        default: hipLaunchKernelGGL((matmul_lds<W_Q4_0, 3>), grid, dim3(256), 0, st, a); break;
+        case W_F32: launch_reg<W_F32>(a, batch_pad, st); break;
+        case W_F16: launch_reg<W_F16>(a, batch_pad, st); break;
+        case W_Q8_0: launch_reg<W_Q8_0>(a, batch_pad, st); break;
+        default: launch_reg<W_Q4_0>(a, batch_pad, st); break;
         }
     }
     e = hipGetLastError();

@@ -14,11 +14,10 @@ float32 dot products of length cols:
   * well-conditioned inputs (N(0,1)): per batch row,
     max|gpu - oracle| <= 1e-5 * max|oracle| and the same against float64.
 
-The shapes cover both product forms: batches under 128 (and quantised
-weights) run the 64 x 64 tiles; F16 / F32 weights at batches of 128 and more
-run the split-K tiles, whose cases include rows that are not a multiple of
-128, a batch with idle waves in its last tile (130), k-step slices with a
-remainder (1056 columns: 33 k-steps) and two batch tiles (384)."""
+The shapes cover the three product forms: batches of up to 16, larger ones,
+and (F16 / F32 weights, large products) the split-K tiles;
+test_matmul_form_edges takes each at the sizes where its indexing can go
+wrong."""
 import numpy as np
 import pytest
 
@@ -118,6 +117,58 @@ def test_matmul_batch_sizes_on_one_weight_set(gi, oracle, dev, t):
     finally:
         wt.close()
         pool.close()
+
+
+# rows, cols, batch.  Up to 16 rows: every padded batch; one k-step, fewer
+# k-steps than waves, ranges of 1, 9 and 17 k-steps (one to five chunks).
+# Over 16: waves with an empty last segment (33 k-steps), and each row-tile
+# count the dispatch takes (rows for 1, 2 and 4 tiles of 16) by each column
+# width.  Split-K: a last batch tile with idle waves, slices of 73 k-steps.
+FORM_EDGES = [(1, 32, 1), (17, 96, 2), (16, 288, 4), (40, 4128, 8), (130, 8224, 3), (130, 8224, 1), (33, 4128, 16),
+              (130, 544, 9), (48, 32, 17), (100, 1056, 33), (8200, 64, 17), (16400, 64, 20), (4100, 160, 70),
+              (8200, 96, 70), (16400, 32, 40), (4104, 4672, 400)]
+
+
+@pytest.mark.parametrize("t", [0, 1, 2, 8], ids=["f32", "f16", "q4_0", "q8_0"])
+@pytest.mark.parametrize("rows,cols,batch", FORM_EDGES)
+def test_matmul_form_edges(gi, oracle, dev, t, rows, cols, batch):
+    """Each form at the edges of its tiles, against the float64 product of
+    the dequantised weights: the rounding bound of a float32 sum, as above,
+    plus the split's own 2^-21 of the largest |x| a row range holds (a hi + lo
+    pair of halves keeps 22 bits of it)."""
+    if (rows, cols, batch) == FORM_EDGES[-1] and t in (2, 8):
+        pytest.skip("split-K serves F16 and F32 weights")
+    rng = np.random.default_rng(rows + cols + batch + t)
+    W = rng.standard_normal((rows, cols), np.float32)
+    x = rng.standard_normal((batch, cols), np.float32)
+    x[batch - 1] *= 1e3
+    raw = oracle.quantize_weights(t, W)
+    got = _run(gi, dev, t, rows, cols, raw, x)
+    wd = np.abs(dequant(oracle, t, raw, rows, cols).astype(np.float64))
+    exact = x.astype(np.float64) @ dequant(oracle, t, raw, rows, cols).astype(np.float64).T
+    bound = 4 * EPS32 * np.sqrt(cols) * (np.abs(x).astype(np.float64) @ wd.T)
+    bound += 2.0**-21 * np.abs(x).max(axis=1, keepdims=True) * wd.sum(axis=1)[None]
+    assert np.isfinite(got).all()
+    assert float((np.abs(got - exact) / bound).max()) <= 1.0
+
+
+def test_matmul_in_place(gi, oracle, dev):
+    """y may be x's own buffer (square weights), whatever the batch."""
+    import torch
+    n = 256
+    raw = oracle.quantize_weights(1, oracle.normal(5, (n, n)))
+    wd = dequant(oracle, 1, raw, n, n).astype(np.float64)
+    pool = gi.PagedKVCache(1, 1, 32, 16, 1, gi.KV_F16)
+    wt = gi.Weights(pool, 1, n, n, raw)
+    for batch in (1, 7, 40):
+        x = oracle.normal(6 + batch, (batch, n))
+        d = torch.from_numpy(x).to(dev)
+        wt.MatMulBatch(d, d)
+        pool.synchronize()
+        exact = x.astype(np.float64) @ wd.T
+        assert float(np.abs(d.cpu().numpy() - exact).max()) <= 1e-5 * np.abs(exact).max()
+    wt.close()
+    pool.close()
 
 
 def test_matmul_errors(gi, dev):
