@@ -273,33 +273,92 @@ __global__ __launch_bounds__(NT) void attn_valu(DecodeArgs a)
 }
 
 // Merges split partials: out = sum_s acc_s e^(m_s - M) / sum_s l_s e^(m_s - M).
-// One workgroup per (query row, head), one thread per output dimension.
-__global__ __launch_bounds__(256) void merge_splits(float *__restrict__ out,
-                                                    const float *__restrict__ ws, int H, int KVH,
-                                                    int HD, int splits)
+// W waves serve one (query row, head): wave w takes splits w, w + W, ...,
+// lane i the HD / 64 dimensions from i * HD / 64, and the waves' sums meet in
+// LDS.  Latency bounds it, so a wave's first kMergeAhead partials are
+// requested together with the maxima of all splits: one round trip for up to
+// W * kMergeAhead splits.  W is 1 (four heads per workgroup, no barrier) for
+// up to kMergeAhead splits and 4 above: four waves per head on 2 splits of 52
+// sequences x 32 heads cost 1 us more than one (19.9 against 18.9 us a step).
+constexpr int kMergeAhead = 8;
+
+template <int HD, int W>
+__global__ __launch_bounds__(256) void merge_splits(float *__restrict__ out, const float *__restrict__ ws,
+                                                    int rows, int H, int KVH, int splits)
 {
-    const int h = blockIdx.x, qrow = blockIdx.y;
+    constexpr int V = HD / 64, ROWS = 4 / W; // (query row, head) pairs per workgroup
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wv = wave % W;
+    const int64_t row = (int64_t)blockIdx.x * ROWS + wave / W;
+    if (row >= rows) // W == 1 only: a workgroup of W == 4 is one row
+        return;
+    const int64_t qrow = row / H;
+    const int h = (int)(row - qrow * H);
     const int G = H / KVH;
     const int kvh = h / G, g = h - kvh * G;
     const int64_t stride = (int64_t)G * (HD + 2);
-    const float *w0 = ws + ((int64_t)qrow * KVH + kvh) * splits * stride;
-    float M = -INFINITY;
-    for (int s = 0; s < splits; s++)
-        M = fmaxf(M, w0[s * stride + G * HD + 2 * g]);
-    for (int d = threadIdx.x; d < HD; d += blockDim.x) {
-        float num = 0.0f, den = 0.0f;
-        if (M != -INFINITY) {
-            for (int s = 0; s < splits; s++) {
-                const float *w = w0 + s * stride;
-                const float m = w[G * HD + 2 * g];
-                if (m == -INFINITY)
-                    continue;
-                const float f = expf(m - M);
-                num = fmaf(w[g * HD + d], f, num);
-                den = fmaf(w[G * HD + 2 * g + 1], f, den);
-            }
+    const float *w0 = ws + (qrow * KVH + kvh) * splits * stride;
+    const float *ml = w0 + G * HD + 2 * g; // (m, l) of split 0
+    const float *wo = w0 + g * HD + V * lane;
+
+    vec o[kMergeAhead];
+    float2 t[kMergeAhead];
+#pragma unroll
+    for (int i = 0; i < kMergeAhead; i++) {
+        const int s = wv + W * i;
+        if (s < splits) {
+            o[i] = *reinterpret_cast<const vec *>(wo + s * stride);
+            t[i] = *reinterpret_cast<const float2 *>(ml + s * stride);
         }
-        out[((int64_t)qrow * H + h) * HD + d] = den > 0.0f ? num / den : 0.0f;
+    }
+    float M = -INFINITY;
+    for (int s = lane; s < splits; s += 64)
+        M = fmaxf(M, ml[s * stride]);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1)
+        M = fmaxf(M, __shfl_xor(M, m));
+
+    vec num = {};
+    float den = 0.0f;
+    auto add = [&](vec x, float2 y) {
+        const float f = y.x == -INFINITY ? 0.0f : expf(y.x - M);
+#pragma unroll
+        for (int v = 0; v < V; v++)
+            num[v] = fmaf(x[v], f, num[v]);
+        den = fmaf(y.y, f, den);
+    };
+#pragma unroll
+    for (int i = 0; i < kMergeAhead; i++)
+        if (wv + W * i < splits)
+            add(o[i], t[i]);
+    for (int s = wv + W * kMergeAhead; s < splits; s += W)
+        add(*reinterpret_cast<const vec *>(wo + s * stride), *reinterpret_cast<const float2 *>(ml + s * stride));
+
+    if constexpr (W == 1) {
+        vec r;
+#pragma unroll
+        for (int v = 0; v < V; v++)
+            r[v] = den > 0.0f ? num[v] / den : 0.0f;
+        *reinterpret_cast<vec *>(out + row * HD + V * lane) = r;
+    } else {
+        __shared__ float s_num[W][HD];
+        __shared__ float s_den[W];
+#pragma unroll
+        for (int v = 0; v < V; v++)
+            s_num[wv][V * lane + v] = num[v];
+        if (lane == 0)
+            s_den[wv] = den;
+        __syncthreads();
+        if (threadIdx.x < HD) {
+            float n = 0.0f, d = 0.0f;
+#pragma unroll
+            for (int x = 0; x < W; x++) {
+                n += s_num[x][threadIdx.x];
+                d += s_den[x];
+            }
+            out[row * HD + threadIdx.x] = d > 0.0f ? n / d : 0.0f;
+        }
     }
 }
 
@@ -329,44 +388,98 @@ size_t decode_workspace_bytes(const PoolLayout &L, int batch, int num_heads, int
     return (size_t)batch * L.num_kv_heads * num_splits * G * (L.head_dim + 2) * sizeof(float);
 }
 
-// Split-K planning: enough (split, kv head, sequence) workgroups for about
-// kDecodeWgPerCu per CU, each split at least kDecodeMinSplit tokens.
-// Measured on MI355X: 1 and 1024 beat finer splits (2/1024, 4/512, 8/256,
-// 16/128) on 32 ragged sequences of 512-4096 tokens (one workgroup per
-// (sequence, kv head), no merge: 2.79 against 2.93 ms per step) and match
-// 2/1024 on 8 sequences of 32768, since every workgroup pays a fixed cost
-// (query load, cross-wave merge, partials) and a split sequence pays the
-// merge launch.  A plan that balances equal token ranges over all
-// workgroups regardless of sequence boundaries (with partial slots per range
-// and a merge per sequence) measured 2-10% slower on long and uniform
-// batches and only 5% faster on ragged ones.
-constexpr int kDecodeWgPerCu = 1;
-constexpr int kDecodeMinSplit = 1024;
+// f32 pages at head dimension 128 stage 32 KiB per wave, so a CU holds one
+// four-wave workgroup of them; every other page type runs one eight-wave or
+// two four-wave workgroups per CU (decode_waves).
+static bool one_wg_per_cu(const PoolLayout &L) { return L.kv_type == KV_F32 && L.head_dim == 128; }
+
+// Whole page pairs and a multiple of 64 tokens: the unit a split holds.
+static int split_unit(const PoolLayout &L)
+{
+    int unit = 2 * L.page_tokens;
+    while (unit % 64)
+        unit += 2 * L.page_tokens;
+    return unit;
+}
+
+static void set_plan(const PoolLayout &L, int max_len, int splits, int *split_tokens, int *num_splits)
+{
+    const int unit = split_unit(L);
+    if (splits < 1)
+        splits = 1;
+    int per = (max_len + splits - 1) / splits;
+    per = (per + unit - 1) / unit * unit;
+    *split_tokens = per;
+    *num_splits = (max_len + per - 1) / per;
+}
+
+// Split-K planning.  A workgroup costs about 4 us beside its tokens (query,
+// table and page latencies, cross-wave merge) and a split sequence a merge
+// launch, so a sequence is split only where that leaves less of the chip
+// idle.  Measured on MI355X in us per layer (start: about one workgroup per
+// CU, rounded up, and at least 1024 tokens per split):
+//  - up to two blocks per wave (four where the pairs themselves use the
+//    CUs), one split: batch 1 x 300 f16 8.6 against 10.0 in splits of 128,
+//    batch 14 x 400-800 (112 pairs) 19.5 against 21.1 in two;
+//  - few (sequence, kv head) pairs: splits of 128 tokens until the CUs are
+//    full.  Batch 1 f16 1000 tokens 16.1 -> 11.1, 6001 18.8 -> 13.5; f32
+//    1000 29.8 -> 13.4; splits of 64 were no faster;
+//  - the number of workgroups is kept at or below one (eight waves) or two
+//    (four waves) per CU, whichever leaves less idle: rounded up it left a
+//    few CUs with twice the work.  f16, 5000 tokens: 72 pairs 43.8 in 4
+//    splits, 35.7 in 3; 96 pairs 55.9 in 3, 45.3 in 5; 160 pairs 82.5 in 2,
+//    69.9 in 3.  f32 at head dimension 128 (one workgroup per CU): 136 pairs
+//    161 in 2 splits, 124 in one;
+//  - 1 to 2 pairs per CU: unsplit, half of the CUs hold one workgroup and
+//    half two; 5 or 3 splits even that out on long sequences.  5000 tokens,
+//    288 pairs: f16 150 -> 125, q4_0 76 -> 57, f32 310 -> 248, q8_0 85 -> 81;
+//    384 pairs, 1500-6500 tokens: f16 157 -> 140, q4_0 87 -> 71, f32 298 ->
+//    268, but q8_0 at 5000 tokens 95 -> 106, which stays unsplit; at 1500
+//    tokens splits lose everywhere;
+//  - from two pairs per CU on the launch has enough rounds to even out: 480
+//    and 640 pairs are fastest unsplit.
+constexpr int kDecodeMinSplit = 128;
 
 void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, int num_cus,
                  int *split_tokens, int *num_splits)
 {
     (void)num_heads;
-    // Split unit: whole page pairs and a multiple of 64 tokens.
-    int unit = 2 * L.page_tokens;
-    while (unit % 64)
-        unit += 2 * L.page_tokens;
     if (max_len < 1)
         max_len = 1;
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
     const int64_t pairs = (int64_t)batch * L.num_kv_heads;
-    const int64_t target = (int64_t)kDecodeWgPerCu * (num_cus > 0 ? num_cus : 256);
-    int splits = (int)((target + pairs - 1) / pairs);
-    // A minimum of tokens per split keeps the merge negligible.
-    int max_splits = (max_len + kDecodeMinSplit - 1) / kDecodeMinSplit;
-    if (splits > max_splits)
-        splits = max_splits;
-    if (splits < 1)
-        splits = 1;
-    int per = (max_len + splits - 1) / splits;
-    per = (per + unit - 1) / unit * unit;
-    splits = (max_len + per - 1) / per;
-    *split_tokens = per;
-    *num_splits = splits;
+    const bool single = one_wg_per_cu(L);
+    int64_t s = 1;
+    int min_split = kDecodeMinSplit;
+    if (pairs < 1 || max_len <= (single ? 256 : pairs * 4 <= cus ? 512 : 1024)) {
+        s = 1;
+    } else if (pairs <= cus / 2) {
+        s = cus / pairs;
+        const int64_t s2 = 2 * cus / pairs;
+        if (!single && pairs * (s2 - 2 * s) * 20 > 3 * 2 * cus) // 15 % more of the chip
+            s = s2;
+    } else if (pairs < cus) {
+        s = single || max_len <= 1024 ? 1 : 2 * cus / pairs;
+        min_split = 512;
+    } else if (pairs > cus && pairs < 2 * cus) {
+        if (pairs * 4 <= 5 * cus && max_len >= 4096)
+            s = 5;
+        else if (pairs * 16 <= 25 * cus && max_len >= 2560 && L.kv_type != KV_Q8_0)
+            s = 3;
+    }
+    set_plan(L, max_len, (int)min(s, (int64_t)(max_len + min_split - 1) / min_split), split_tokens, num_splits);
+}
+
+// The plan with the fewest partials: about one workgroup per CU, splits of
+// at least 1024 tokens.  For scratch that decode_plan's partials overflow.
+void decode_plan_coarse(const PoolLayout &L, int batch, int max_len, int num_cus, int *split_tokens, int *num_splits)
+{
+    if (max_len < 1)
+        max_len = 1;
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    const int64_t pairs = (int64_t)batch * L.num_kv_heads;
+    const int64_t s = pairs > 0 ? (cus + pairs - 1) / pairs : 1;
+    set_plan(L, max_len, (int)min(s, ((int64_t)max_len + 1023) / 1024), split_tokens, num_splits);
 }
 
 // Whether a decode step stores its token inside the matrix-core decode
@@ -429,8 +542,22 @@ hipError_t launch_decode(const DecodeArgs &a, hipStream_t st)
     }
     if (e != hipSuccess || a.num_splits <= 1)
         return e;
-    hipLaunchKernelGGL(merge_splits, dim3(a.num_heads, a.batch * n_q), dim3(min(L.head_dim, 256)),
-                       0, st, a.out, a.ws, a.num_heads, L.num_kv_heads, L.head_dim, a.num_splits);
+    const int rows = a.batch * n_q * a.num_heads;
+#define GI_MERGE(HDv, Wv)                                                                              \
+    hipLaunchKernelGGL((merge_splits<HDv, Wv>), dim3((unsigned)((rows + 4 / Wv - 1) / (4 / Wv))),       \
+                       dim3(256), 0, st, a.out, a.ws, rows, a.num_heads, L.num_kv_heads, a.num_splits)
+    if (a.num_splits <= kMergeAhead) {
+        if (L.head_dim == 128)
+            GI_MERGE(128, 1);
+        else
+            GI_MERGE(64, 1);
+    } else {
+        if (L.head_dim == 128)
+            GI_MERGE(128, 4);
+        else
+            GI_MERGE(64, 4);
+    }
+#undef GI_MERGE
     return hipGetLastError();
 }
 

@@ -87,6 +87,11 @@ bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num
 void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, int num_cus,
                  int *split_tokens, int *num_splits);
 
+// The same with longer splits and so less workspace, for callers whose
+// scratch cannot hold decode_plan's partials.
+void decode_plan_coarse(const PoolLayout &L, int batch, int max_len, int num_cus, int *split_tokens,
+                        int *num_splits);
+
 // Waves per workgroup of the matrix-core decode launch: 8 when the grid of
 // (split, kv head, sequence) workgroups fits the CUs once, so that every
 // SIMD still streams with two waves; 4 otherwise.

@@ -634,9 +634,27 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
     const int max_len = (int)(max_seq_len > 0 && max_seq_len < mapped ? max_seq_len
                               : mapped < INT32_MAX ? mapped : INT32_MAX);
     gi::decode_plan(h->L, batch, num_heads, max_len, h->num_cus, &a.split_tokens, &a.num_splits);
-    a.waves = gi::decode_waves(h->L, batch, a.num_splits, h->num_cus);
     // the workspace first: a call refused here has queued nothing
-    const size_t need = gi::decode_workspace_bytes(h->L, batch, num_heads, a.num_splits);
+    size_t need = gi::decode_workspace_bytes(h->L, batch, num_heads, a.num_splits);
+    int coarse_tokens, coarse_splits;
+    gi::decode_plan_coarse(h->L, batch, max_len, h->num_cus, &coarse_tokens, &coarse_splits);
+    const size_t coarse = gi::decode_workspace_bytes(h->L, batch, num_heads, coarse_splits);
+    if (need > (fixed_ws ? fixed_cap : h->plan_ws.bytes)) {
+        // partials that the scratch cannot hold, or that a capturing stream
+        // cannot allocate: fewer, longer splits may still fit
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusActive;
+        if (!fixed_ws) {
+            hipError_t e = hipStreamIsCapturing(h->stream, &cs);
+            if (e != hipSuccess)
+                return hip_fail(e, "decode attention: hipStreamIsCapturing");
+        }
+        if (cs != hipStreamCaptureStatusNone) {
+            a.split_tokens = coarse_tokens;
+            a.num_splits = coarse_splits;
+            need = coarse;
+        }
+    }
+    a.waves = gi::decode_waves(h->L, batch, a.num_splits, h->num_cus);
     std::unique_lock<std::mutex> order; // the shared scratch's users, in turn
     bool eager = false;
     if (fixed_ws) {
@@ -660,7 +678,17 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
                 return hip_fail(e, "gi_paged_decode_attention_noalloc: hipStreamWaitEvent");
         }
     } else {
-        const int rc = gi::devbuf_reserve(h->plan_ws, need, h->stream, "decode attention");
+        // an eager call also makes room for the coarse plan of its shape, so
+        // that a later capture of any shape no larger finds room
+        const bool grows = h->plan_ws.bytes < need || h->plan_ws.bytes < coarse;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (grows) {
+            const hipError_t e = hipStreamIsCapturing(h->stream, &cs);
+            if (e != hipSuccess)
+                return hip_fail(e, "decode attention: hipStreamIsCapturing");
+        }
+        const size_t want = grows && cs == hipStreamCaptureStatusNone && coarse > need ? coarse : need;
+        const int rc = gi::devbuf_reserve(h->plan_ws, want, h->stream, "decode attention");
         if (rc)
             return rc;
         a.ws = (float *)h->plan_ws.ptr;

@@ -265,11 +265,13 @@ int gi_paged_gather(gi_paged *h, int layer, const int32_t *block_table, int n_to
  *
  * Workspace: the handle keeps the partials of split sequences, batch *
  * num_kv_heads * splits slots of (num_heads / num_kv_heads) * (head_dim + 2)
- * floats, where splits falls as batch * num_kv_heads grows (about one
- * workgroup per CU).  A call that needs it to grow while the handle's stream
- * is capturing a graph fails with GI_ERR_BAD_ARG (make one eager call with
- * the same shape first); once any call has been captured, growth keeps the
- * old buffers alive until gi_paged_destroy, so captured graphs stay valid. */
+ * floats, where splits falls as batch * num_kv_heads grows (at most six
+ * workgroups per CU).  A call that needs it to grow while the handle's stream
+ * is capturing a graph takes fewer, longer splits (at least 1024 tokens, about
+ * one workgroup per CU), and fails with GI_ERR_BAD_ARG where their partials
+ * do not fit either (make one eager call with the same shape first); once any
+ * call has been captured, growth keeps the old buffers alive until
+ * gi_paged_destroy, so captured graphs stay valid. */
 int gi_paged_decode_attention(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                               float *out, const int32_t *block_tables, int max_blocks,
                               const int32_t *seq_lens, int max_seq_len, float scale);
@@ -279,8 +281,9 @@ int gi_paged_decode_attention(gi_paged *h, int layer, int batch, int num_heads, 
  * under HIP graph capture, tight serving loops, hosts that forbid it).  The
  * split partials live in a fixed 4 MiB scratch array that the library holds
  * on each device it runs on until the process ends, instead of the handle's
- * growable workspace.  On a 256-CU device every shape with up to 8 query
- * heads per kv head fits (fewer than 512 partial slots of 4 KiB); with 16
+ * growable workspace; partials that would not fit it are avoided by fewer,
+ * longer splits, as under capture above.  On a 256-CU device every shape with
+ * up to 8 query heads per kv head fits; with 16
  * per kv head at head_dim 128 the batches with batch * num_kv_heads of 253
  * to 255 and contexts over 1024 tokens (two splits, 506 to 510 slots of
  * 8 KiB) would need up to 4.25 MB and fail with GI_ERR_BAD_ARG before any
