@@ -11,6 +11,7 @@
 // from HBM once per decode step.
 #include "gi_common.h"
 #include "gi_kernels.h"
+#include "token_store.h"
 
 #include <math.h>
 
@@ -278,13 +279,16 @@ __global__ __launch_bounds__(NT) void attn_valu(DecodeArgs a)
 // LDS.  Latency bounds it, so a wave's first kMergeAhead partials are
 // requested together with the maxima of all splits: one round trip for up to
 // W * kMergeAhead splits.  W is 1 (four heads per workgroup, no barrier) for
-// up to kMergeAhead splits and 4 above: four waves per head on 2 splits of 52
+// up to kMergeAhead splits and 4 above (both also write a step's turned q,
+// DecodeArgs.rope, which every split has read by then): four waves per head on 2 splits of 52
 // sequences x 32 heads cost 1 us more than one (19.9 against 18.9 us a step).
 constexpr int kMergeAhead = 8;
 
 template <int HD, int W>
-__global__ __launch_bounds__(256) void merge_splits(float *__restrict__ out, const float *__restrict__ ws,
-                                                    int rows, int H, int KVH, int splits)
+__global__ __launch_bounds__(256) void merge_splits(float *out, const float *__restrict__ ws,
+                                                    int rows, int H, int KVH, int splits,
+                                                    float *q, const float2 *__restrict__ rope,
+                                                    int rope_max_pos, const int32_t *__restrict__ seq_lens)
 {
     constexpr int V = HD / 64, ROWS = 4 / W; // (query row, head) pairs per workgroup
     typedef float vec __attribute__((ext_vector_type(V)));
@@ -310,6 +314,14 @@ __global__ __launch_bounds__(256) void merge_splits(float *__restrict__ out, con
         if (s < splits) {
             o[i] = *reinterpret_cast<const vec *>(wo + s * stride);
             t[i] = *reinterpret_cast<const float2 *>(ml + s * stride);
+        }
+    }
+    if (rope && wv == 0 && lane < HD / 2) {
+        const int pos = seq_lens[qrow] - 1;
+        if (pos >= 0 && pos < rope_max_pos) {
+            float *x = q + row * HD + lane;
+            const float2 cs = rope[(int64_t)pos * (HD / 2) + lane];
+            rope_pair(x[0], x[HD / 2], cs.x, cs.y, &x[0], &x[HD / 2]);
         }
     }
     float M = -INFINITY;
@@ -497,6 +509,38 @@ bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num
     return wgs <= (int64_t)2 * (num_cus > 0 ? num_cus : 256);
 }
 
+// The matrix-core decode turns whole heads: a pair's two elements are then
+// in one lane of the query operand.  Turning q and storing the token inside
+// the launch saves the one before it (4 us; 8 us at 48 sequences), and costs
+// each workgroup the wait for its token's store and the q write at its end.
+// With RoPE, us per layer, fused / separate:
+//  - one round (two workgroups per CU): batch 1 x 6001 f16 14.9 / 19.1,
+//    batch 64 x 2000 q4_0 41.0 / 45.5, q8_0 51.3 / 55.4, f16 80.1 / 80.7;
+//  - q4_0, and 16-bit or 8-bit pages at head dimension 64 (three or more
+//    workgroups per CU at once): up to six per CU.  q4_0 48 x 6500 (1152)
+//    78.6 / 83.6, 200 x 2000 (1600) 101.8 / 100.3; head dimension 64 f16
+//    200 x 2000 (800) 74.6 / 76.7;
+//  - f16 and f32 at head dimension 128 stream at the HBM rate from the first
+//    block, so long splits hide the separate launch: f16 64 x 5000 182.9 /
+//    180.6, 64 x 12000 422 / 414, f32 64 x 2000 159.8 / 154.2, 64 x 700
+//    69.9 / 71.6.
+bool decode_fuses_rope(const PoolLayout &L, int batch, int num_heads, int requested, int rope_half,
+                       int split_tokens, int num_splits, int num_cus)
+{
+    if (rope_half != L.head_dim / 2 || decode_kernel_kind(L, num_heads, requested) != 1)
+        return false;
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    const int64_t wgs = (int64_t)batch * L.num_kv_heads * (num_splits > 0 ? num_splits : 1);
+    if (wgs <= cus)
+        return true;
+    if (L.kv_type == KV_Q4_0 || (L.head_dim == 64 && L.kv_type != KV_F32))
+        return wgs <= 6 * cus;
+    if (L.head_dim == 128 && (L.kv_type == KV_F32 || L.kv_type == KV_F16) &&
+        split_tokens >= (L.kv_type == KV_F32 ? 2000 : 4096))
+        return false;
+    return wgs <= 2 * cus;
+}
+
 int decode_waves(const PoolLayout &L, int batch, int num_splits, int num_cus)
 {
     const int64_t wgs = (int64_t)batch * L.num_kv_heads * (num_splits > 0 ? num_splits : 1);
@@ -545,7 +589,8 @@ hipError_t launch_decode(const DecodeArgs &a, hipStream_t st)
     const int rows = a.batch * n_q * a.num_heads;
 #define GI_MERGE(HDv, Wv)                                                                              \
     hipLaunchKernelGGL((merge_splits<HDv, Wv>), dim3((unsigned)((rows + 4 / Wv - 1) / (4 / Wv))),       \
-                       dim3(256), 0, st, a.out, a.ws, rows, a.num_heads, L.num_kv_heads, a.num_splits)
+                       dim3(256), 0, st, a.out, a.ws, rows, a.num_heads, L.num_kv_heads, a.num_splits, \
+                       a.q_rot, a.rope, a.rope_max_pos, a.seq_lens)
     if (a.num_splits <= kMergeAhead) {
         if (L.head_dim == 128)
             GI_MERGE(128, 1);

@@ -1119,8 +1119,11 @@ __device__ __forceinline__ void softmax_pv_q(f4 s0, f4 s1, QBlock<KT, HD> &B, in
 }
 
 // Body of the decode kernels.  KT: KV_F16, or KV_Q8_0 / KV_Q4_0 (packed GP
-// only).  STG: fp16 pages with K staged through LDS (F16KStage).
-template <int KT, int HD, int GP, bool NT, bool PREFETCH, int NW, bool STG = false>
+// only).  STG: fp16 pages with K staged through LDS (F16KStage).  ROPE: a
+// decode step that also turns q and the token's K (DecodeArgs.rope); a
+// variant of its own, since the extra code costs the plain launch 0.15 us at
+// batch 1.
+template <int KT, int HD, int GP, bool NT, bool PREFETCH, int NW, bool ROPE, bool STG = false>
 __device__ __forceinline__ void decode_body(const DecodeArgs &a)
 {
     static_assert(!STG || (KT == KV_F16 && HD == 128), "staged fp16 pages at head_dim 128");
@@ -1170,11 +1173,27 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     int sblk = -1;          // the token's block, in the wave that stores it
     int64_t st_page = 0;    // and where the token goes
     int st_slot = 0;
+    // With ROPE the step's position turns q and the token's K; a
+    // position outside the table is flagged, its q left as it is and nothing
+    // stored, as the separate launch has it.
+    const float2 *cs = nullptr;
+    auto token_k = [&](int64_t e0, int d) {
+        const float x = a.new_k[e0 + d];
+        if constexpr (ROPE)
+            return rope_elem<HD>(d, x, a.new_k[e0 + (d ^ (HD / 2))], cs[d & (HD / 2 - 1)]);
+        return x;
+    };
     if (a.new_k) {
         const int raw = a.seq_lens[b], pos = raw - 1;
-        if (pos < 0 && threadIdx.x == 0 && split == 0 && a.status)
-            atomicOr(a.status, FLAG_BAD_SLOT);
-        if (raw == len && t0 <= pos && pos < t1) {
+        bool bad = pos < 0;
+        if constexpr (ROPE) {
+            bad = pos < 0 || pos >= a.rope_max_pos;
+            if (!bad)
+                cs = a.rope + (int64_t)pos * (HD / 2);
+        }
+        if (bad && threadIdx.x == 0 && split == 0 && a.status)
+            atomicOr(a.status, ROPE ? FLAG_BAD_POS : FLAG_BAD_SLOT);
+        if (!bad && raw == len && t0 <= pos && pos < t1) {
             const int64_t pg = a.block_tables[(int64_t)b * a.max_blocks + pos / P];
             const bool okp = pg >= 0 && pg < L.num_pages;
             if (!okp && threadIdx.x == 0 && a.status)
@@ -1186,10 +1205,11 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
                     st_slot = pos % P;
                 }
             } else {
-                const int64_t e = ((int64_t)b * L.num_kv_heads + kvh) * HD + threadIdx.x;
-                if (okp && threadIdx.x < HD)
-                    store_token_elem<KT>(L, a.append_base + pg * L.page_bytes, pos % P, kvh, threadIdx.x,
-                                         a.new_k[e], a.new_v[e], true);
+                const int64_t e0 = ((int64_t)b * L.num_kv_heads + kvh) * HD;
+                const int d = threadIdx.x;
+                if (okp && d < HD)
+                    store_token_elem<KT>(L, a.append_base + pg * L.page_bytes, pos % P, kvh, d, token_k(e0, d),
+                                         a.new_v[e0 + d], true);
                 __syncthreads();
             }
         }
@@ -1198,7 +1218,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
         const int64_t e0 = ((int64_t)b * L.num_kv_heads + kvh) * HD;
 #pragma unroll
         for (int d = lane; d < HD; d += 64)
-            store_token_elem<KT>(L, a.append_base + st_page * L.page_bytes, st_slot, kvh, d, a.new_k[e0 + d],
+            store_token_elem<KT>(L, a.append_base + st_page * L.page_bytes, st_slot, kvh, d, token_k(e0, d),
                                  a.new_v[e0 + d], true);
     };
 
@@ -1266,10 +1286,24 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
             qv[kk][5] = x1.y;
             qv[kk][6] = x1.z;
             qv[kk][7] = x1.w;
+        }
+        if (ROPE && cs) {
+            // a pair (d, d + HD / 2) is k-steps kk and kk + KK / 2 of one lane
+#pragma unroll
+            for (int kk = 0; kk < KK / 2; kk++)
+#pragma unroll
+                for (int v = 0; v < 8; v += 2) {
+                    const float4 t = *reinterpret_cast<const float4 *>(cs + 32 * kk + 8 * g + v);
+                    float *x = &qv[kk][v], *y = &qv[kk + KK / 2][v];
+                    rope_pair(x[0], y[0], t.x, t.y, &x[0], &y[0]);
+                    rope_pair(x[1], y[1], t.z, t.w, &x[1], &y[1]);
+                }
+        }
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
 #pragma unroll
             for (int v = 0; v < 8; v++)
                 mq = fmaxf(mq, fabsf(qv[kk][v]));
-        }
         mq = fmaxf(mq, __shfl_xor(mq, 16));
         mq = fmaxf(mq, __shfl_xor(mq, 32));
         const int qe = pow2_exponent_for(mq);
@@ -1566,8 +1600,37 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
         softmax_pv<HD, GP>(s0, s1, v, base, ok, t1, j, g, c, S);
     }
 
+    // An unsplit step with RoPE writes the turned q back: its pairs are read
+    // here and written after the barrier, which every wave's reads of q
+    // precede (no other workgroup reads these heads; merge_splits writes the
+    // q of split steps).
+    constexpr int QP = !ROPE ? 1 : GP ? (GP * HD / 2 + 64 * NW - 1) / (64 * NW) : 16 * HD / 2 / (64 * NW);
+    float2 qr[QP];
+    const bool turn = ROPE && cs && !wsp;
+    if (turn) {
+#pragma unroll
+        for (int i = 0; i < QP; i++) {
+            const int p = threadIdx.x + 64 * NW * i, d = p % (HD / 2);
+            if (p < G * HD / 2) {
+                const float *x = a.q + (qrow + p / (HD / 2)) * HD + d;
+                const float2 t = cs[d];
+                rope_pair(x[0], x[HD / 2], t.x, t.y, &qr[i].x, &qr[i].y);
+            }
+        }
+    }
     // every wave is done with its staging area before the merge reuses it
     __syncthreads();
+    if (turn) {
+#pragma unroll
+        for (int i = 0; i < QP; i++) {
+            const int p = threadIdx.x + 64 * NW * i, d = p % (HD / 2);
+            if (p < G * HD / 2) {
+                float *x = a.q_rot + (qrow + p / (HD / 2)) * HD + d;
+                x[0] = qr[i].x;
+                x[HD / 2] = qr[i].y;
+            }
+        }
+    }
     // wave totals -> LDS
     float lt = S.lsum;
     if constexpr (QUANT && GP == 4)
@@ -1634,25 +1697,26 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
 // are issued as soon as this block's K (then V) registers are consumed.
 // OCC: minimum waves per SIMD requested from the register allocator.  NW:
 // waves per workgroup (DecodeArgs.waves).
-template <int HD, int GP, bool NT, bool PREFETCH, int OCC, int NW = 4, bool STG = false>
+template <int HD, int GP, bool NT, bool PREFETCH, int OCC, int NW, bool ROPE, bool STG>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) void attn_mfma_f16(DecodeArgs a)
 {
-    decode_body<KV_F16, HD, GP, NT, PREFETCH, NW, STG>(a);
+    decode_body<KV_F16, HD, GP, NT, PREFETCH, NW, ROPE, STG>(a);
 }
 
 // f32 pages, packed form (GP = G in {1, 2, 4, 8}).  NW: waves per
 // workgroup, 4, or 8 at head dimension 64 (DecodeArgs.waves).
-template <int HD, int GP, bool NT, bool PREFETCH, int OCC, int NW = 4>
+template <int HD, int GP, bool NT, bool PREFETCH, int OCC, int NW, bool ROPE>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) void attn_mfma_f32(DecodeArgs a)
 {
-    decode_body<KV_F32, HD, GP, NT, PREFETCH, NW>(a);
+    decode_body<KV_F32, HD, GP, NT, PREFETCH, NW, ROPE>(a);
 }
 
-// q8_0 / q4_0 pages, packed form (GP = G in {1, 2, 4, 8}).
-template <int KT, int HD, int GP, bool NT, bool PREFETCH, int OCC, int NW = 4>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC))) void attn_mfma_q(DecodeArgs a)
+// q8_0 / q4_0 pages, packed form (GP = G in {1, 2, 4, 8}).  OMAX: at most so
+// many waves per SIMD.
+template <int KT, int HD, int GP, bool NT, bool PREFETCH, int OCC, int OMAX, int NW, bool ROPE>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(OCC, OMAX))) void attn_mfma_q(DecodeArgs a)
 {
-    decode_body<KT, HD, GP, NT, PREFETCH, NW>(a);
+    decode_body<KT, HD, GP, NT, PREFETCH, NW, ROPE>(a);
 }
 
 } // namespace mfma_decode
@@ -1693,47 +1757,52 @@ constexpr bool kDecodePack = true;
 // register loads.
 constexpr int kDecodeStgTokens = 4096;
 
-template <int HD, int GP>
+template <int HD, int GP, bool ROPE>
 static void launch_mfma_hd(const DecodeArgs &a, dim3 grid, hipStream_t st)
 {
     const int P = a.L.page_tokens;
     const bool stg = HD == 128 && GP != 0 && (P == 16 || P == 32);
     constexpr bool STG = HD == 128 && GP != 0;
+#define GI_H(NW, STGv)                                                                                         \
+    hipLaunchKernelGGL((mfma_decode::attn_mfma_f16<HD, GP, kDecodeNt, kDecodePrefetch, kDecodeOcc, NW, ROPE, STGv>), \
+                       grid, dim3(64 * NW), 0, st, a)
     if (a.waves == 8) {
         if (stg && a.split_tokens <= kDecodeStgTokens)
-            hipLaunchKernelGGL((mfma_decode::attn_mfma_f16<HD, GP, kDecodeNt, kDecodePrefetch, kDecodeOcc, 8, STG>),
-                               grid, dim3(512), 0, st, a);
+            GI_H(8, STG);
         else
-            hipLaunchKernelGGL((mfma_decode::attn_mfma_f16<HD, GP, kDecodeNt, kDecodePrefetch, kDecodeOcc, 8>),
-                               grid, dim3(512), 0, st, a);
+            GI_H(8, false);
     } else if (stg) {
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_f16<HD, GP, kDecodeNt, kDecodePrefetch, kDecodeOcc, 4, STG>),
-                           grid, dim3(256), 0, st, a);
+        GI_H(4, STG);
     } else {
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_f16<HD, GP, kDecodeNt, kDecodePrefetch, kDecodeOcc, 4>),
-                           grid, dim3(256), 0, st, a);
+        GI_H(4, false);
     }
+#undef GI_H
 }
 
 // q4_0 pages are bound by the vector ALU: three waves per SIMD (the
 // register allocator then keeps the kernel at 168 VGPRs, unspilled) measured
-// 0.487 against 0.522 ms per launch at batch 256 x 8192.  q8_0 pages are
-// bound by the texture path, where a third wave costs (0.855 against 0.78).
+// 0.487 against 0.522 ms per launch at batch 256 x 8192.  q8_0 pages at head
+// dimension 128 are bound by the texture path, where a third wave costs
+// (0.855 against 0.78; at 168 VGPRs, which would allow one, 0.642 against
+// 0.633 at batch 256 x 6144-8192): at most two with four heads per kv head.
+// With eight, three waves are the better (90 x 1500-3000 0.106 against 0.116).
 template <int KT>
 constexpr int kDecodeOccQ = KT == KV_Q4_0 ? 3 : kDecodeOcc;
+template <int KT, int HD, int GP>
+constexpr int kDecodeOccMaxQ = KT == KV_Q8_0 && HD == 128 && GP == 4 ? 2 : 8;
 
-template <int KT, int HD>
+template <int KT, int HD, bool ROPE>
 static void launch_mfma_q(const DecodeArgs &a, dim3 grid, hipStream_t st)
 {
-#define GI_Q(GPv)                                                                                        \
-    if (a.waves == 8)                                                                                    \
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_q<KT, HD, GPv, kDecodeNt, kDecodePrefetch,             \
-                                                     kDecodeOccQ<KT>, 8>),                              \
-                           grid, dim3(512), 0, st, a);                                                  \
-    else                                                                                                 \
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_q<KT, HD, GPv, kDecodeNt, kDecodePrefetch,             \
-                                                     kDecodeOccQ<KT>, 4>),                              \
-                           grid, dim3(256), 0, st, a)
+#define GI_QW(GPv, NW)                                                                                   \
+    hipLaunchKernelGGL((mfma_decode::attn_mfma_q<KT, HD, GPv, kDecodeNt, kDecodePrefetch, kDecodeOccQ<KT>, \
+                                                 kDecodeOccMaxQ<KT, HD, GPv>, NW, ROPE>),                      \
+                       grid, dim3(64 * NW), 0, st, a)
+#define GI_Q(GPv)         \
+    if (a.waves == 8)     \
+        GI_QW(GPv, 8);    \
+    else                  \
+        GI_QW(GPv, 4)
     switch (a.num_heads / a.L.num_kv_heads) {
     case 1: GI_Q(1); break;
     case 2: GI_Q(2); break;
@@ -1741,22 +1810,22 @@ static void launch_mfma_q(const DecodeArgs &a, dim3 grid, hipStream_t st)
     default: GI_Q(8); break;
     }
 #undef GI_Q
+#undef GI_QW
 }
 
-template <int HD>
+template <int HD, bool ROPE>
 static void launch_mfma_f32(const DecodeArgs &a, dim3 grid, hipStream_t st)
 {
     // eight waves (decode_waves) only at head dimension 64: 8 x 16 KiB stages
     constexpr int NW8 = HD == 64 ? 8 : 4;
-#define GI_F(GPv)                                                                                 \
-    if (a.waves == 8)                                                                             \
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_f32<HD, GPv, kDecodeNt, kDecodePrefetch,       \
-                                                       kDecodeOcc, NW8>),                         \
-                           grid, dim3(64 * NW8), 0, st, a);                                       \
-    else                                                                                          \
-        hipLaunchKernelGGL((mfma_decode::attn_mfma_f32<HD, GPv, kDecodeNt, kDecodePrefetch,       \
-                                                       kDecodeOcc>),                              \
-                           grid, dim3(256), 0, st, a)
+#define GI_FW(GPv, NW)                                                                                   \
+    hipLaunchKernelGGL((mfma_decode::attn_mfma_f32<HD, GPv, kDecodeNt, kDecodePrefetch, kDecodeOcc, NW, ROPE>), \
+                       grid, dim3(64 * NW), 0, st, a)
+#define GI_F(GPv)          \
+    if (a.waves == 8)      \
+        GI_FW(GPv, NW8);   \
+    else                   \
+        GI_FW(GPv, 4)
     switch (a.num_heads / a.L.num_kv_heads) {
     case 1: GI_F(1); break;
     case 2: GI_F(2); break;
@@ -1764,49 +1833,45 @@ static void launch_mfma_f32(const DecodeArgs &a, dim3 grid, hipStream_t st)
     default: GI_F(8); break;
     }
 #undef GI_F
+#undef GI_FW
 }
 
-template <int HD>
+template <int HD, bool ROPE>
 static void launch_mfma_g(const DecodeArgs &a, dim3 grid, hipStream_t st)
 {
     switch (a.num_heads / a.L.num_kv_heads) {
-    case 1: launch_mfma_hd<HD, kDecodePack ? 1 : 0>(a, grid, st); break;
-    case 2: launch_mfma_hd<HD, kDecodePack ? 2 : 0>(a, grid, st); break;
-    case 4: launch_mfma_hd<HD, kDecodePack ? 4 : 0>(a, grid, st); break;
-    case 8: launch_mfma_hd<HD, kDecodePack ? 8 : 0>(a, grid, st); break;
-    default: launch_mfma_hd<HD, 0>(a, grid, st); break;
+    case 1: launch_mfma_hd<HD, kDecodePack ? 1 : 0, ROPE>(a, grid, st); break;
+    case 2: launch_mfma_hd<HD, kDecodePack ? 2 : 0, ROPE>(a, grid, st); break;
+    case 4: launch_mfma_hd<HD, kDecodePack ? 4 : 0, ROPE>(a, grid, st); break;
+    case 8: launch_mfma_hd<HD, kDecodePack ? 8 : 0, ROPE>(a, grid, st); break;
+    default: launch_mfma_hd<HD, 0, ROPE>(a, grid, st); break;
+    }
+}
+
+template <int HD, bool ROPE>
+static void launch_mfma_kt(const DecodeArgs &a, dim3 grid, hipStream_t st)
+{
+    switch (a.L.kv_type) {
+    case KV_Q8_0: launch_mfma_q<KV_Q8_0, HD, ROPE>(a, grid, st); break;
+    case KV_Q4_0: launch_mfma_q<KV_Q4_0, HD, ROPE>(a, grid, st); break;
+    case KV_F32: launch_mfma_f32<HD, ROPE>(a, grid, st); break;
+    default: launch_mfma_g<HD, ROPE>(a, grid, st); break;
     }
 }
 
 hipError_t launch_decode_mfma(const DecodeArgs &a, hipStream_t st)
 {
     dim3 grid(a.num_splits, a.L.num_kv_heads, a.batch);
-    const bool h128 = a.L.head_dim == 128;
-    switch (a.L.kv_type) {
-    case KV_Q8_0:
-        if (h128)
-            launch_mfma_q<KV_Q8_0, 128>(a, grid, st);
+    if (a.L.head_dim == 128) {
+        if (a.rope)
+            launch_mfma_kt<128, true>(a, grid, st);
         else
-            launch_mfma_q<KV_Q8_0, 64>(a, grid, st);
-        break;
-    case KV_Q4_0:
-        if (h128)
-            launch_mfma_q<KV_Q4_0, 128>(a, grid, st);
+            launch_mfma_kt<128, false>(a, grid, st);
+    } else {
+        if (a.rope)
+            launch_mfma_kt<64, true>(a, grid, st);
         else
-            launch_mfma_q<KV_Q4_0, 64>(a, grid, st);
-        break;
-    case KV_F32:
-        if (h128)
-            launch_mfma_f32<128>(a, grid, st);
-        else
-            launch_mfma_f32<64>(a, grid, st);
-        break;
-    default:
-        if (h128)
-            launch_mfma_g<128>(a, grid, st);
-        else
-            launch_mfma_g<64>(a, grid, st);
-        break;
+            launch_mfma_kt<64, false>(a, grid, st);
     }
     return hipGetLastError();
 }

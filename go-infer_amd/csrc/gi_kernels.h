@@ -73,6 +73,14 @@ struct DecodeArgs {
     // does; null for attention alone.  append_base is base, writable.
     const float *new_k, *new_v;
     uint8_t *append_base;
+    // RoPE over the whole head dimension inside such a step (null: none):
+    // q (raw, [batch][num_heads][head_dim]) is turned at seq_lens[b] - 1 by
+    // every reader and written back to q_rot (q, writable) after the last
+    // read, and new_k is turned before it is stored.  Entry j of position p
+    // is rope[p * head_dim / 2 + j].
+    const float2 *rope;
+    int rope_max_pos;
+    float *q_rot;
 };
 
 // Bytes of split-K workspace needed for a decode launch.
@@ -81,6 +89,11 @@ size_t decode_workspace_bytes(const PoolLayout &L, int batch, int num_heads, int
 // Whether a decode step's token store goes into the matrix-core decode
 // launch (DecodeArgs.new_k) for this grid, rather than an append launch.
 bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num_cus);
+
+// Whether a step's rotary embedding and token store go into the decode launch
+// (DecodeArgs.rope), rather than a rope + append launch before it.
+bool decode_fuses_rope(const PoolLayout &L, int batch, int num_heads, int requested, int rope_half,
+                       int split_tokens, int num_splits, int num_cus);
 
 // Picks (split_tokens, num_splits) for a batch whose longest sequence has
 // max_len tokens, so the grid fills the device.

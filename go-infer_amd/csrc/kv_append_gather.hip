@@ -538,20 +538,6 @@ hipError_t append_any(const PoolLayout &L, uint8_t *base, int n_tok, const Dest 
     return hipGetLastError();
 }
 
-// One rotated pair of ApplyRoPE (kernels.go:31-33): each product is rounded
-// before the sum or difference, as Go's amd64 code evaluates it, so no
-// multiply-add may be contracted here.
-__device__ __forceinline__ void rope_pair(float x0, float x1, float c, float s, float *y0, float *y1)
-{
-#pragma clang fp contract(off)
-    float a = x0 * c;
-    float b = x1 * s;
-    float e = x0 * s;
-    float f = x1 * c;
-    *y0 = a - b;
-    *y1 = e + f;
-}
-
 // Rotates the first 2*rh dims of each of n_heads heads of x (head stride hd)
 // into y; the dims past 2*rh are copied.  Pair p = (head, j) is (j, j + rh)
 // of that head.  Pairs [p0, p0 + step * k) go to the threads of the

@@ -605,11 +605,13 @@ int gi_paged_gather(gi_paged *h, int layer, const int32_t *block_table, int n_to
 }
 
 // fixed_ws: the allocate-nothing form's scratch (fixed_cap bytes) in place
-// of the handle's growable workspace.
+// of the handle's growable workspace.  new_k, new_v: a decode step's token,
+// stored first.  rope_q (q, writable): that step turns q and new_k.
 static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                          float *out, const int32_t *block_tables, int max_blocks,
                          const int32_t *seq_lens, int max_seq_len, float scale, void *fixed_ws = nullptr,
-                         size_t fixed_cap = 0, const float *new_k = nullptr, const float *new_v = nullptr)
+                         size_t fixed_cap = 0, const float *new_k = nullptr, const float *new_v = nullptr,
+                         float *rope_q = nullptr)
 {
     gi::DecodeArgs a{};
     a.L = h->L;
@@ -696,9 +698,24 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
     if (new_k) {
         // a decode step: the token goes into the decode launch where that
         // pays (one round of workgroups), else into an append launch first
-        if (gi::decode_fuses_append(h->L, batch, a.num_splits, h->num_cus)) {
+        const bool fuse = rope_q ? gi::decode_fuses_rope(h->L, batch, num_heads, h->decode_kernel, h->rope_half,
+                                                         a.split_tokens, a.num_splits, h->num_cus)
+                                 : gi::decode_fuses_append(h->L, batch, a.num_splits, h->num_cus);
+        if (fuse) {
             a.new_k = new_k;
             a.new_v = new_v;
+            if (rope_q) {
+                a.rope = h->d_rope;
+                a.rope_max_pos = h->rope_max_pos;
+                a.q_rot = rope_q;
+            }
+        } else if (rope_q) {
+            const hipError_t e = gi::launch_rope_append(h->L, a.append_base, batch, nullptr, nullptr, block_tables,
+                                                        max_blocks, seq_lens,
+                                                        rope_args(h, num_heads, nullptr, rope_q, rope_q), new_k, new_v,
+                                                        h->d_status, h->stream);
+            if (e != hipSuccess)
+                return hip_fail(e, "decode step: rope + append");
         } else {
             const hipError_t e = gi::launch_append_at_len(h->L, a.append_base, batch, block_tables, max_blocks,
                                                           seq_lens, new_k, new_v, h->d_status, h->stream);
@@ -800,13 +817,10 @@ int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, 
     if (batch == 0)
         return GI_OK;
     std::lock_guard<std::mutex> g(h->mu);
-    hipError_t e = gi::launch_rope_append(h->L, h->layer_base[(size_t)layer], batch, nullptr, nullptr,
-                                          block_tables, max_blocks, seq_lens,
-                                          rope_args(h, num_heads, nullptr, q, q), k, v, h->d_status,
-                                          h->stream);
-    if (e != hipSuccess)
-        return hip_fail(e, "gi_paged_rope_decode_step: rope + append");
-    return decode_locked(h, layer, batch, num_heads, q, out, block_tables, max_blocks, seq_lens, max_seq_len, scale);
+    // RoPE and the store go into the decode launch where they fit
+    // (decode_fuses_append, decode_fuses_rope), else into a launch before it
+    return decode_locked(h, layer, batch, num_heads, q, out, block_tables, max_blocks, seq_lens, max_seq_len, scale,
+                         nullptr, 0, k, v, q);
 }
 
 int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len, int num_heads,

@@ -47,6 +47,30 @@ __device__ __forceinline__ void quant_store_q4(const PoolLayout &L, uint8_t *pg,
     }
 }
 
+// One rotated pair of ApplyRoPE (kernels.go:31-33): each product is rounded
+// before the sum or difference, as Go's amd64 code evaluates it, so no
+// multiply-add may be contracted here.
+__device__ __forceinline__ void rope_pair(float x0, float x1, float c, float s, float *y0, float *y1)
+{
+#pragma clang fp contract(off)
+    float a = x0 * c;
+    float b = x1 * s;
+    float e = x0 * s;
+    float f = x1 * c;
+    *y0 = a - b;
+    *y1 = e + f;
+}
+
+// Element d of a head of HD dimensions that is turned whole: x is the element,
+// y the other of its pair (dimension d ^ HD / 2), t the pair's (cos, sin).
+template <int HD>
+__device__ __forceinline__ float rope_elem(int d, float x, float y, float2 t)
+{
+    float y0, y1;
+    rope_pair(d < HD / 2 ? x : y, d < HD / 2 ? y : x, t.x, t.y, &y0, &y1);
+    return d < HD / 2 ? y0 : y1;
+}
+
 // Element d of kv head kvh of one token (K value kx, V value vx) into slot s
 // of page pg: f32 copied, f16 truncated (FP32ToFP16, fp16.go:38-69), q8_0 and
 // q4_0 quantised per 32-element block (QuantizeQ8_0 / QuantizeQ4_0,

@@ -195,3 +195,85 @@ def test_rope_bad_position_and_errors(gi, oracle, dev):
     ko, _ = pool.Get(0, t, 1)
     pool.synchronize()
     assert not ko.cpu().numpy().any()                     # nothing stored for it
+
+
+@pytest.mark.parametrize("kv_type", [0, 1, 2, 3], ids=["f32", "f16", "q8_0", "q4_0"])
+@pytest.mark.parametrize("H,kvh,hd,P,rd,lens", [
+    (32, 8, 128, 16, 128, [90]), (32, 4, 64, 16, 64, [33, 1, 511]),         # one split
+    (64, 8, 128, 32, 128, [700]), (8, 8, 64, 16, 64, [1025, 900]),           # merged by one wave
+    (16, 2, 128, 16, 128, [4000]), (16, 4, 64, 32, 64, [64, 4100]),          # merged by four
+    (32, 8, 128, 64, 128, [640, 65]), (16, 8, 128, 16, 64, [300]),           # wide pages; half of a head turned
+    (32, 8, 128, 16, 128, [40 + i for i in range(40)]),                      # four-wave workgroups
+    (32, 8, 128, 16, 128, [0, 50, 60, 33]),                                  # a position before the table's start
+])
+def test_rope_decode_step_equals_its_parts(gi, oracle, dev, kv_type, H, kvh, hd, P, rd, lens):
+    """The step that turns q and stores the token inside the decode launch
+    leaves the bits of RoPEWrite followed by AttentionGQA: q, the pages, and
+    the output.  The table ends at the last position but one of the last
+    sequence of three or more, whose q, pages and status must show that."""
+    import torch
+    max_pos = max(lens) if len(lens) < 3 else lens[-1] - 1
+    kv_dim = kvh * hd
+    rng = np.random.default_rng(5)
+    pages = sum((n + P - 1) // P for n in lens) + 4
+    ids = rng.permutation(pages).astype(np.int32)
+    bt = np.zeros((len(lens), max(1, max((n + P - 1) // P for n in lens))), np.int32)
+    o = 0
+    for i, n in enumerate(lens):
+        m = (n + P - 1) // P
+        bt[i, :m] = ids[o:o + m]
+        o += m
+    btd = torch.from_numpy(bt).to(dev)
+    sl = torch.tensor(lens, dtype=torch.int32, device=dev)
+    pools = []
+    for _ in range(2):
+        pool = gi.PagedKVCache(1, kvh, hd, P, pages, kv_type)
+        pool.SetRoPE(10000.0, rd, max_pos)
+        for i, n in enumerate(lens):
+            if n > 1:
+                t = np.arange(n - 1)
+                pool.Write(0, torch.from_numpy(bt[i, t // P].astype(np.int32)).to(dev),
+                           torch.from_numpy((t % P).astype(np.int32)).to(dev),
+                           torch.from_numpy(oracle.normal(30 + i, (n - 1, kv_dim))).to(dev),
+                           torch.from_numpy(oracle.normal(60 + i, (n - 1, kv_dim))).to(dev))
+        pools.append(pool)
+    B = len(lens)
+    q = torch.from_numpy(oracle.normal(7, (B, H * hd))).to(dev)
+    k = torch.from_numpy(oracle.normal(8, (B, kv_dim))).to(dev)
+    v = torch.from_numpy(oracle.normal(9, (B, kv_dim))).to(dev)
+    scale = oracle.attn_scale(hd)
+    bad = [i for i, n in enumerate(lens) if not 0 < n <= max_pos]
+
+    def status(pool):
+        try:
+            pool.synchronize()
+            return 0
+        except gi.GIError as e:
+            return e.value if hasattr(e, "value") else e.code
+
+    fused, parts = pools
+    qf, of = q.clone(), torch.full_like(q, float("nan"))
+    fused.RoPEDecodeStep(of, qf, k, v, 0, btd, sl, H, scale, max(lens))
+    sf = status(fused)
+    qp, op = q.clone(), torch.full_like(q, float("nan"))
+    pos = np.array(lens, np.int32) - 1
+    at = np.maximum(pos, 0)
+    parts.RoPEWrite(0, torch.from_numpy(pos).to(dev),
+                    torch.from_numpy(bt[np.arange(B), at // P].copy()).to(dev),
+                    torch.from_numpy((at % P).astype(np.int32)).to(dev), qp, k, v)
+    sp = status(parts)
+    assert sf == sp and (sf != 0) == bool(bad), (sf, sp, bad)
+    parts.AttentionGQA(op, qp, 0, btd, sl, H, scale, max(lens))
+    parts.synchronize()
+    assert torch.equal(qf, qp)
+    for i in bad:
+        assert torch.equal(qf[i], q[i])
+    for i, n in enumerate(lens):
+        if n == 0:
+            continue
+        m = n - 1 if i in bad else n
+        t = btd[i, :(n + P - 1) // P].contiguous()
+        for x, y in zip(fused.Get(0, t, m), parts.Get(0, t, m)):
+            assert torch.equal(x, y), i
+    good = [i for i in range(B) if i not in bad]
+    assert torch.equal(of[good], op[good])
