@@ -136,7 +136,19 @@ struct PrefillArgs {
     float scale;
     int *status;
     int kernel; // -1 automatic, 0 vector ALU, 1 matrix core
+    // prefill_plan's choice: splits of the context (1: none) and whether a
+    // wave takes one group of 16 columns where it could take two.  ws holds
+    // prefill_workspace_bytes.
+    int num_splits;
+    bool narrow;
+    float *ws;
 };
+
+// Context splits and column groups of a prefill launch whose block tables
+// map `mapped` tokens per sequence.
+void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
+                  int num_cus, int *num_splits, bool *narrow);
+size_t prefill_workspace_bytes(const PrefillArgs &a);
 
 hipError_t launch_prefill(const PrefillArgs &a, hipStream_t st);
 

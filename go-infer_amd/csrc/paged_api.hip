@@ -850,6 +850,24 @@ int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len,
     p.scale = scale;
     p.status = h->d_status;
     p.kernel = h->decode_kernel;
+    gi::prefill_plan(h->L, batch, chunk_len, num_heads, (int64_t)max_blocks * h->L.page_tokens, p.kernel, h->num_cus,
+                     &p.num_splits, &p.narrow);
+    const size_t need = gi::prefill_workspace_bytes(p);
+    if (need) {
+        // a capturing stream cannot allocate: the context stays in one piece
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        hipError_t e = need > h->plan_ws.bytes ? hipStreamIsCapturing(h->stream, &cs) : hipSuccess;
+        if (e != hipSuccess)
+            return hip_fail(e, "gi_paged_prefill_attention: hipStreamIsCapturing");
+        if (cs != hipStreamCaptureStatusNone) {
+            p.num_splits = 1;
+        } else {
+            rc = gi::devbuf_reserve(h->plan_ws, need, h->stream, "prefill attention");
+            if (rc)
+                return rc;
+            p.ws = (float *)h->plan_ws.ptr;
+        }
+    }
     hipError_t e = gi::launch_prefill(p, h->stream);
     return e == hipSuccess ? GI_OK : hip_fail(e, "gi_paged_prefill_attention");
 }

@@ -25,6 +25,7 @@
 #include "gi_kernels.h"
 #include "mfma_ops.h"
 
+#include <algorithm>
 #include <math.h>
 #include <type_traits>
 
@@ -1575,9 +1576,39 @@ struct WaveAttn {
                 o[cg][nb] *= f;
     }
 
-    __device__ __forceinline__ void finish(const PrefillArgs &a, int b, int kvh, int col0, int j, int g)
+    // part: which split of the context this is (-1: all of it).  A split
+    // leaves (m2, l) and the unnormalised O of its columns in a.ws for
+    // merge_prefill.
+    __device__ __forceinline__ void finish(const PrefillArgs &a, int b, int kvh, int col0, int j, int g,
+                                           int part = -1)
     {
         const int H = a.num_heads, G = H / a.L.num_kv_heads, chunk = a.chunk_len;
+        if (part >= 0) {
+            const int64_t rows = (int64_t)a.batch * chunk * H;
+            float2 *ml = reinterpret_cast<float2 *>(a.ws) + part * rows;
+            float *ow = a.ws + 2 * a.num_splits * rows + part * rows * HD;
+#pragma unroll
+            for (int cg = 0; cg < NCG; cg++) {
+                float lt = lsum[cg];
+                lt += __shfl_xor(lt, 16);
+                lt += __shfl_xor(lt, 32);
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float l = __shfl(lt, 4 * g + r), m = __shfl(m2[cg], 4 * g + r);
+                    const int c = col0 + 16 * cg + 4 * g + r;
+                    const int qi = c / G;
+                    if (qi >= chunk)
+                        continue;
+                    const int64_t row = ((int64_t)b * chunk + qi) * H + kvh * G + c % G;
+                    if (j == 0)
+                        ml[row] = float2{m, l};
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++)
+                        ow[row * HD + 16 * nb + j] = o[cg][nb][r];
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int cg = 0; cg < NCG; cg++) {
             float lt = lsum[cg];
@@ -1600,6 +1631,24 @@ struct WaveAttn {
     }
 };
 
+// Tokens per split of a context of len tokens cut in at most n: whole blocks,
+// at least kMinSplit.  Contexts of one chunk stay whole (us per 512-token
+// chunk from position 0, Llama-3-8B shape, whole / in two: fp16 28.7 / 30.5,
+// q8_0 36.1 / 38.5, q4_0 32.3 / 36.1); f32 pages and q8_0 pages at head
+// dimension 64, whose blocks take longest, from 384 tokens only (f32 at 64
+// 33.2 / 28.4, q8_0 at 64 30.5 / 28.0).
+constexpr int kMinSplit = 256;
+__host__ __device__ __forceinline__ int whole_len(const PoolLayout &L)
+{
+    return L.kv_type == KV_F32 || (L.kv_type == KV_Q8_0 && L.head_dim == 64) ? 384 : 512;
+}
+__device__ __forceinline__ int split_len(const PoolLayout &L, int len, int n)
+{
+    if (len <= whole_len(L))
+        return whole_len(L);
+    return max(kMinSplit, ((len + n - 1) / n + kTB - 1) / kTB * kTB);
+}
+
 // Work split shared by the staged kernels: the workgroup's columns, the
 // context each wave and the workgroup must cover, and the block-table reads.
 // A tile is the NW * 16 * NCG consecutive columns of one workgroup.  PAIRED
@@ -1608,16 +1657,24 @@ struct WaveAttn {
 // short causal range and a long one share each SIMD and every workgroup gets
 // about the same work; each half then decides alone which blocks it sees
 // whole (wg_full is per half).
-template <int P, int NCG, int NW = 4, bool PAIRED = false>
+//
+// SPLIT: blockIdx.x holds split * tiles + tile, and the workgroup covers the
+// context tokens [t0, t0 + per) of split_len; everything else stays in
+// absolute token positions.  part is the split, or -1 if the sequence is
+// short enough for one.
+template <int P, int NCG, int NW = 4, bool PAIRED = false, bool SPLIT = false>
 struct PrefillWork {
     int wx, kvh, b, tid, lane, w, j, g, start, mapped, col0, wave_len, wg_full, wg_len;
+    int t0 = 0, part = -1;
     bool wave_active;
     const int32_t *bt;
 
     __device__ __forceinline__ PrefillWork(const PrefillArgs &a)
     {
         constexpr int WCOLS = 16 * NCG;
-        wx = gridDim.x - 1 - blockIdx.x; // heaviest (latest-query) workgroups first
+        const int tiles = SPLIT ? gridDim.x / a.num_splits : gridDim.x;
+        const int tile = SPLIT ? blockIdx.x % tiles : blockIdx.x;
+        wx = tiles - 1 - tile; // heaviest (latest-query) workgroups first
         kvh = blockIdx.y;
         b = blockIdx.z;
         tid = threadIdx.x;
@@ -1631,7 +1688,7 @@ struct PrefillWork {
         mapped = a.max_blocks * P;
         auto len = [&](int col) { return min(start + min(col / G, chunk - 1) + 1, mapped); };
         if (PAIRED) {
-            const int ta = wx, tb = gridDim.x - 1 - wx; // tiles of the two halves
+            const int ta = wx, tb = tiles - 1 - wx; // tiles of the two halves
             const int t = w < NW / 2 ? ta : tb;
             col0 = (t * NW + w) * WCOLS;
             // shortest column of this half
@@ -1646,7 +1703,20 @@ struct PrefillWork {
         wave_active = col0 / G < chunk;
         if (start + chunk > mapped && tid == 0 && a.status)
             atomicOr(a.status, FLAG_BAD_SLOT);
+        if (SPLIT) {
+            const int len = min(start + chunk, mapped), per = split_len(a.L, len, a.num_splits);
+            const int split = blockIdx.x / tiles;
+            t0 = split * per;
+            part = per < len ? split : -1;
+            const int t1 = t0 + per;
+            wave_len = min(wave_len, t1);
+            wg_full = min(wg_full, t1);
+            wg_len = min(wg_len, t1);
+        }
     }
+
+    // SPLIT: no column of the workgroup reaches this split's tokens.
+    __device__ __forceinline__ bool empty() const { return SPLIT && t0 >= wg_len; }
 
     // Whether the block at `base` is whole for every column of the workgroup
     // (PAIRED: of this wave's half): all its tokens valid and before the
@@ -1672,12 +1742,14 @@ struct PrefillWork {
 
 // NW waves per workgroup share its staging: 4, or 8 (two per SIMD in one
 // workgroup, so that one workgroup per CU holds two staging buffers).
-template <int HD, int KT, int P, int NBUF, int NCG, int NW>
+template <int HD, int KT, int P, int NBUF, int NCG, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void attn_prefill_lds(PrefillArgs a)
 {
     constexpr bool F32 = KT == KV_F32;
     static_assert(!F32 || NBUF == 1, "f32 pages exchange block maxima at the single-buffer barrier");
-    const PrefillWork<P, NCG, NW> W(a);
+    const PrefillWork<P, NCG, NW, false, SPLIT> W(a);
+    if (W.empty())
+        return;
     __shared__ Lds<HD, KT, NBUF> S;
     __shared__ float s_bmax[NW][2]; // f32 pages: per-wave |K|, |V| maxima of the block being staged
     WaveAttn<HD, KT, NCG> A;
@@ -1711,10 +1783,10 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_lds(PrefillArgs a)
             vsc_run = block_scale(mv, vsc_run);
         }
     };
-    int tb = W.table(0);
-    uint64_t mask_c = W.valid_mask(a, tb, 0);
+    int tb = W.table(W.t0);
+    uint64_t mask_c = W.valid_mask(a, tb, W.t0);
     stage_load<HD, KT, P, NW>(a, W.kvh, W.tid, W.w, tb, R);
-    tb = W.table(kTB);
+    tb = W.table(W.t0 + kTB);
     f32_scales(mask_c);
     stage_store<HD, KT, P, NBUF, NW>(a, W.kvh, W.tid, W.w, 0, mask_c, R, S, ksc_run, vsc_run, A.neg1);
     ksc_cur = ksc_run;
@@ -1722,7 +1794,7 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_lds(PrefillArgs a)
     __syncthreads();
 
     // One staged block; FULL: no column of the workgroup needs masking.
-    int base = 0, it = 0;
+    int base = W.t0, it = 0;
     auto step = [&](auto full) {
         constexpr bool FULL = decltype(full)::value;
         const int buf = NBUF == 2 ? (it & 1) : 0;
@@ -1768,7 +1840,7 @@ __global__ __launch_bounds__(64 * NW) void attn_prefill_lds(PrefillArgs a)
     if (W.wave_active) {
         if (F32 && vsc_o != 0.0f)
             A.scale_o(pow2_recip(vsc_o));
-        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g);
+        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g, W.part);
     }
 }
 
@@ -1861,11 +1933,11 @@ __device__ __forceinline__ void wait_direct_loads()
 // n + 1) and wait for at the end of the next phase 1.  Each group runs its
 // own copy of the loop (pp_loop<GB>), so that neither carries the other's
 // live values; both pass the same barriers.
-template <int HD, int P, int NCG>
+template <int HD, int P, int NCG, bool SPLIT>
 struct PingPong {
     static constexpr int NW = 8;
     const PrefillArgs &a;
-    const PrefillWork<P, NCG, NW, true> &W;
+    const PrefillWork<P, NCG, NW, true, SPLIT> &W;
     LdsDirect<HD> &S;
     WaveAttn<HD, KV_F16, NCG> &A;
 
@@ -1876,12 +1948,12 @@ struct PingPong {
     __device__ __forceinline__ void run(int tbv, int tbk, uint64_t mask_c, uint64_t mask_n, int nblk)
     {
         f4 s[NCG][2][2]; // a block's scores, then its P (softmax_block)
-        if (GB && live(0))
+        if (GB && live(W.t0))
             A.qk_block(S, 0, s, W.j, W.g);
         int n = 0;
         auto step = [&](auto full) {
             constexpr bool FULL = decltype(full)::value;
-            const int base = n * kTB, cur = n & 1;
+            const int base = W.t0 + n * kTB, cur = n & 1;
             // phase 1
             if (!GB) {
                 __builtin_amdgcn_s_setprio(1);
@@ -1924,49 +1996,51 @@ struct PingPong {
             mask_n = mask_nn;
             n++;
         };
-        while (n < nblk && W.block_full(n * kTB, mask_c))
+        while (n < nblk && W.block_full(W.t0 + n * kTB, mask_c))
             step(std::true_type{});
         while (n < nblk)
             step(std::false_type{});
-        if (!GB && nblk > 0 && live((nblk - 1) * kTB))
+        if (!GB && nblk > 0 && live(W.t0 + (nblk - 1) * kTB))
             A.pv_block(S, (nblk - 1) & 1, s, W.j, W.g);
     }
 };
 
-template <int HD, int P, int NCG>
+template <int HD, int P, int NCG, bool SPLIT>
 __global__ __launch_bounds__(512) void attn_prefill_pp(PrefillArgs a)
 {
-    constexpr int NW = PingPong<HD, P, NCG>::NW;
-    const PrefillWork<P, NCG, NW, true> W(a);
+    constexpr int NW = PingPong<HD, P, NCG, SPLIT>::NW;
+    const PrefillWork<P, NCG, NW, true, SPLIT> W(a);
+    if (W.empty())
+        return;
     __shared__ LdsDirect<HD> S;
     WaveAttn<HD, KV_F16, NCG> A;
-    const int nblk = (W.wg_len + kTB - 1) / kTB;
+    const int nblk = (W.wg_len - W.t0 + kTB - 1) / kTB;
 
     // prologue: K and V of block 0, K of block 1, in flight while Q is
     // loaded and split
-    const int tb = W.table(0);
-    const int tbv = W.table(kTB); // block whose V is issued next
+    const int tb = W.table(W.t0);
+    const int tbv = W.table(W.t0 + kTB); // block whose V is issued next
     issue_k<HD, P, NW>(a, W.kvh, W.w, W.lane, tb, S, 0);
     issue_v<HD, P, NW>(a, W.kvh, W.w, W.lane, tb, S, 0);
     issue_k<HD, P, NW>(a, W.kvh, W.w, W.lane, tbv, S, 1);
-    const int tbk = W.table(2 * kTB); // block whose K is issued next
+    const int tbk = W.table(W.t0 + 2 * kTB); // block whose K is issued next
     A.template init<true>(a, W.b, W.kvh, W.col0, W.start, W.mapped, W.wave_active, W.j, W.g);
-    const uint64_t mask_c = W.valid_mask(a, tb, 0);
-    const uint64_t mask_n = W.valid_mask(a, tbv, kTB);
+    const uint64_t mask_c = W.valid_mask(a, tb, W.t0);
+    const uint64_t mask_n = W.valid_mask(a, tbv, W.t0 + kTB);
     wait_direct_loads();
     __syncthreads();
     if (mask_c != ~0ull) {
         zero_dead_v<HD, 64 * NW>(S, 0, mask_c, W.tid);
         __syncthreads();
     }
-    PingPong<HD, P, NCG> pp{a, W, S, A};
+    PingPong<HD, P, NCG, SPLIT> pp{a, W, S, A};
     if (W.w >= NW / 2)
         pp.template run<true>(tbv, tbk, mask_c, mask_n, nblk);
     else
         pp.template run<false>(tbv, tbk, mask_c, mask_n, nblk);
     wait_direct_loads(); // loads issued past the end, before the workgroup's LDS is released
     if (W.wave_active)
-        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g);
+        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g, W.part);
 }
 
 // Quantised pages (q8_0, q4_0; head_dim 128), two waves per SIMD in
@@ -1978,11 +2052,11 @@ __global__ __launch_bounds__(512) void attn_prefill_pp(PrefillArgs a)
 // block n:
 //   phase 1: A: P V (n - 1), scores (n)      B: softmax (n), K (n + 1) staged
 //   phase 2: A: softmax (n), V (n + 1) staged B: P V (n), scores (n + 1)
-template <int HD, int KT, int P, int NCG>
+template <int HD, int KT, int P, int NCG, bool SPLIT>
 struct PingPongQ {
     static constexpr int NW = 8;
     const PrefillArgs &a;
-    const PrefillWork<P, NCG, NW, true> &W;
+    const PrefillWork<P, NCG, NW, true, SPLIT> &W;
     Lds<HD, KT, 2, true> &S;
     WaveAttn<HD, KT, NCG> &A;
 
@@ -1995,12 +2069,12 @@ struct PingPongQ {
     {
         const int st = W.tid & 255;
         f4 s[NCG][2][2]; // a block's scores, then its P (softmax_block)
-        if (GB && live(0))
+        if (GB && live(W.t0))
             A.qk_block_kc(S, 0, s, W.j, W.g);
         int n = 0;
         auto step = [&](auto full) {
             constexpr bool FULL = decltype(full)::value;
-            const int base = n * kTB, cur = n & 1;
+            const int base = W.t0 + n * kTB, cur = n & 1;
             // phase 1
             if (!GB) {
                 __builtin_amdgcn_s_setprio(1);
@@ -2041,30 +2115,32 @@ struct PingPongQ {
             mask_n = mask_nn;
             n++;
         };
-        while (n < nblk && W.block_full(n * kTB, mask_c))
+        while (n < nblk && W.block_full(W.t0 + n * kTB, mask_c))
             step(std::true_type{});
         while (n < nblk)
             step(std::false_type{});
-        if (!GB && nblk > 0 && live((nblk - 1) * kTB))
+        if (!GB && nblk > 0 && live(W.t0 + (nblk - 1) * kTB))
             A.pv_block(S, (nblk - 1) & 1, s, W.j, W.g);
     }
 };
 
-template <int HD, int KT, int P, int NCG>
+template <int HD, int KT, int P, int NCG, bool SPLIT>
 __global__ __launch_bounds__(512) void attn_prefill_ppq(PrefillArgs a)
 {
-    constexpr int NW = PingPongQ<HD, KT, P, NCG>::NW;
-    const PrefillWork<P, NCG, NW, true> W(a);
+    constexpr int NW = PingPongQ<HD, KT, P, NCG, SPLIT>::NW;
+    const PrefillWork<P, NCG, NW, true, SPLIT> W(a);
+    if (W.empty())
+        return;
     __shared__ Lds<HD, KT, 2, true> S;
     WaveAttn<HD, KT, NCG> A;
-    const int nblk = (W.wg_len + kTB - 1) / kTB;
+    const int nblk = (W.wg_len - W.t0 + kTB - 1) / kTB;
     const bool gb = W.w >= NW / 2;
     const int st = W.tid & 255;
 
     // prologue: both planes of block 0 staged (B: K, A: V), and each group's
     // plane of block 1 loaded; block 0's loads are in flight while Q is
     // loaded and split
-    const int tb0 = W.table(0), tb1 = W.table(kTB);
+    const int tb0 = W.table(W.t0), tb1 = W.table(W.t0 + kTB);
     PlaneRegs<HD, KT> R;
     PlaneScales<HD, KT> C;
     if (gb) {
@@ -2075,8 +2151,8 @@ __global__ __launch_bounds__(512) void attn_prefill_ppq(PrefillArgs a)
         plane_scales<1, HD, KT, P>(a, W.kvh, st, R, C);
     }
     A.template init<true>(a, W.b, W.kvh, W.col0, W.start, W.mapped, W.wave_active, W.j, W.g);
-    const uint64_t mask_c = W.valid_mask(a, tb0, 0);
-    const uint64_t mask_n = W.valid_mask(a, tb1, kTB);
+    const uint64_t mask_c = W.valid_mask(a, tb0, W.t0);
+    const uint64_t mask_n = W.valid_mask(a, tb1, W.t0 + kTB);
     if (gb) {
         plane_store<0, HD, KT, P, 2>(a, W.kvh, st, 0, 0, R, C, S);
         plane_load<0, HD, KT, P>(a, W.kvh, st, tb1, R);
@@ -2084,15 +2160,15 @@ __global__ __launch_bounds__(512) void attn_prefill_ppq(PrefillArgs a)
         plane_store<1, HD, KT, P, 2>(a, W.kvh, st, 0, mask_c, R, C, S);
         plane_load<1, HD, KT, P>(a, W.kvh, st, tb1, R);
     }
-    const int tb2 = W.table(2 * kTB);
+    const int tb2 = W.table(W.t0 + 2 * kTB);
     __syncthreads();
-    PingPongQ<HD, KT, P, NCG> pp{a, W, S, A};
+    PingPongQ<HD, KT, P, NCG, SPLIT> pp{a, W, S, A};
     if (gb)
         pp.template run<true>(R, tb2, mask_c, mask_n, nblk);
     else
         pp.template run<false>(R, tb2, mask_c, mask_n, nblk);
     if (W.wave_active)
-        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g);
+        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g, W.part);
 }
 
 // f32 pages (head_dim 128): one plane of a 64-token block staged by the four
@@ -2252,11 +2328,11 @@ __device__ __forceinline__ void plane_store_f32(int ws, int lane, uint64_t vmask
 //            B: convert K (n + 1), softmax (n)
 //   phase 2: A: convert V (n + 1), softmax (n)
 //            B: P V (n) with the loads of K (n + 2), scores (n + 1)
-template <int HD, int P, int NCG>
+template <int HD, int P, int NCG, bool SPLIT>
 struct PingPongF {
     static constexpr int NW = 8;
     const PrefillArgs &a;
-    const PrefillWork<P, NCG, NW, true> &W;
+    const PrefillWork<P, NCG, NW, true, SPLIT> &W;
     Lds<HD, KV_F32, 2> &S;
     float (&sc)[2][2][4]; // [plane][buffer][staging wave]
     WaveAttn<HD, KV_F32, NCG> &A;
@@ -2301,12 +2377,12 @@ struct PingPongF {
     {
         const int ws = W.w & 3;
         f4 s[NCG][2][2]; // a block's scores, then its P (softmax_block)
-        if (GB && live(0))
+        if (GB && live(W.t0))
             scores(0, s);
         int n = 0;
         auto step = [&](auto full) {
             constexpr bool FULL = decltype(full)::value;
-            const int base = n * kTB, cur = n & 1;
+            const int base = W.t0 + n * kTB, cur = n & 1;
             int tb2; // page ids of block n + 2
             // phase 1
             if (!GB) {
@@ -2343,32 +2419,34 @@ struct PingPongF {
             mask_n = mask_nn;
             n++;
         };
-        while (n < nblk && W.block_full(n * kTB, mask_c))
+        while (n < nblk && W.block_full(W.t0 + n * kTB, mask_c))
             step(std::true_type{});
         while (n < nblk)
             step(std::false_type{});
-        if (!GB && nblk > 0 && live((nblk - 1) * kTB))
+        if (!GB && nblk > 0 && live(W.t0 + (nblk - 1) * kTB))
             pv((nblk - 1) & 1, s);
     }
 };
 
-template <int HD, int P, int NCG>
+template <int HD, int P, int NCG, bool SPLIT>
 __global__ __launch_bounds__(512) void attn_prefill_ppf(PrefillArgs a)
 {
     static_assert(HD == 128, "f32 ping-pong staging maps head_dim 128");
-    constexpr int NW = PingPongF<HD, P, NCG>::NW;
-    const PrefillWork<P, NCG, NW, true> W(a);
+    constexpr int NW = PingPongF<HD, P, NCG, SPLIT>::NW;
+    const PrefillWork<P, NCG, NW, true, SPLIT> W(a);
+    if (W.empty())
+        return;
     __shared__ Lds<HD, KV_F32, 2> S;
     __shared__ __attribute__((aligned(16))) float sc[2][2][4];
     WaveAttn<HD, KV_F32, NCG> A;
-    const int nblk = (W.wg_len + kTB - 1) / kTB;
+    const int nblk = (W.wg_len - W.t0 + kTB - 1) / kTB;
     const bool gb = W.w >= NW / 2;
     const int ws = W.w & 3;
 
     // prologue: both planes of block 0 staged (B: K, A: V), and B's plane of
     // block 1 loaded; block 0's loads are in flight while Q is loaded and
     // split
-    const int tb0 = W.table(0), tb1 = W.table(kTB), tb2 = W.table(2 * kTB);
+    const int tb0 = W.table(W.t0), tb1 = W.table(W.t0 + kTB), tb2 = W.table(W.t0 + 2 * kTB);
     PlaneF32 R;
     float run = 0.0f;
     if (gb)
@@ -2376,8 +2454,8 @@ __global__ __launch_bounds__(512) void attn_prefill_ppf(PrefillArgs a)
     else
         plane_load_f32<1, P>(a, W.kvh, ws, W.lane, tb0, R);
     A.template init<true>(a, W.b, W.kvh, W.col0, W.start, W.mapped, W.wave_active, W.j, W.g);
-    const uint64_t mask_c = W.valid_mask(a, tb0, 0);
-    const uint64_t mask_n = W.valid_mask(a, tb1, kTB);
+    const uint64_t mask_c = W.valid_mask(a, tb0, W.t0);
+    const uint64_t mask_n = W.valid_mask(a, tb1, W.t0 + kTB);
     if (gb) {
         plane_store_f32<0, 2>(ws, W.lane, mask_c, R, run, sc[0][0], A.neg1, S, 0);
         plane_load_f32<0, P>(a, W.kvh, ws, W.lane, tb1, R);
@@ -2385,15 +2463,54 @@ __global__ __launch_bounds__(512) void attn_prefill_ppf(PrefillArgs a)
         plane_store_f32<1, 2>(ws, W.lane, mask_c, R, run, sc[1][0], A.neg1, S, 0);
     }
     __syncthreads();
-    PingPongF<HD, P, NCG> pp{a, W, S, sc, A};
+    PingPongF<HD, P, NCG, SPLIT> pp{a, W, S, sc, A};
     if (gb)
         pp.template run<true>(R, run, tb2, mask_c, mask_n, nblk);
     else
         pp.template run<false>(R, run, tb1, mask_c, mask_n, nblk);
     if (W.wave_active) {
         A.v_units_out();
-        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g);
+        A.finish(a, W.b, W.kvh, W.col0, W.j, W.g, W.part);
     }
+}
+
+// Merges the splits of a prefill: thread (row, 4 dimensions).  A row's splits
+// are those that start before its end; a sequence that one split covers has
+// its output already.  Bound by the partials it reads once (12 MB of a
+// 512-token chunk of 32 heads of 128 per split).
+template <int HD>
+__global__ __launch_bounds__(256) void merge_prefill(PrefillArgs a)
+{
+    constexpr int TPR = HD / 4;
+    const int H = a.num_heads, chunk = a.chunk_len;
+    const int64_t rows = (int64_t)a.batch * chunk * H;
+    const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+    if (row >= rows)
+        return;
+    const int d = 4 * (threadIdx.x % TPR);
+    const int64_t tok = row / H;
+    const int b = (int)(tok / chunk), qi = (int)(tok - (int64_t)b * chunk);
+    const int mapped = a.max_blocks * a.L.page_tokens, start = a.start_pos[b];
+    const int len = min(start + chunk, mapped), per = split_len(a.L, len, a.num_splits);
+    if (per >= len)
+        return;
+    const int n = (min(start + qi + 1, mapped) + per - 1) / per;
+    const float2 *ml = reinterpret_cast<const float2 *>(a.ws) + row;
+    const float *ow = a.ws + 2 * a.num_splits * rows + row * HD + d;
+    float M = -INFINITY;
+    for (int s = 0; s < n; s++)
+        M = fmaxf(M, ml[s * rows].x);
+    f4 num = {};
+    float den = 0.0f;
+    if (M != -INFINITY)
+        for (int s = 0; s < n; s++) {
+            const float2 t = ml[s * rows];
+            const float f = exp2f(t.x - M);
+            num += *reinterpret_cast<const f4 *>(ow + s * rows * HD) * f;
+            den = fmaf(t.y, f, den);
+        }
+    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+    *reinterpret_cast<f4 *>(a.out + row * HD + d) = num * inv;
 }
 
 } // namespace mfma_prefill
@@ -2463,62 +2580,110 @@ static void launch_lds(const PrefillArgs &a, hipStream_t st)
         const int64_t per_wg = nw * 16 * ncg;
         return dim3((unsigned)((cols + per_wg - 1) / per_wg), a.L.num_kv_heads, a.batch);
     };
+    // one launch of KERNEL<..., SPLIT>, its grid widened by the splits
+#define GI_PGRID(ncg, nw) dim3(grid(ncg, nw).x * a.num_splits, a.L.num_kv_heads, a.batch)
+#define GI_PP(KERNEL, ...)                                                                                \
+    do {                                                                                                  \
+        if (a.num_splits > 1)                                                                             \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, true>), GI_PGRID(1, 8), dim3(512), 0, st, a);      \
+        else if (NCG == 1 || a.narrow)                                                                    \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, false>), GI_PGRID(1, 8), dim3(512), 0, st, a);     \
+        else                                                                                              \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, NCG, false>), GI_PGRID(NCG, 8), dim3(512), 0, st, a); \
+    } while (0)
+    const int P = a.L.page_tokens;
     if constexpr (KT == KV_F16) {
         constexpr int NCG = kPrefillPingPongNcg;
-        switch (a.L.page_tokens) {
-        case 16:
-            hipLaunchKernelGGL((attn_prefill_pp<HD, 16, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        case 32:
-            hipLaunchKernelGGL((attn_prefill_pp<HD, 32, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        default:
-            hipLaunchKernelGGL((attn_prefill_pp<HD, 64, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
+        switch (P) {
+        case 16: GI_PP(attn_prefill_pp, HD, 16); break;
+        case 32: GI_PP(attn_prefill_pp, HD, 32); break;
+        default: GI_PP(attn_prefill_pp, HD, 64); break;
         }
     } else if constexpr (KT == KV_F32 && HD == 128) {
         constexpr int NCG = kPrefillF32Ncg;
-        switch (a.L.page_tokens) {
-        case 16:
-            hipLaunchKernelGGL((attn_prefill_ppf<HD, 16, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        case 32:
-            hipLaunchKernelGGL((attn_prefill_ppf<HD, 32, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        default:
-            hipLaunchKernelGGL((attn_prefill_ppf<HD, 64, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
+        switch (P) {
+        case 16: GI_PP(attn_prefill_ppf, HD, 16); break;
+        case 32: GI_PP(attn_prefill_ppf, HD, 32); break;
+        default: GI_PP(attn_prefill_ppf, HD, 64); break;
         }
     } else if constexpr ((KT == KV_Q8_0 || KT == KV_Q4_0) && HD == 128) {
         constexpr int NCG = kPrefillPingPongNcg;
-        switch (a.L.page_tokens) {
-        case 16:
-            hipLaunchKernelGGL((attn_prefill_ppq<HD, KT, 16, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        case 32:
-            hipLaunchKernelGGL((attn_prefill_ppq<HD, KT, 32, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
-        default:
-            hipLaunchKernelGGL((attn_prefill_ppq<HD, KT, 64, NCG>), grid(NCG, 8), dim3(512), 0, st, a);
-            break;
+        switch (P) {
+        case 16: GI_PP(attn_prefill_ppq, HD, KT, 16); break;
+        case 32: GI_PP(attn_prefill_ppq, HD, KT, 32); break;
+        default: GI_PP(attn_prefill_ppq, HD, KT, 64); break;
         }
     } else {
-#define GI_PFL(PT)                                                                           \
-    hipLaunchKernelGGL((attn_prefill_lds<HD, KT, PT, NBUF, prefill_lds_ncg<HD, KT, PT>(), NW>), \
-                       grid(prefill_lds_ncg<HD, KT, PT>(), NW), dim3(64 * NW), 0, st, a)
-    switch (a.L.page_tokens) {
-    case 16:
-        GI_PFL(16);
-        break;
-    case 32:
-        GI_PFL(32);
-        break;
-    default:
-        GI_PFL(64);
-        break;
-    }
+#define GI_PFL(PT)                                                                                         \
+    do {                                                                                                   \
+        constexpr int NCG = prefill_lds_ncg<HD, KT, PT>();                                                 \
+        if (a.num_splits > 1)                                                                              \
+            hipLaunchKernelGGL((attn_prefill_lds<HD, KT, PT, NBUF, NCG, NW, true>), GI_PGRID(NCG, NW),     \
+                               dim3(64 * NW), 0, st, a);                                                   \
+        else                                                                                               \
+            hipLaunchKernelGGL((attn_prefill_lds<HD, KT, PT, NBUF, NCG, NW, false>), GI_PGRID(NCG, NW),    \
+                               dim3(64 * NW), 0, st, a);                                                   \
+    } while (0)
+        switch (P) {
+        case 16: GI_PFL(16); break;
+        case 32: GI_PFL(32); break;
+        default: GI_PFL(64); break;
+        }
 #undef GI_PFL
     }
+#undef GI_PP
+#undef GI_PGRID
+    if (a.num_splits > 1) {
+        const int64_t rows = (int64_t)a.batch * a.chunk_len * a.num_heads;
+        constexpr int RPW = 256 / (HD / 4);
+        hipLaunchKernelGGL(merge_prefill<HD>, dim3((unsigned)((rows + RPW - 1) / RPW)), dim3(256), 0, st, a);
+    }
+}
+
+// The shape of a prefill launch.  A workgroup of 256 columns (query, head)
+// has the fewest LDS reads per product, but a single user's chunk of 512
+// queries is then 64 workgroups on 256 CUs: so 128 columns where that still
+// leaves no more than about one workgroup per CU (Llama-3-8B shape, 512
+// queries behind 2000 tokens: fp16 112 -> 76 us, q8_0 160 -> 107; at 4 x 512,
+// 256 against 512 workgroups, 145 -> 163), and the context cut until the
+// workgroups of 128 fill the CUs, merged by a second launch (the same: fp16
+// 59, q8_0 77, f32 120 -> 85; 128 queries behind 6000 tokens 157 -> 47).
+//  - One workgroup per CU, rounded down: a few more than the CUs hold took a
+//    second round (128 queries behind 2000: 8 splits 31.9, 9 41.9).
+//  - q8_0 pages at head dimension 64 run four-wave workgroups, two per CU
+//    (512 behind 2000: 2 splits 63, 4 55).
+//  - 1/2 to 2/3 of the CUs: three splits leave less idle than one (2 x 300
+//    queries behind 2000: q8_0 102 -> 97, f32 116 -> 112, head dimension 64
+//    fp16 51 -> 45, f32 115 -> 90), but not for fp16 at 128 (74 -> 76).
+// The kernels cut each sequence's own context (split_len); the mapped length
+// only bounds the number of pieces.
+void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
+                  int num_cus, int *num_splits, bool *narrow)
+{
+    *num_splits = 1;
+    *narrow = false;
+    const int P = L.page_tokens;
+    if (requested == 0 || batch <= 0 || chunk_len <= 0 || !mfma_prefill_supported(L, num_heads) ||
+        !(P == 16 || P == 32 || P == 64))
+        return;
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    const int64_t cols = (int64_t)chunk_len * (num_heads / L.num_kv_heads);
+    const int64_t wgs = (cols + 127) / 128 * L.num_kv_heads * batch; // of 128 columns
+    const int64_t two = (cols + 255) / 256 * L.num_kv_heads * batch; // of 256 columns
+    *narrow = 16 * two <= 9 * cus;
+    int64_t s = (L.kv_type == KV_Q8_0 && L.head_dim == 64 ? 2 * cus : cus) / wgs;
+    if (s == 1 && 2 * wgs > cus && 3 * wgs <= 2 * cus && !(L.kv_type == KV_F16 && L.head_dim == 128))
+        s = 3;
+    s = std::min(s, mapped / mfma_prefill::kMinSplit);
+    if (mapped > mfma_prefill::whole_len(L) && s > 1)
+        *num_splits = (int)s;
+}
+
+size_t prefill_workspace_bytes(const PrefillArgs &a)
+{
+    if (a.num_splits <= 1)
+        return 0;
+    return (size_t)a.num_splits * a.batch * a.chunk_len * a.num_heads * (a.L.head_dim + 2) * sizeof(float);
 }
 
 hipError_t launch_prefill_mfma(const PrefillArgs &a, hipStream_t st)
