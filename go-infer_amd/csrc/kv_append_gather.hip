@@ -356,7 +356,187 @@ __global__ __launch_bounds__(kThreads) void append_rows(PoolLayout L, uint8_t *b
     }
 }
 
-// Gather one sequence's tokens [0, n_tok) of one layer.
+// Gather of pages of whole 16-token groups at head dimension 64 or 128.  A
+// workgroup takes kGatherTok tokens of one kv head, K and V.  Bytes bound it
+// (each read and written once), so every load and store is 16 bytes of one
+// run: f32 and f16 K rows go straight through; V, and the codes and scales
+// of quantised pages, are put together in LDS as the token rows the host's
+// layout has (ROW bytes: f32 and f16 elements, 34- or 18-byte blocks), which
+// leave as 16-byte (quantised rows: 4-byte) stores or widened to float4.  V
+// pages are dimension-major: read element by element in output order, as
+// gather_kernel does, a wave touched 64 sectors per 128 bytes.  Bytes are
+// gather_kernel's.  Llama-3-8B shape, us a call, gather_kernel / here: 6001
+// tokens fp16 23.75 / 8.94, q8_0 29.2 / 8.4, q4_0 15.4 / 7.2; 16000 tokens fp16
+// 58.4 / 20.8, widened 64.1 / 33.7.
+constexpr int kGatherTok = 32;
+
+template <int KT, int HD, bool WIDEN>
+__global__ __launch_bounds__(kThreads) void gather_tiles(PoolLayout L, const uint8_t *base,
+                                                         const int32_t *__restrict__ table, int n_tok,
+                                                         uint8_t *kout, uint8_t *vout, int *status)
+{
+    constexpr bool QUANT = KT == KV_Q8_0 || KT == KV_Q4_0;
+    constexpr int NB = HD / 32;
+    constexpr int ROW = KT == KV_F32 ? 4 * HD : KT == KV_F16 ? 2 * HD : KT == KV_Q8_0 ? 34 * NB : 18 * NB;
+    // row stride in LDS: 16-byte aligned rows that start 4 (f32, f16) banks
+    // apart, quantised rows packed
+    constexpr int LROW = QUANT ? ROW : ROW + 16;
+    constexpr int T = kGatherTok;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    __shared__ __align__(16) uint8_t s_v[T * LROW];
+    __shared__ __align__(16) uint8_t s_k[QUANT ? T * LROW : 16];
+    __shared__ int64_t s_page[T / 16]; // page offset of each 16-token group, -1: none
+    const int t0 = blockIdx.x * T, kvh = blockIdx.y, tid = threadIdx.x;
+    const int P = L.page_tokens;
+    if (tid < T / 16) {
+        const int t = t0 + 16 * tid;
+        int64_t off = -1;
+        if (t < n_tok) {
+            const int64_t page = table[t / P];
+            if (page >= 0 && page < L.num_pages)
+                off = page * L.page_bytes;
+            else if (kvh == 0)
+                raise_flag(status, FLAG_BAD_PAGE);
+        }
+        s_page[tid] = off;
+    }
+    __syncthreads();
+    const int64_t row_out = (int64_t)L.num_kv_heads * (WIDEN ? 4 * HD : ROW); // bytes of a token vector
+    const int64_t head_out = (int64_t)kvh * (WIDEN ? 4 * HD : ROW);
+
+    // ---- K rows and V units of 16 bytes ----
+    if constexpr (!QUANT) {
+        constexpr int E = KT == KV_F32 ? 4 : 2, U = ROW / 16; // 16-byte units of a K row
+        for (int u = tid; u < T * U; u += kThreads) {
+            const int r = u / U, c = u - r * U, t = t0 + r;
+            const int64_t off = s_page[r >> 4];
+            if (t >= n_tok || off < 0)
+                continue;
+            const u4 x = *reinterpret_cast<const u4 *>(base + off + L.k_off + ((int64_t)kvh * P + t % P) * ROW + 16 * c);
+            uint8_t *o = kout + t * row_out + head_out;
+            if constexpr (WIDEN && KT == KV_F16) {
+                float4 *w = reinterpret_cast<float4 *>(o + 32 * c);
+                w[0] = float4{half_bits_to_float(x[0] & 0xFFFFu), half_bits_to_float(x[0] >> 16),
+                              half_bits_to_float(x[1] & 0xFFFFu), half_bits_to_float(x[1] >> 16)};
+                w[1] = float4{half_bits_to_float(x[2] & 0xFFFFu), half_bits_to_float(x[2] >> 16),
+                              half_bits_to_float(x[3] & 0xFFFFu), half_bits_to_float(x[3] >> 16)};
+            } else {
+                *reinterpret_cast<u4 *>(o + 16 * c) = x;
+            }
+        }
+        // V unit: TU tokens of one dimension
+        constexpr int TU = 16 / E, UG = 16 / TU; // units per dimension and 16-token group
+        for (int u = tid; u < T / TU * HD; u += kThreads) {
+            const int grp = u / (UG * HD), d = u % (UG * HD) / UG, q = u % UG;
+            const int r = 16 * grp + TU * q;
+            const int64_t off = s_page[grp];
+            if (off < 0)
+                continue;
+            const u4 x = *reinterpret_cast<const u4 *>(base + off + L.v_off +
+                                                       (((int64_t)kvh * HD + d) * P + (t0 + r) % P) * E);
+#pragma unroll
+            for (int i = 0; i < TU; i++) {
+                if constexpr (E == 4)
+                    *reinterpret_cast<uint32_t *>(&s_v[(r + i) * LROW + 4 * d]) = x[i];
+                else
+                    *reinterpret_cast<uint16_t *>(&s_v[(r + i) * LROW + 2 * d]) = (uint16_t)(x[i / 2] >> (16 * (i & 1)));
+            }
+        }
+    } else {
+        constexpr int CB = KT == KV_Q8_0 ? 32 : 16, BB = CB + 2; // code bytes and bytes of a block
+        constexpr int KU = NB * CB / 16;                         // 16-byte units of a K code row
+        auto put = [&](uint8_t *row, int at, u4 x) { // 16 code bytes at an even offset
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                *reinterpret_cast<uint16_t *>(row + at + 2 * i) = (uint16_t)(x[i / 2] >> (16 * (i & 1)));
+        };
+        for (int u = tid; u < T * KU; u += kThreads) {
+            const int r = u / KU, c = u - r * KU;
+            const int64_t off = s_page[r >> 4];
+            if (off < 0)
+                continue;
+            const u4 x = *reinterpret_cast<const u4 *>(base + off + L.k_off +
+                                                       (((int64_t)kvh * P + (t0 + r) % P) * KU + c) * 16);
+            const int b = c * 16 / CB;
+            put(&s_k[r * LROW], b * BB + 2 + c * 16 % CB, x);
+        }
+        // V unit: 16 tokens of one code row
+        for (int u = tid; u < T / 16 * NB * CB; u += kThreads) {
+            const int grp = u / (NB * CB), cr = u % (NB * CB);
+            const int64_t off = s_page[grp];
+            if (off < 0)
+                continue;
+            const u4 x = *reinterpret_cast<const u4 *>(base + off + L.v_off + ((int64_t)kvh * NB * CB + cr) * P +
+                                                       (t0 + 16 * grp) % P);
+            const int at = cr / CB * BB + 2 + cr % CB;
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                s_v[(16 * grp + i) * LROW + at] = (uint8_t)(x[i / 4] >> (8 * (i & 3)));
+        }
+        for (int u = tid; u < T * NB; u += kThreads) {
+            const int r = u / NB, b = u - r * NB, s = (t0 + r) % P;
+            const int64_t off = s_page[r >> 4];
+            if (off < 0)
+                continue;
+            *reinterpret_cast<uint16_t *>(&s_k[r * LROW + b * BB]) =
+                reinterpret_cast<const uint16_t *>(base + off + L.ks_off)[((int64_t)kvh * P + s) * NB + b];
+            *reinterpret_cast<uint16_t *>(&s_v[r * LROW + b * BB]) =
+                reinterpret_cast<const uint16_t *>(base + off + L.vs_off)[((int64_t)kvh * NB + b) * P + s];
+        }
+    }
+    __syncthreads();
+
+    // ---- LDS rows to the output ----
+    auto emit = [&](const uint8_t *rows, uint8_t *out) {
+        if constexpr (!WIDEN || KT == KV_F32) {
+            constexpr int OU = QUANT ? 4 : 16, U = ROW / OU;
+            for (int u = tid; u < T * U; u += kThreads) {
+                const int r = u / U, c = u - r * U, t = t0 + r;
+                if (t >= n_tok || s_page[r >> 4] < 0)
+                    continue;
+                uint8_t *o = out + t * row_out + head_out + OU * c;
+                if constexpr (QUANT)
+                    *reinterpret_cast<uint32_t *>(o) = *reinterpret_cast<const uint32_t *>(rows + r * LROW + 4 * c);
+                else
+                    *reinterpret_cast<u4 *>(o) = *reinterpret_cast<const u4 *>(rows + r * LROW + 16 * c);
+            }
+        } else {
+            constexpr int U = HD / 4;
+            for (int u = tid; u < T * U; u += kThreads) {
+                const int r = u / U, d = 4 * (u - r * U), t = t0 + r;
+                if (t >= n_tok || s_page[r >> 4] < 0)
+                    continue;
+                const uint8_t *row = rows + r * LROW;
+                float f[4];
+                if constexpr (KT == KV_F16) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        f[i] = half_bits_to_float(*reinterpret_cast<const uint16_t *>(row + 2 * (d + i)));
+                } else if constexpr (KT == KV_Q8_0) {
+                    const uint8_t *blk = row + d / 32 * 34;
+                    const float sc = half_bits_to_float(*reinterpret_cast<const uint16_t *>(blk));
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        f[i] = (float)(int8_t)blk[2 + d % 32 + i] * sc;
+                } else {
+                    const uint8_t *blk = row + d / 32 * 18;
+                    const float sc = half_bits_to_float(*reinterpret_cast<const uint16_t *>(blk));
+                    const int sh = d & 16 ? 4 : 0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        f[i] = (float)(((blk[2 + (d & 15) + i] >> sh) & 15) - 8) * sc;
+                }
+                *reinterpret_cast<float4 *>(out + t * row_out + head_out + 4 * d) = float4{f[0], f[1], f[2], f[3]};
+            }
+        }
+    };
+    if constexpr (QUANT)
+        emit(s_k, kout);
+    emit(s_v, vout);
+}
+
+// Gather one sequence's tokens [0, n_tok) of one layer, element by element:
+// the page sizes and output alignments gather_tiles does not take.
 //   widen == 0: stored format, the reference's bytes per token vector
 //               (f32: 4*kv_dim, f16: 2*kv_dim, q8_0: kv_dim/32 blocks of
 //               34 bytes = LE fp16 scale + 32 int8, quant.go:38-41).
@@ -718,6 +898,37 @@ hipError_t launch_gather(const PoolLayout &L, const uint8_t *base, const int32_t
                                                          : kv_dim;
     dim3 grid(grid_for((int64_t)n_tok * per_tok)), block(kThreads);
     uint8_t *ko = (uint8_t *)k_out, *vo = (uint8_t *)v_out;
+    // gather_tiles' 16-byte accesses: pages of whole 16-token groups, output
+    // rows on 16-byte (stored quantised blocks: 4-byte) boundaries
+    const uintptr_t mask = ((L.kv_type == KV_Q8_0 || L.kv_type == KV_Q4_0) && !widen) ? 3 : 15;
+    if (L.page_tokens % 16 == 0 && (L.head_dim == 64 || L.head_dim == 128) &&
+        (((uintptr_t)k_out | (uintptr_t)v_out) & mask) == 0 && L.num_kv_heads <= 65535) {
+        const dim3 tg((unsigned)((n_tok + kGatherTok - 1) / kGatherTok), (unsigned)L.num_kv_heads);
+#define GI_TILES(KT, W)                                                                                            \
+    do {                                                                                                           \
+        if (L.head_dim == 128)                                                                                     \
+            hipLaunchKernelGGL((gather_tiles<KT, 128, W>), tg, block, 0, st, L, base, table, n_tok, ko, vo, status); \
+        else                                                                                                       \
+            hipLaunchKernelGGL((gather_tiles<KT, 64, W>), tg, block, 0, st, L, base, table, n_tok, ko, vo, status); \
+        return hipGetLastError();                                                                                  \
+    } while (0)
+        switch (L.kv_type) {
+        case KV_F32: GI_TILES(KV_F32, false);
+        case KV_F16:
+            if (widen)
+                GI_TILES(KV_F16, true);
+            GI_TILES(KV_F16, false);
+        case KV_Q4_0:
+            if (widen)
+                GI_TILES(KV_Q4_0, true);
+            GI_TILES(KV_Q4_0, false);
+        default:
+            if (widen)
+                GI_TILES(KV_Q8_0, true);
+            GI_TILES(KV_Q8_0, false);
+        }
+#undef GI_TILES
+    }
 #define GI_GATHER(KT, W) \
     hipLaunchKernelGGL((gather_kernel<KT, W>), grid, block, 0, st, L, base, table, n_tok, ko, vo, status)
     if (L.kv_type == KV_F32) {

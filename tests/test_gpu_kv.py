@@ -208,3 +208,37 @@ def test_bad_page_ids_are_reported(gi, dev):
     with pytest.raises(gi.GIError) as ei:
         pool.Write(3, ids, slots, k, k)                              # bad layer, host check
     assert ei.value.code == -3
+
+
+@pytest.mark.parametrize("kv_type", [0, 1, 2, 3], ids=["f32", "f16", "q8_0", "q4_0"])
+@pytest.mark.parametrize("kvh,hd,P", [(8, 128, 16), (3, 64, 16), (2, 128, 32), (4, 64, 48), (1, 128, 64), (2, 64, 8)])
+def test_gather_tile_edges(gi, oracle, dev, kv_type, kvh, hd, P):
+    """Token counts around the gather's 16-token groups and 32-token tiles,
+    pages that tiles straddle (48) and that only the element-wise kernel
+    takes (8), special values among them; nothing past the last token is
+    written, and an output that is not 16-byte aligned holds the same bytes."""
+    import torch
+    kv_dim = kvh * hd
+    pop = Populated(gi, dev, kv_type, 1, kvh, hd, P, [130], seed=17, specials=True)
+    ks, vs = pop.stored(0, 0)
+    t = torch.from_numpy(pop.table(0)).to(dev)
+    for n in (1, 15, 16, 17, 31, 33, 64, 97, 130):
+        ko, vo = pop.pool.Get(0, t, n)
+        assert np.array_equal(ko.cpu().numpy(), ks[:n]), n
+        assert np.array_equal(vo.cpu().numpy(), vs[:n]), n
+        kw, vw = pop.pool.Get(0, t, n, widen=True)
+        for got, st in ((kw, ks), (vw, vs)):
+            want = oracle.widen(kv_type, kv_dim, st[:n])
+            assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32)), n
+    n, rb = 50, ks.shape[1]
+    for widen, bytes_per, shift in ((0, rb, 4), (0, rb, 2), (1, 4 * kv_dim, 4)):
+        if shift == 2 and kv_type == 0:
+            continue  # float elements need 4
+        buf = torch.full((2, n * bytes_per + 64), 0xA5, dtype=torch.uint8, device=dev)
+        gi._check(gi.lib().gi_paged_gather(pop.pool._h, 0, t.data_ptr(), n, buf[0].data_ptr() + shift,
+                                           buf[1].data_ptr() + shift, widen))
+        pop.pool.synchronize()
+        for row, st in zip(buf.cpu().numpy(), (ks, vs)):
+            want = st[:n] if not widen else oracle.widen(kv_type, kv_dim, st[:n]).view(np.uint8)
+            assert np.array_equal(row[shift:shift + n * bytes_per].reshape(n, -1), want.reshape(n, -1)), (widen, shift)
+            assert (row[:shift] == 0xA5).all() and (row[shift + n * bytes_per:] == 0xA5).all()
