@@ -2584,7 +2584,10 @@ static void launch_lds(const PrefillArgs &a, hipStream_t st)
 #define GI_PGRID(ncg, nw) dim3(grid(ncg, nw).x * a.num_splits, a.L.num_kv_heads, a.batch)
 #define GI_PP(KERNEL, ...)                                                                                \
     do {                                                                                                  \
-        if (a.num_splits > 1)                                                                             \
+        constexpr int WIDE = HD == 128 ? NCG : 1; /* columns of a wide split, see prefill_plan */         \
+        if (a.num_splits > 1 && !a.narrow)                                                                \
+            hipLaunchKernelGGL((KERNEL<__VA_ARGS__, WIDE, true>), GI_PGRID(WIDE, 8), dim3(512), 0, st, a); \
+        else if (a.num_splits > 1)                                                                        \
             hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, true>), GI_PGRID(1, 8), dim3(512), 0, st, a);      \
         else if (NCG == 1 || a.narrow)                                                                    \
             hipLaunchKernelGGL((KERNEL<__VA_ARGS__, 1, false>), GI_PGRID(1, 8), dim3(512), 0, st, a);     \
@@ -2652,9 +2655,12 @@ static void launch_lds(const PrefillArgs &a, hipStream_t st)
 //    second round (128 queries behind 2000: 8 splits 31.9, 9 41.9).
 //  - q8_0 pages at head dimension 64 run four-wave workgroups, two per CU
 //    (512 behind 2000: 2 splits 63, 4 55).
-//  - 1/2 to 2/3 of the CUs: three splits leave less idle than one (2 x 300
-//    queries behind 2000: q8_0 102 -> 97, f32 116 -> 112, head dimension 64
-//    fp16 51 -> 45, f32 115 -> 90), but not for fp16 at 128 (74 -> 76).
+//  - 1/2 to 2/3 of the CUs: three splits leave less idle than one, of 256
+//    columns where a wave can take them at head dimension 128 (2 x 300 queries
+//    behind 2000, one / three narrow / three wide: fp16 74 / 76 / 65, q8_0
+//    102 / 97 / 83, q4_0 97 / 92 / 76; f32 116 / 112, head dimension 64 fp16
+//    51 / 43 / 44, f32 115 / 90).  Wide splits elsewhere win by a few per
+//    cent at contexts over 3000 and lose more below.
 // The kernels cut each sequence's own context (split_len); the mapped length
 // only bounds the number of pieces.
 void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
@@ -2672,11 +2678,16 @@ void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, 
     const int64_t two = (cols + 255) / 256 * L.num_kv_heads * batch; // of 256 columns
     *narrow = 16 * two <= 9 * cus;
     int64_t s = (L.kv_type == KV_Q8_0 && L.head_dim == 64 ? 2 * cus : cus) / wgs;
-    if (s == 1 && 2 * wgs > cus && 3 * wgs <= 2 * cus && !(L.kv_type == KV_F16 && L.head_dim == 128))
+    bool wide = false;
+    if (s == 1 && 2 * wgs > cus && 3 * wgs <= 2 * cus) {
         s = 3;
+        wide = L.head_dim == 128 && L.kv_type != KV_F32;
+    }
     s = std::min(s, mapped / mfma_prefill::kMinSplit);
-    if (mapped > mfma_prefill::whole_len(L) && s > 1)
+    if (mapped > mfma_prefill::whole_len(L) && s > 1) {
         *num_splits = (int)s;
+        *narrow = !wide;
+    }
 }
 
 size_t prefill_workspace_bytes(const PrefillArgs &a)

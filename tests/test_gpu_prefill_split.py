@@ -35,6 +35,7 @@ SHAPES = [
     (16, 4, 128, 16, [0, 700, 1300], 45), (8, 2, 128, 32, [2040], 64), (8, 2, 128, 64, [449], 64),
     (16, 4, 128, 16, [448], 65), (8, 4, 64, 16, [321, 1000], 64), (16, 2, 64, 32, [320], 64),
     (8, 8, 64, 64, [1531], 130), (4, 4, 128, 16, [5, 3001], 1), (8, 1, 128, 16, [250], 515),
+    (32, 8, 128, 16, [0, 900], 257),  # wide splits: 144 workgroups of 128 columns on 256 CUs
 ]
 
 
