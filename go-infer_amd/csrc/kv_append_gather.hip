@@ -171,29 +171,88 @@ __global__ __launch_bounds__(kThreads) void append_q4(PoolLayout L, uint8_t *bas
 // Bytes are identical to append_plain / append_q8 / append_q4 (the same
 // conversion and quantisation code).  head_dim is a multiple of 32 and at
 // most kRowMaxHd.
-constexpr int kRowTok = 16, kRowMaxHd = 256;
+// s_v rows are kRowPad words apart: 16 put the lanes of a token, 4 rows
+// each, on one bank.
+//
+// ROPE (gi_paged_rope_append of a chunk): K is turned on its way, and
+// workgroups of blockIdx.y >= num_kv_heads turn the tile's q, 4 pairs per
+// thread and step, into q_out (which may be q: a pair's two ends are read and
+// written by one thread).  Same products and sums as rope_append, which took
+// one 4-byte pair per thread and stored V element by element.
+constexpr int kRowTok = 16, kRowPad = 17, kRowMaxHd = 256;
 
-template <int KT>
+// 4 consecutive elements x of a head turned with y, the other ends of their
+// pairs; lo: x are the first ends (dimensions below rope_half).
+__device__ __forceinline__ f4 rope4(f4 x, f4 y, const float2 *cs, bool lo)
+{
+    const f4 a = *reinterpret_cast<const f4 *>(cs), b = *reinterpret_cast<const f4 *>(cs + 2);
+    const float c[4] = {a[0], a[2], b[0], b[2]}, s[4] = {a[1], a[3], b[1], b[3]};
+    f4 r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float y0, y1;
+        rope_pair(lo ? x[i] : y[i], lo ? y[i] : x[i], c[i], s[i], &y0, &y1);
+        r[i] = lo ? y0 : y1;
+    }
+    return r;
+}
+
+template <int KT, bool ROPE>
 __global__ __launch_bounds__(kThreads) void append_rows(PoolLayout L, uint8_t *base, int n_tok, Dest D,
                                                         const float *__restrict__ k, const float *__restrict__ v,
-                                                        int *status)
+                                                        int *status, RopeArgs R)
 {
     const int hd = L.head_dim, P = L.page_tokens, nb = hd / 32;
     const int kv_dim = L.num_kv_heads * hd;
     const int h = blockIdx.y, i0 = blockIdx.x * kRowTok, tid = threadIdx.x;
     const int nt = min(kRowTok, n_tok - i0);
+    const int rh = ROPE ? R.rope_half : 0;
+    if (ROPE && h >= L.num_kv_heads) {
+        // q: per head rh / 4 units of 4 pairs, then the dimensions past 2 rh
+        const int upr = rh / 4, per = upr + (hd - 2 * rh) / 4;
+        const int total = nt * R.num_heads * per, step = (gridDim.y - L.num_kv_heads) * kThreads;
+        for (int u = (h - L.num_kv_heads) * kThreads + tid; u < total; u += step) {
+            const int hq = u / per, c = u - hq * per, t = hq / R.num_heads;
+            const int pos = R.positions[i0 + t];
+            if (pos < 0 || pos >= R.max_pos)
+                continue; // reported with its K
+            const int64_t o = ((int64_t)i0 * R.num_heads + hq) * hd;
+            if (c < upr) {
+                const float2 *cs = R.table + (int64_t)pos * rh + 4 * c;
+                const f4 x = *reinterpret_cast<const f4 *>(R.q + o + 4 * c);
+                const f4 y = *reinterpret_cast<const f4 *>(R.q + o + rh + 4 * c);
+                *reinterpret_cast<f4 *>(R.q_out + o + 4 * c) = rope4(x, y, cs, true);
+                *reinterpret_cast<f4 *>(R.q_out + o + rh + 4 * c) = rope4(y, x, cs, false);
+            } else {
+                const int64_t e = o + 2 * rh + 4 * (c - upr);
+                *reinterpret_cast<f4 *>(R.q_out + e) = *reinterpret_cast<const f4 *>(R.q + e);
+            }
+        }
+        return;
+    }
     const int gpt = hd / 4; // 4-element groups per token
     const int ngroups = kRowTok * gpt;
     __shared__ int64_t s_page[kRowTok];
     __shared__ int s_slot[kRowTok];              // -1: token not stored
-    __shared__ uint32_t s_v[kRowMaxHd * kRowTok]; // V element bits (or codes, q4 bytes) [row][token]
+    __shared__ int s_pos[kRowTok];               // ROPE: its position
+    __shared__ uint32_t s_v[kRowMaxHd * kRowPad]; // V element bits (or codes, q4 bytes) [row][token]
     __shared__ uint16_t s_vs[kRowMaxHd / 32 * kRowTok]; // V block scales [block][token]
 
     if (tid < kRowTok) {
         int64_t pg = 0;
         int sl = -1;
         // the kv head 0 workgroup reports each bad token once
-        if (tid < nt && !resolve(D, L, i0 + tid, &pg, &sl, h == 0 ? status : nullptr))
+        bool take = tid < nt;
+        if (ROPE && take) {
+            const int pos = R.positions[i0 + tid];
+            s_pos[tid] = pos;
+            if (pos < 0 || pos >= R.max_pos) { // skipped whole
+                take = false;
+                if (h == 0)
+                    raise_flag(status, FLAG_BAD_POS);
+            }
+        }
+        if (take && !resolve(D, L, i0 + tid, &pg, &sl, h == 0 ? status : nullptr))
             sl = -1;
         s_page[tid] = pg;
         s_slot[tid] = sl;
@@ -211,6 +270,11 @@ __global__ __launch_bounds__(kThreads) void append_rows(PoolLayout L, uint8_t *b
             const int64_t e = (int64_t)(i0 + t) * kv_dim + (int64_t)h * hd + d0;
             kx = *reinterpret_cast<const f4 *>(k + e);
             vx = *reinterpret_cast<const f4 *>(v + e);
+            if (ROPE && d0 < 2 * rh && s_slot[t] >= 0) {
+                const bool lo = d0 < rh;
+                const f4 y = *reinterpret_cast<const f4 *>(k + e + (lo ? rh : -rh));
+                kx = rope4(kx, y, R.table + (int64_t)s_pos[t] * rh + (lo ? d0 : d0 - rh), lo);
+            }
         }
         const int sl = g < ngroups ? s_slot[t] : -1;
         uint8_t *pg = base + (g < ngroups ? s_page[t] : 0) * L.page_bytes;
@@ -294,11 +358,11 @@ __global__ __launch_bounds__(kThreads) void append_rows(PoolLayout L, uint8_t *b
                 if (a < 4) // byte rows 4a .. 4a + 3 of block blk
 #pragma unroll
                     for (int c = 0; c < 4; c++)
-                        s_v[(blk * 16 + 4 * a + c) * kRowTok + t] = vb[c];
+                        s_v[(blk * 16 + 4 * a + c) * kRowPad + t] = vb[c];
             } else {
 #pragma unroll
                 for (int c = 0; c < 4; c++)
-                    s_v[(d0 + c) * kRowTok + t] = vb[c];
+                    s_v[(d0 + c) * kRowPad + t] = vb[c];
             }
         }
     }
@@ -326,7 +390,7 @@ __global__ __launch_bounds__(kThreads) void append_rows(PoolLayout L, uint8_t *b
         uint32_t x[8];
 #pragma unroll
         for (int t = 0; t < 8; t++)
-            x[t] = scale_row ? (uint32_t)s_vs[(row - vrows) * kRowTok + t0 + t] : s_v[row * kRowTok + t0 + t];
+            x[t] = scale_row ? (uint32_t)s_vs[(row - vrows) * kRowTok + t0 + t] : s_v[row * kRowPad + t0 + t];
         if (run) {
             if (esz == 4) {
                 reinterpret_cast<u4 *>(dst0)[0] = u4{x[0], x[1], x[2], x[3]};
@@ -666,7 +730,8 @@ hipError_t append_any(const PoolLayout &L, uint8_t *base, int n_tok, const Dest 
     const bool aligned16 = ((uintptr_t)k % 16 == 0) && ((uintptr_t)v % 16 == 0);
     if (!at_len && aligned16 && L.head_dim % 32 == 0 && L.head_dim <= kRowMaxHd) {
         dim3 rgrid((unsigned)((n_tok + kRowTok - 1) / kRowTok), (unsigned)L.num_kv_heads);
-#define GI_ROWS(KT) hipLaunchKernelGGL((append_rows<KT>), rgrid, dim3(kThreads), 0, st, L, base, n_tok, D, k, v, status)
+#define GI_ROWS(KT) hipLaunchKernelGGL((append_rows<KT, false>), rgrid, dim3(kThreads), 0, st, L, base, n_tok, D, k, v, status, \
+                       RopeArgs{})
         switch (L.kv_type) {
         case KV_F32:
             GI_ROWS(KV_F32);
@@ -845,6 +910,14 @@ hipError_t launch_append_at_len(const PoolLayout &L, uint8_t *base, int batch,
     return append_any(L, base, batch, D, k, v, status, st);
 }
 
+// Elements of q (or 4 x K) from which a RoPE append goes by rows: below, the
+// rows' longer chain (destinations, LDS) costs more than its wider accesses
+// give.  us a call, rope_append / rows: Llama-3-8B shape fp16 512 tokens 8.5 /
+// 7.7, 1024 13.7 / 10.2, 2048 24.0 / 16.4, f32 2048 31.3 / 17.3, q8_0 300 9.9 /
+// 10.7; TinyLlama shape f32 300 tokens with the attention behind it 24.8 /
+// 25.4, 2048 tokens 13.7 / 8.6.
+constexpr int64_t kRopeRowsMin = 512 * 4096;
+
 hipError_t launch_rope_append(const PoolLayout &L, uint8_t *base, int n_tok, const int32_t *block_ids,
                               const int32_t *slots, const int32_t *block_tables, int max_blocks,
                               const int32_t *seq_lens, const RopeArgs &R, const float *k,
@@ -855,6 +928,26 @@ hipError_t launch_rope_append(const PoolLayout &L, uint8_t *base, int n_tok, con
     Dest D{block_ids, slots, block_tables, seq_lens, max_blocks};
     const bool at_len = block_ids == nullptr;
     const size_t lds = sizeof(float) * (size_t)L.num_kv_heads * L.head_dim;
+    // a chunk: whole rows, where 16-byte accesses and groups of 4 pairs fit
+    const uintptr_t ptrs = (uintptr_t)k | (uintptr_t)v | (uintptr_t)R.q | (uintptr_t)R.q_out | (uintptr_t)R.table;
+    const int64_t elems = (int64_t)n_tok * std::max(R.num_heads, 4 * L.num_kv_heads) * L.head_dim;
+    if (!at_len && elems >= kRopeRowsMin && ptrs % 16 == 0 && R.rope_half % 4 == 0 && L.head_dim % 32 == 0 &&
+        L.head_dim <= kRowMaxHd) {
+        const int per = R.rope_half / 4 + (L.head_dim - 2 * R.rope_half) / 4;
+        const int64_t qb = ((int64_t)kRowTok * R.num_heads * per + kThreads - 1) / kThreads;
+        const dim3 rgrid((unsigned)((n_tok + kRowTok - 1) / kRowTok),
+                         (unsigned)(L.num_kv_heads + std::min<int64_t>(qb, 1024)));
+#define GI_ROPE_ROWS(KT) \
+    hipLaunchKernelGGL((append_rows<KT, true>), rgrid, dim3(kThreads), 0, st, L, base, n_tok, D, k, v, status, R)
+        switch (L.kv_type) {
+        case KV_F32: GI_ROPE_ROWS(KV_F32); break;
+        case KV_F16: GI_ROPE_ROWS(KV_F16); break;
+        case KV_Q4_0: GI_ROPE_ROWS(KV_Q4_0); break;
+        default: GI_ROPE_ROWS(KV_Q8_0); break;
+        }
+#undef GI_ROPE_ROWS
+        return hipGetLastError();
+    }
     // q blocks: one rotated pair (or copied dim past rope_dim) per thread
     const int64_t q_units = (int64_t)R.num_heads *
                             std::max(R.rope_half, L.head_dim - 2 * R.rope_half);

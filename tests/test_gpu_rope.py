@@ -73,6 +73,45 @@ def test_rope_append_bit_exact(gi, oracle, dev, kv_type, shape):
         assert np.array_equal(vo.cpu().numpy(), want_v), i
 
 
+@pytest.mark.parametrize("kv_type", [0, 1, 2, 3], ids=["f32", "f16", "q8_0", "q4_0"])
+@pytest.mark.parametrize("H,kvh,hd,P,rd,n,heads_q", [
+    (32, 8, 128, 16, 128, 517, True), (32, 4, 64, 32, 64, 1025, True), (16, 8, 128, 16, 64, 1031, True),
+    (8, 8, 128, 24, 128, 600, False)])
+def test_rope_append_by_rows(gi, oracle, dev, kv_type, H, kvh, hd, P, rd, n, heads_q):
+    """A chunk large enough to go by rows, with a short last tile, half of a
+    head turned, pages that split a tile, q in place, and K alone: the bits
+    of ApplyRoPE and of the store.  A position past the table and one before
+    it skip their tokens whole."""
+    import torch
+    kv_dim = kvh * hd
+    pages = (n + P - 1) // P + 2
+    ids = np.random.default_rng(3).permutation(pages).astype(np.int32)
+    pool = gi.PagedKVCache(1, kvh, hd, P, pages, kv_type)
+    pool.SetRoPE(10000.0, rd, n + 5)
+    t = np.arange(n)
+    pos = t.astype(np.int32)
+    bad = [7, n - 1]
+    pos[bad[0]], pos[bad[1]] = n + 5, -1
+    bid, slot = ids[t // P].copy(), (t % P).astype(np.int32)
+    q, k, v = oracle.normal(1, (n, H * hd)), oracle.normal(2, (n, kv_dim)), oracle.normal(3, (n, kv_dim))
+    qd = torch.from_numpy(q.copy()).to(dev) if heads_q else None
+    pool.RoPEWrite(0, *(torch.from_numpy(x).to(dev) for x in (pos, bid, slot)), qd,
+                   torch.from_numpy(k).to(dev), torch.from_numpy(v).to(dev))
+    with pytest.raises(gi.GIError) as e:
+        pool.synchronize()
+    assert e.value.code == -7 and "RoPE" in str(e.value)
+    good = np.setdiff1d(t, bad)
+    if heads_q:
+        want = q.copy()
+        want[good] = oracle.rope_heads(q[good], pos[good], H, hd, rd, 10000.0)
+        assert np.array_equal(qd.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    ko, vo = pool.Get(0, torch.from_numpy(ids[:(n + P - 1) // P].copy()).to(dev), n)
+    ks = oracle.store_vectors(kv_type, oracle.rope_heads(k[good], pos[good], kvh, hd, rd, 10000.0))
+    assert np.array_equal(ko.cpu().numpy()[good], ks)
+    assert np.array_equal(vo.cpu().numpy()[good], oracle.store_vectors(kv_type, v[good]))
+    assert not ko.cpu().numpy()[bad].any() and not vo.cpu().numpy()[bad].any()
+
+
 def test_rope_in_place_and_long_positions(gi, oracle, dev):
     """q rotated in place; positions up to 131071 (theta 5e5, the Llama-3
     base); K-only call (no q)."""
