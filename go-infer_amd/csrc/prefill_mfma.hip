@@ -2476,8 +2476,8 @@ __global__ __launch_bounds__(512) void attn_prefill_ppf(PrefillArgs a)
 
 // Merges the splits of a prefill: thread (row, 4 dimensions).  A row's splits
 // are those that start before its end; a sequence that one split covers has
-// its output already.  Bound by the partials it reads once (12 MB of a
-// 512-token chunk of 32 heads of 128 per split).
+// its output already.  Bound by the partials it reads once (8.5 MB per
+// split for a 512-token chunk of 32 heads of 128).
 template <int HD>
 __global__ __launch_bounds__(256) void merge_prefill(PrefillArgs a)
 {
