@@ -93,6 +93,7 @@ struct gi_paged {
     hipStream_t stream = nullptr;
     int *d_status = nullptr;
     gi::DevBuffer plan_ws; // decode: partials of split sequences
+    gi::DevBuffer prefill_ws; // partials of split prefill contexts
     void *scratch = nullptr; // this device's address of `scratch` (allocate-nothing decode)
     struct ScratchOrder *scratch_order = nullptr; // and the ordering of its users
     int decode_kernel = -1; // -1 automatic, 0 vector ALU, 1 matrix core
@@ -312,6 +313,7 @@ void gi_paged_destroy(gi_paged *h)
     if (h->d_layer_base)
         (void)hipFree(h->d_layer_base);
     gi::devbuf_release(h->plan_ws);
+    gi::devbuf_release(h->prefill_ws);
     if (h->d_rope)
         (void)hipFree(h->d_rope);
     if (h->own_stream)
@@ -690,7 +692,19 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
                 return hip_fail(e, "decode attention: hipStreamIsCapturing");
         }
         const size_t want = grows && cs == hipStreamCaptureStatusNone && coarse > need ? coarse : need;
-        const int rc = gi::devbuf_reserve(h->plan_ws, want, h->stream, "decode attention");
+        int rc = gi::devbuf_reserve(h->plan_ws, want, h->stream, "decode attention");
+        if (rc == GI_ERR_OOM && want > coarse) { // a full device: the plan with fewer partials
+            (void)hipGetLastError();
+            gi::clear_error();
+            a.split_tokens = coarse_tokens;
+            a.num_splits = coarse_splits;
+            a.waves = gi::decode_waves(h->L, batch, a.num_splits, h->num_cus);
+            rc = gi::devbuf_reserve(h->plan_ws, coarse, h->stream, "decode attention");
+        } else if (rc == GI_ERR_OOM && need == 0) { // unsplit: it was for a later capture only
+            (void)hipGetLastError();
+            gi::clear_error();
+            rc = GI_OK;
+        }
         if (rc)
             return rc;
         a.ws = (float *)h->plan_ws.ptr;
@@ -855,17 +869,23 @@ int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len,
     const size_t need = gi::prefill_workspace_bytes(p);
     if (need) {
         // a capturing stream cannot allocate: the context stays in one piece
+        // where no earlier call has made room
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hipError_t e = need > h->plan_ws.bytes ? hipStreamIsCapturing(h->stream, &cs) : hipSuccess;
+        hipError_t e = need > h->prefill_ws.bytes ? hipStreamIsCapturing(h->stream, &cs) : hipSuccess;
         if (e != hipSuccess)
             return hip_fail(e, "gi_paged_prefill_attention: hipStreamIsCapturing");
         if (cs != hipStreamCaptureStatusNone) {
             p.num_splits = 1;
         } else {
-            rc = gi::devbuf_reserve(h->plan_ws, need, h->stream, "prefill attention");
-            if (rc)
+            rc = gi::devbuf_reserve(h->prefill_ws, need, h->stream, "prefill attention");
+            if (rc == GI_ERR_OOM) { // a full device: one piece needs no memory
+                (void)hipGetLastError();
+                gi::clear_error();
+                p.num_splits = 1;
+            } else if (rc) {
                 return rc;
-            p.ws = (float *)h->plan_ws.ptr;
+            }
+            p.ws = (float *)h->prefill_ws.ptr;
         }
     }
     hipError_t e = gi::launch_prefill(p, h->stream);

@@ -354,9 +354,11 @@ int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, 
  * chunk's K/V are already appended; query i of sequence b attends tokens
  * [0, start_pos[b] + i + 1).  q, out [batch][chunk_len][num_heads][head_dim]
  * float32.  Launches that leave CUs idle cut the context, as decode does; the
- * partials take splits * batch * chunk_len * num_heads * (head_dim + 2) floats
- * of the handle's workspace (at most 34 MB on a 256-CU device).  A capturing
- * stream whose workspace is too small keeps the context in one piece. */
+ * handle keeps splits * batch * chunk_len * num_heads * (head_dim + 2) floats
+ * for the partials (at most 34 MB on a 256-CU device), grown as needed and kept
+ * as decode's; a capturing stream that would need it to grow, or a device
+ * without room, keeps the context in one piece.  Replays of captured calls
+ * that could overlap other prefill calls of the handle must be serialised. */
 int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len, int num_heads,
                                const float *q, float *out, const int32_t *block_tables,
                                int max_blocks, const int32_t *start_pos, float scale);
