@@ -501,12 +501,15 @@ void decode_plan_coarse(const PoolLayout &L, int batch, int max_len, int num_cus
 // 32768 (page 32) 14.64-14.69 against 14.93-14.97, batch 1 (TinyLlama,
 // one graph) 5,245 against 4,315 tokens/s; but batch 256 x 8192 (four
 // rounds) 42.63-42.96 against 42.09-42.42 ms, the fused launch slower by
-// more than the append launch it saves.
+// more than the append launch it saves.  Each 64 rows of a step cost every
+// wave another look for pages that rows share (share_tokens, about 1 us for
+// the first two), so steps of more than kFuseRows rows are not fused either.
+constexpr int kFuseRows = 128;
 bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num_cus)
 {
     // one round: as many workgroups as the CUs hold at once (two each)
     const int64_t wgs = (int64_t)batch * L.num_kv_heads * (num_splits > 0 ? num_splits : 1);
-    return wgs <= (int64_t)2 * (num_cus > 0 ? num_cus : 256);
+    return batch <= kFuseRows && wgs <= (int64_t)2 * (num_cus > 0 ? num_cus : 256);
 }
 
 // The matrix-core decode turns whole heads: a pair's two elements are then
@@ -517,9 +520,11 @@ bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num
 //  - one round (two workgroups per CU): batch 1 x 6001 f16 14.9 / 19.1,
 //    batch 64 x 2000 q4_0 41.0 / 45.5, q8_0 51.3 / 55.4, f16 80.1 / 80.7;
 //  - q4_0, and 16-bit or 8-bit pages at head dimension 64 (three or more
-//    workgroups per CU at once): up to six per CU.  q4_0 48 x 6500 (1152)
-//    78.6 / 83.6, 200 x 2000 (1600) 101.8 / 100.3; head dimension 64 f16
-//    200 x 2000 (800) 74.6 / 76.7;
+//    workgroups per CU at once): up to six per CU, or three above 64 rows.
+//    q4_0 48 x 1500-6500 (1152) 74.6 / 77.1, 64 x 1500-3000 (512) 53.8 /
+//    56.6, 90 x 1500-3000 (720) 67.4 / 69.0, but 128 x 1500-3000 (1024)
+//    98.3 / 96.5; head dimension 64 q4_0 128 x 300-600 (512) 18.6 / 19.0,
+//    300 x 1000-2000 (1200) 66.2 / 59.1;
 //  - f16 and f32 at head dimension 128 stream at the HBM rate from the first
 //    block, so long splits hide the separate launch: f16 64 x 5000 182.9 /
 //    180.6, 64 x 12000 422 / 414, f32 64 x 2000 159.8 / 154.2, 64 x 700
@@ -527,14 +532,14 @@ bool decode_fuses_append(const PoolLayout &L, int batch, int num_splits, int num
 bool decode_fuses_rope(const PoolLayout &L, int batch, int num_heads, int requested, int rope_half,
                        int split_tokens, int num_splits, int num_cus)
 {
-    if (rope_half != L.head_dim / 2 || decode_kernel_kind(L, num_heads, requested) != 1)
+    if (batch > kFuseRows || rope_half != L.head_dim / 2 || decode_kernel_kind(L, num_heads, requested) != 1)
         return false;
     const int64_t cus = num_cus > 0 ? num_cus : 256;
     const int64_t wgs = (int64_t)batch * L.num_kv_heads * (num_splits > 0 ? num_splits : 1);
     if (wgs <= cus)
         return true;
     if (L.kv_type == KV_Q4_0 || (L.head_dim == 64 && L.kv_type != KV_F32))
-        return wgs <= 6 * cus;
+        return wgs <= (batch <= 64 ? 6 : 3) * cus;
     if (L.head_dim == 128 && (L.kv_type == KV_F32 || L.kv_type == KV_F16) &&
         split_tokens >= (L.kv_type == KV_F32 ? 2000 : 4096))
         return false;

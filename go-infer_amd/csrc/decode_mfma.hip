@@ -1141,6 +1141,11 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     const int j = lane & 15, g = lane >> 4;
     const int H = a.num_heads, KVH = L.num_kv_heads, G = H / KVH, P = L.page_tokens;
     const int h0 = kvh * G;
+    // a step of several rows: their lengths, for share_tokens
+    const bool rows_meet = a.new_k && a.batch > 1;
+    int lens = 0;
+    if (rows_meet)
+        lens = a.seq_lens[min(lane, a.batch - 1)];
     int len = a.seq_lens[b];
     if (len > a.max_blocks * P || len < 0) {
         // more tokens than the block table maps (read what it maps), or a
@@ -1166,10 +1171,12 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     // which should not hold up the block's loads), and waits for the stores
     // to complete only before it issues the token's block.  The other waves
     // never wait.  Wider pages share lines between the blocks of two waves,
-    // so there every thread joins the store and a barrier follows.  No other
-    // workgroup reads that token's bytes (other kv heads are other bytes,
-    // split ranges are whole pages).  A length the tables cannot hold is
-    // flagged, as the separate append does, and nothing is stored.
+    // so there every thread joins the store and a barrier follows.  Other kv
+    // heads are other bytes and split ranges are whole pages, so within the
+    // row no other workgroup reads that token's bytes; other rows that map
+    // its page store it for themselves (share_tokens).  A length the tables
+    // cannot hold is flagged, as the separate append does, and nothing is
+    // stored.
     int sblk = -1;          // the token's block, in the wave that stores it
     int64_t st_page = 0;    // and where the token goes
     int st_slot = 0;
@@ -1177,10 +1184,10 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     // position outside the table is flagged, its q left as it is and nothing
     // stored, as the separate launch has it.
     const float2 *cs = nullptr;
-    auto token_k = [&](int64_t e0, int d) {
+    auto token_k = [&](int64_t e0, int d, const float2 *t) {
         const float x = a.new_k[e0 + d];
         if constexpr (ROPE)
-            return rope_elem<HD>(d, x, a.new_k[e0 + (d ^ (HD / 2))], cs[d & (HD / 2 - 1)]);
+            return rope_elem<HD>(d, x, a.new_k[e0 + (d ^ (HD / 2))], t[d & (HD / 2 - 1)]);
         return x;
     };
     if (a.new_k) {
@@ -1208,19 +1215,20 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
                 const int64_t e0 = ((int64_t)b * L.num_kv_heads + kvh) * HD;
                 const int d = threadIdx.x;
                 if (okp && d < HD)
-                    store_token_elem<KT>(L, a.append_base + pg * L.page_bytes, pos % P, kvh, d, token_k(e0, d),
+                    store_token_elem<KT>(L, a.append_base + pg * L.page_bytes, pos % P, kvh, d, token_k(e0, d, cs),
                                          a.new_v[e0 + d], true);
                 __syncthreads();
             }
         }
     }
-    auto store_token = [&]() {
-        const int64_t e0 = ((int64_t)b * L.num_kv_heads + kvh) * HD;
+    auto store_row = [&](int row, int64_t page, int slot, const float2 *t) {
+        const int64_t e0 = ((int64_t)row * L.num_kv_heads + kvh) * HD;
 #pragma unroll
         for (int d = lane; d < HD; d += 64)
-            store_token_elem<KT>(L, a.append_base + st_page * L.page_bytes, st_slot, kvh, d, token_k(e0, d),
+            store_token_elem<KT>(L, a.append_base + page * L.page_bytes, slot, kvh, d, token_k(e0, d, t),
                                  a.new_v[e0 + d], true);
     };
+    auto store_token = [&]() { store_row(b, st_page, st_slot, cs); };
 
     // The per-wave staging areas of the block loop (quantised and f32 pages,
     // and fp16 K) and, after it, the cross-wave merge share one LDS
@@ -1232,7 +1240,8 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     constexpr int MERGE_BYTES = NW * 16 * HD * (int)sizeof(float);
     __shared__ __align__(16) uint8_t s_stage[STAGE_BYTES > MERGE_BYTES ? STAGE_BYTES : MERGE_BYTES];
     float(*s_o)[16][HD] = reinterpret_cast<float(*)[16][HD]>(s_stage);
-    __shared__ float s_m[NW][16], s_l[NW][16];
+    __shared__ float s_ml[2][NW][16];
+    float(*s_m)[16] = s_ml[0], (*s_l)[16] = s_ml[1];
 
     float *wsp = nullptr;
     if (a.num_splits > 1)
@@ -1270,7 +1279,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     h8 qh[KK], ql[KK], qh1[KK];
     f4 qz[KK]; // quantised pages: the initial value of each k-step's product
     float c = 0.0f;
-    auto load_q = [&]() {
+    auto load_q = [&](auto &&between) {
         float qv[KK][8];
         float mq = 0.0f;
         const float *qp = a.q + (qrow + qhead) * HD + 8 * g;
@@ -1287,13 +1296,22 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
             qv[kk][6] = x1.z;
             qv[kk][7] = x1.w;
         }
+        float4 turn[ROPE ? KK / 2 : 1][4];
+        if (ROPE && cs) {
+#pragma unroll
+            for (int kk = 0; kk < KK / 2; kk++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    turn[kk][v] = *reinterpret_cast<const float4 *>(cs + 32 * kk + 8 * g + 2 * v);
+        }
+        between();
         if (ROPE && cs) {
             // a pair (d, d + HD / 2) is k-steps kk and kk + KK / 2 of one lane
 #pragma unroll
             for (int kk = 0; kk < KK / 2; kk++)
 #pragma unroll
                 for (int v = 0; v < 8; v += 2) {
-                    const float4 t = *reinterpret_cast<const float4 *>(cs + 32 * kk + 8 * g + v);
+                    const float4 t = turn[kk][v / 2];
                     float *x = &qv[kk][v], *y = &qv[kk + KK / 2][v];
                     rope_pair(x[0], y[0], t.x, t.y, &x[0], &y[0]);
                     rope_pair(x[1], y[1], t.z, t.w, &x[1], &y[1]);
@@ -1384,6 +1402,87 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     const bool store_late = sblk >= 0 && sblk != base;
     if (sblk >= 0 && !store_late)
         store_token();
+    // Rows of one step may attend each other's tokens (the same table at
+    // lengths n, n + 1, ...), and the workgroup that stores another row's
+    // token is not ordered with this one.  So a wave whose blocks hold a page
+    // that another row writes stores that row's token too: the same bytes as
+    // its owner, visible to this wave's own loads once the stores have
+    // completed.  Lane i holds the page that row r0 + i writes (row_page);
+    // the pages of the wave's blocks (own_page, one per 16 tokens) go into a
+    // hash of 1024 bits in LDS, and what it lets through is compared exactly.
+    // The first 64 of both are requested before the first block (row_page
+    // depends on lens, requested with this row's length) and looked at while
+    // the block and q are in flight: +0.5 us for 64 x 1500-3000 q4_0 and q8_0,
+    // nothing for f16 and f32 (after q's loads had returned, 32 compares of
+    // one page each: +1.5 to 2.5).
+    auto row_page = [&](int r0, int len_) { // of row r0 + lane, whose length is len_
+        const int row = min(r0 + lane, a.batch - 1), at = min(max(len_ - 1, 0), a.max_blocks * P - 1);
+        return a.block_tables[(int64_t)row * a.max_blocks + at / P];
+    };
+    auto own_page = [&](int t) { // of the lane's 16 tokens of the 32 blocks from t
+        return bt[min(t + stride * (lane >> 1) + 16 * (lane & 1), t1 - 1) / P];
+    };
+    volatile uint32_t *seen = reinterpret_cast<volatile uint32_t *>(s_ml[0][w]);
+    int rows_pg = 0, own_pg = 0;
+    auto look = [&]() {
+        if (rows_meet) {
+            rows_pg = row_page(0, lens);
+            own_pg = own_page(base);
+        }
+    };
+    // Returns whether it stored anything; the caller then loads its first
+    // block again.
+    auto share_tokens = [&]() {
+        if (!rows_meet)
+            return false;
+        bool any = false;
+        int len_ = lens, page = rows_pg;
+        for (int r0 = 0;;) {
+            const int row = r0 + lane, at = len_ - 1;
+            const bool live = row < a.batch && row != b && at >= 0 && at < a.max_blocks * P &&
+                              (!ROPE || at < a.rope_max_pos) && page >= 0 && page < L.num_pages;
+            uint64_t hit = 0;
+            int id = own_pg;
+            for (int t = base;;) {
+                // the groups' pages as bits of a hash (groups past t1 repeat
+                // the last page), then the exact look at what it lets through
+                auto bits = [&](int x) { return seen + ((x >> 9) & 1) * (NW * 16) + ((x >> 5) & 15); };
+                if (lane < 32)
+                    *bits(lane << 5) = 0;
+                __builtin_amdgcn_wave_barrier();
+                __hip_atomic_fetch_or(bits(id), 1u << (id & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+                __builtin_amdgcn_wave_barrier();
+                uint64_t may = __ballot(*bits(page) >> (page & 31) & 1);
+                __builtin_amdgcn_wave_barrier();
+                for (may &= __ballot(live); __builtin_expect(may != 0, 0); may &= may - 1) {
+                    const int i = __builtin_ctzll(may);
+                    if (__ballot(id == __builtin_amdgcn_readlane(page, i)))
+                        hit |= 1ull << i;
+                }
+                t += 32 * stride;
+                if (t >= t1)
+                    break;
+                id = own_page(t);
+            }
+            any |= hit != 0;
+            for (; __builtin_expect(hit != 0, 0); hit &= hit - 1) {
+                const int i = __builtin_ctzll(hit);
+                const int pos = __builtin_amdgcn_readlane(at, i);
+                const float2 *t = nullptr;
+                if constexpr (ROPE)
+                    t = a.rope + (int64_t)pos * (HD / 2);
+                store_row(r0 + i, __builtin_amdgcn_readlane(page, i), pos % P, t);
+            }
+            r0 += 64;
+            if (r0 >= a.batch)
+                break;
+            len_ = a.seq_lens[min(r0 + lane, a.batch - 1)];
+            page = row_page(r0, len_);
+        }
+        if (any)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return any;
+    };
     if constexpr (QUANT) {
         const int64_t ksoff = L.ks_off + (int64_t)kvh * P * KK * 2;
         const int64_t vsoff = L.vs_off + (int64_t)kvh * KK * P * 2;
@@ -1394,9 +1493,16 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
             int ok;
             store_done(base);
             block_pages(a, bt, base, t1, pA, pB, sA, sB, ok);
-            issue_qk<KT, HD, kStageAux>(a, pA, pB, sA, sB, koff, lane, Sq);
-            issue_qv<KT, HD, kStageAux>(a, pA, pB, sA, sB, ksoff, voff, vsoff, lane, Sq);
-            load_q();
+            look();
+            auto first = [&]() {
+                issue_qk<KT, HD, kStageAux>(a, pA, pB, sA, sB, koff, lane, Sq);
+                issue_qv<KT, HD, kStageAux>(a, pA, pB, sA, sB, ksoff, voff, vsoff, lane, Sq);
+            };
+            first();
+            load_q([&]() {
+                if (share_tokens())
+                    first();
+            });
             if (store_late)
                 store_token();
             // Loads go out in the order K codes, scales, V codes of one
@@ -1463,8 +1569,12 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
             int ok;
             store_done(base);
             block_pages(a, bt, base, t1, pA, pB, sA, sB, ok);
+            look();
             issue_f32<HD, kStageAux>(a, pA, pB, sA, sB, koff, voff, fl, Sf);
-            load_q();
+            load_q([&]() {
+                if (share_tokens())
+                    issue_f32<HD, kStageAux>(a, pA, pB, sA, sB, koff, voff, fl, Sf);
+            });
             if (store_late)
                 store_token();
             for (;;) {
@@ -1522,9 +1632,16 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
             int ok;
             store_done(base);
             block_pages(a, bt, base, t1, pA, pB, sA, sB, ok);
-            issue_k_f16(a, pA, pB, sA, sB, koff, lane, Sk);
-            load_v<HD, NT>(a, pA, pB, sA, sB, voff, j, g, v);
-            load_q();
+            look();
+            auto first = [&]() {
+                issue_k_f16(a, pA, pB, sA, sB, koff, lane, Sk);
+                load_v<HD, NT>(a, pA, pB, sA, sB, voff, j, g, v);
+            };
+            first();
+            load_q([&]() {
+                if (share_tokens())
+                    first();
+            });
             if (store_late)
                 store_token();
             // the first block: everything issued so far
@@ -1567,9 +1684,16 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
         int ok;
         store_done(base);
         block_pages(a, bt, base, t1, pA, pB, sA, sB, ok);
-        load_k<HD, NT>(a, pA, pB, sA, sB, koff, j, g, k0, k1);
-        load_v<HD, NT>(a, pA, pB, sA, sB, voff, j, g, v);
-        load_q();
+        look();
+        auto first = [&]() {
+            load_k<HD, NT>(a, pA, pB, sA, sB, koff, j, g, k0, k1);
+            load_v<HD, NT>(a, pA, pB, sA, sB, voff, j, g, v);
+        };
+        first();
+        load_q([&]() {
+            if (share_tokens())
+                first();
+        });
         if (store_late)
             store_token();
         f4 s0, s1;

@@ -304,7 +304,9 @@ int gi_paged_decode_attention_noalloc(gi_paged *h, int layer, int batch, int num
  * included), as Forward stores then attends (forward.go:236-267).  Where the
  * decode grid is one round of workgroups (small batches), the matrix-core
  * kernels store the token themselves in the same launch; the stored bytes
- * and the outputs are those of the two calls. */
+ * and the outputs are those of the two calls, also where rows share pages
+ * (draft tokens of one sequence as rows of lengths n, n + 1, ...): each row
+ * attends the tokens that the step's other rows store below its length. */
 int gi_paged_decode_step(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                          const float *k, const float *v, float *out, const int32_t *block_tables,
                          int max_blocks, const int32_t *seq_lens, int max_seq_len, float scale);
@@ -345,7 +347,7 @@ int gi_paged_rope_append_at_len(gi_paged *h, int layer, int batch, int num_heads
 /* One decode step of one layer from the projections: q (rotated in place,
  * as ApplyRoPE turns a.Q) and k are turned at position seq_lens[b]-1, k/v
  * appended, then gi_paged_decode_attention over seq_lens[b] tokens
- * (forward.go:228-267). */
+ * (forward.go:228-267); rows may share pages as in gi_paged_decode_step. */
 int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, float *q, const float *k,
                               const float *v, float *out, const int32_t *block_tables, int max_blocks,
                               const int32_t *seq_lens, int max_seq_len, float scale);
