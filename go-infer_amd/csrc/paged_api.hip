@@ -29,57 +29,6 @@ int set_error(int code, const std::string &msg)
 
 void clear_error() { g_last_error.clear(); }
 
-int devbuf_reserve(DevBuffer &b, size_t need, hipStream_t st, const char *what)
-{
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(st, &cs);
-    if (e != hipSuccess)
-        return set_error(GI_ERR_HIP, std::string(what) + ": hipStreamIsCapturing: " + hipGetErrorString(e));
-    const bool capturing = cs != hipStreamCaptureStatusNone;
-    if (capturing)
-        b.captured = true;
-    if (need <= b.bytes)
-        return GI_OK;
-    if (capturing)
-        return set_error(GI_ERR_BAD_ARG,
-                         std::string(what) + ": needs " + std::to_string(need) + " bytes of workspace (holds " +
-                             std::to_string(b.bytes) +
-                             ") while the stream is capturing a graph; make one eager call of this shape "
-                             "(or a larger batch) before capturing");
-    if (b.ptr) {
-        if (b.captured) {
-            // a captured graph may still address it: keep it until release
-            b.retired.push_back(b.ptr);
-        } else {
-            // work already queued may still read it
-            e = hipStreamSynchronize(st);
-            if (e != hipSuccess)
-                return set_error(GI_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
-            (void)hipFree(b.ptr);
-        }
-        b.ptr = nullptr;
-        b.bytes = 0;
-    }
-    const size_t want = need + need / 4;
-    void *p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess)
-        return set_error(GI_ERR_OOM, std::string(what) + ": hipMalloc(" + std::to_string(want) + ") failed");
-    b.ptr = p;
-    b.bytes = want;
-    return GI_OK;
-}
-
-void devbuf_release(DevBuffer &b)
-{
-    if (b.ptr)
-        (void)hipFree(b.ptr);
-    for (void *p : b.retired)
-        (void)hipFree(p);
-    b.retired.clear();
-    b.ptr = nullptr;
-    b.bytes = 0;
-}
-
 } // namespace gi
 
 struct gi_paged {
@@ -638,25 +587,24 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
     const int max_len = (int)(max_seq_len > 0 && max_seq_len < mapped ? max_seq_len
                               : mapped < INT32_MAX ? mapped : INT32_MAX);
     gi::decode_plan(h->L, batch, num_heads, max_len, h->num_cus, &a.split_tokens, &a.num_splits);
-    // the workspace first: a call refused here has queued nothing
+    // the workspace first: a call refused here has queued nothing.  Partials
+    // that the scratch cannot hold, that a capturing stream cannot allocate or
+    // that a full device has no room for: fewer, longer splits may still fit.
     size_t need = gi::decode_workspace_bytes(h->L, batch, num_heads, a.num_splits);
     int coarse_tokens, coarse_splits;
     gi::decode_plan_coarse(h->L, batch, max_len, h->num_cus, &coarse_tokens, &coarse_splits);
     const size_t coarse = gi::decode_workspace_bytes(h->L, batch, num_heads, coarse_splits);
-    if (need > (fixed_ws ? fixed_cap : h->plan_ws.bytes)) {
-        // partials that the scratch cannot hold, or that a capturing stream
-        // cannot allocate: fewer, longer splits may still fit
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusActive;
-        if (!fixed_ws) {
-            hipError_t e = hipStreamIsCapturing(h->stream, &cs);
-            if (e != hipSuccess)
-                return hip_fail(e, "decode attention: hipStreamIsCapturing");
-        }
-        if (cs != hipStreamCaptureStatusNone) {
-            a.split_tokens = coarse_tokens;
-            a.num_splits = coarse_splits;
-            need = coarse;
-        }
+    bool use_coarse = fixed_ws && need > fixed_cap;
+    if (!fixed_ws) {
+        const int rc = gi::devbuf_reserve_plan(h->plan_ws, need, coarse, h->stream, "decode attention", &use_coarse);
+        if (rc)
+            return rc;
+        a.ws = (float *)h->plan_ws.ptr;
+    }
+    if (use_coarse) {
+        a.split_tokens = coarse_tokens;
+        a.num_splits = coarse_splits;
+        need = coarse;
     }
     a.waves = gi::decode_waves(h->L, batch, a.num_splits, h->num_cus);
     std::unique_lock<std::mutex> order; // the shared scratch's users, in turn
@@ -681,33 +629,6 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
             if (e != hipSuccess)
                 return hip_fail(e, "gi_paged_decode_attention_noalloc: hipStreamWaitEvent");
         }
-    } else {
-        // an eager call also makes room for the coarse plan of its shape, so
-        // that a later capture of any shape no larger finds room
-        const bool grows = h->plan_ws.bytes < need || h->plan_ws.bytes < coarse;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (grows) {
-            const hipError_t e = hipStreamIsCapturing(h->stream, &cs);
-            if (e != hipSuccess)
-                return hip_fail(e, "decode attention: hipStreamIsCapturing");
-        }
-        const size_t want = grows && cs == hipStreamCaptureStatusNone && coarse > need ? coarse : need;
-        int rc = gi::devbuf_reserve(h->plan_ws, want, h->stream, "decode attention");
-        if (rc == GI_ERR_OOM && want > coarse) { // a full device: the plan with fewer partials
-            (void)hipGetLastError();
-            gi::clear_error();
-            a.split_tokens = coarse_tokens;
-            a.num_splits = coarse_splits;
-            a.waves = gi::decode_waves(h->L, batch, a.num_splits, h->num_cus);
-            rc = gi::devbuf_reserve(h->plan_ws, coarse, h->stream, "decode attention");
-        } else if (rc == GI_ERR_OOM && need == 0) { // unsplit: it was for a later capture only
-            (void)hipGetLastError();
-            gi::clear_error();
-            rc = GI_OK;
-        }
-        if (rc)
-            return rc;
-        a.ws = (float *)h->plan_ws.ptr;
     }
     if (new_k) {
         // a decode step: the token goes into the decode launch where that
@@ -866,28 +787,16 @@ int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len,
     p.kernel = h->decode_kernel;
     gi::prefill_plan(h->L, batch, chunk_len, num_heads, (int64_t)max_blocks * h->L.page_tokens, p.kernel, h->num_cus,
                      &p.num_splits, &p.narrow);
-    const size_t need = gi::prefill_workspace_bytes(p);
-    if (need) {
-        // a capturing stream cannot allocate: the context stays in one piece
-        // where no earlier call has made room
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        hipError_t e = need > h->prefill_ws.bytes ? hipStreamIsCapturing(h->stream, &cs) : hipSuccess;
-        if (e != hipSuccess)
-            return hip_fail(e, "gi_paged_prefill_attention: hipStreamIsCapturing");
-        if (cs != hipStreamCaptureStatusNone) {
-            p.num_splits = 1;
-        } else {
-            rc = gi::devbuf_reserve(h->prefill_ws, need, h->stream, "prefill attention");
-            if (rc == GI_ERR_OOM) { // a full device: one piece needs no memory
-                (void)hipGetLastError();
-                gi::clear_error();
-                p.num_splits = 1;
-            } else if (rc) {
-                return rc;
-            }
-            p.ws = (float *)h->prefill_ws.ptr;
-        }
-    }
+    // no room for the partials (a capturing stream cannot allocate, the device
+    // may be full): the context stays in one piece, which needs none
+    bool whole = false;
+    rc = gi::devbuf_reserve_plan(h->prefill_ws, gi::prefill_workspace_bytes(p), 0, h->stream, "prefill attention",
+                                 &whole);
+    if (rc)
+        return rc;
+    if (whole)
+        p.num_splits = 1;
+    p.ws = (float *)h->prefill_ws.ptr;
     hipError_t e = gi::launch_prefill(p, h->stream);
     return e == hipSuccess ? GI_OK : hip_fail(e, "gi_paged_prefill_attention");
 }
