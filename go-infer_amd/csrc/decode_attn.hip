@@ -494,6 +494,18 @@ void decode_plan_coarse(const PoolLayout &L, int batch, int max_len, int num_cus
     set_plan(L, max_len, (int)min(s, ((int64_t)max_len + 1023) / 1024), split_tokens, num_splits);
 }
 
+// Both plans keep to two workgroups per CU up to one (sequence, kv head) pair
+// per CU; decode_plan's five splits of up to 1.25 pairs per CU are the most of
+// all.
+size_t decode_workspace_ahead(const PoolLayout &L, int batch, int num_heads, int num_cus)
+{
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    const int64_t pairs = (int64_t)batch * L.num_kv_heads;
+    const int64_t slots = pairs <= cus ? 2 * cus : min(5 * pairs, 25 * cus / 4);
+    const int G = num_heads / L.num_kv_heads;
+    return (size_t)slots * G * (L.head_dim + 2) * sizeof(float);
+}
+
 // Whether a decode step stores its token inside the matrix-core decode
 // launch (DecodeArgs.new_k) rather than in an append launch before it:
 // when the grid fits the CUs at once (two workgroups each).  Measured

@@ -6,7 +6,7 @@
 
 namespace gi {
 
-int devbuf_reserve(DevBuffer &b, size_t need, hipStream_t st, const char *what)
+int devbuf_reserve(DevBuffer &b, size_t need, hipStream_t st, const char *what, size_t ahead)
 {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(st, &cs);
@@ -25,7 +25,7 @@ int devbuf_reserve(DevBuffer &b, size_t need, hipStream_t st, const char *what)
                              "before capturing");
     size_t got = 0;
     void *p = nullptr;
-    for (size_t want : {need + need / 4, need}) {
+    for (size_t want : {ahead ? std::max(ahead, need) : need + need / 4, need}) {
         if (hipMalloc(&p, want) == hipSuccess) {
             got = want;
             break;
@@ -54,7 +54,8 @@ int devbuf_reserve(DevBuffer &b, size_t need, hipStream_t st, const char *what)
     return GI_OK;
 }
 
-int devbuf_reserve_plan(DevBuffer &b, size_t need, size_t lean, hipStream_t st, const char *what, bool *use_lean)
+int devbuf_reserve_plan(DevBuffer &b, size_t need, size_t lean, size_t ahead, hipStream_t st, const char *what,
+                        bool *use_lean)
 {
     *use_lean = false;
     if (need == 0 && lean == 0)
@@ -71,7 +72,7 @@ int devbuf_reserve_plan(DevBuffer &b, size_t need, size_t lean, hipStream_t st, 
     if (std::max(need, lean) <= b.bytes)
         return GI_OK;
     // room for either plan, or for the better one, or for the lean one
-    int rc = devbuf_reserve(b, std::max(need, lean), st, what);
+    int rc = devbuf_reserve(b, std::max(need, lean), st, what, ahead);
     if (rc != GI_ERR_OOM)
         return rc;
     if (need < lean) {

@@ -85,6 +85,9 @@ struct DecodeArgs {
 
 // Bytes of split-K workspace needed for a decode launch.
 size_t decode_workspace_bytes(const PoolLayout &L, int batch, int num_heads, int num_splits);
+// The most of it that either plan below asks for at this head count, for any
+// context and any batch up to this one.
+size_t decode_workspace_ahead(const PoolLayout &L, int batch, int num_heads, int num_cus);
 
 // Whether a decode step's token store goes into the matrix-core decode
 // launch (DecodeArgs.new_k) for this grid, rather than an append launch.
@@ -149,6 +152,8 @@ struct PrefillArgs {
 void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
                   int num_cus, int *num_splits, bool *narrow);
 size_t prefill_workspace_bytes(const PrefillArgs &a);
+// The most that any plan asks for.
+size_t prefill_workspace_ahead(const PoolLayout &L, int num_cus);
 
 hipError_t launch_prefill(const PrefillArgs &a, hipStream_t st);
 

@@ -596,7 +596,9 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
     const size_t coarse = gi::decode_workspace_bytes(h->L, batch, num_heads, coarse_splits);
     bool use_coarse = fixed_ws && need > fixed_cap;
     if (!fixed_ws) {
-        const int rc = gi::devbuf_reserve_plan(h->plan_ws, need, coarse, h->stream, "decode attention", &use_coarse);
+        const size_t ahead = gi::decode_workspace_ahead(h->L, batch, num_heads, h->num_cus);
+        const int rc =
+            gi::devbuf_reserve_plan(h->plan_ws, need, coarse, ahead, h->stream, "decode attention", &use_coarse);
         if (rc)
             return rc;
         a.ws = (float *)h->plan_ws.ptr;
@@ -790,8 +792,8 @@ int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len,
     // no room for the partials (a capturing stream cannot allocate, the device
     // may be full): the context stays in one piece, which needs none
     bool whole = false;
-    rc = gi::devbuf_reserve_plan(h->prefill_ws, gi::prefill_workspace_bytes(p), 0, h->stream, "prefill attention",
-                                 &whole);
+    rc = gi::devbuf_reserve_plan(h->prefill_ws, gi::prefill_workspace_bytes(p), 0,
+                                 gi::prefill_workspace_ahead(h->L, h->num_cus), h->stream, "prefill attention", &whole);
     if (rc)
         return rc;
     if (whole)

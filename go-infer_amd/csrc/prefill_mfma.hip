@@ -2697,6 +2697,12 @@ size_t prefill_workspace_bytes(const PrefillArgs &a)
     return (size_t)a.num_splits * a.batch * a.chunk_len * a.num_heads * (a.L.head_dim + 2) * sizeof(float);
 }
 
+// Split workgroups of 128 columns, at most two per CU (prefill_plan).
+size_t prefill_workspace_ahead(const PoolLayout &L, int num_cus)
+{
+    return (size_t)2 * (num_cus > 0 ? num_cus : 256) * 128 * (L.head_dim + 2) * sizeof(float);
+}
+
 hipError_t launch_prefill_mfma(const PrefillArgs &a, hipStream_t st)
 {
     using namespace mfma_prefill;

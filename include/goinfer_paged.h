@@ -265,13 +265,17 @@ int gi_paged_gather(gi_paged *h, int layer, const int32_t *block_table, int n_to
  *
  * Workspace: the handle keeps the partials of split sequences, batch *
  * num_kv_heads * splits slots of (num_heads / num_kv_heads) * (head_dim + 2)
- * floats, where splits falls as batch * num_kv_heads grows (at most six
- * workgroups per CU).  A call that needs it to grow while the handle's stream
- * is capturing a graph takes fewer, longer splits (at least 1024 tokens, about
- * one workgroup per CU), and fails with GI_ERR_BAD_ARG where their partials
- * do not fit either (make one eager call with the same shape first); once any
- * call has been captured, growth keeps the old buffers alive until
- * gi_paged_destroy, so captured graphs stay valid. */
+ * floats, where splits falls as batch * num_kv_heads grows: at most two slots
+ * per CU up to batch * num_kv_heads of one per CU, and 6.25 in all.  The first
+ * eager call that splits allocates the most that its head count and any batch
+ * up to its own can need, whatever the context (just its own partials where
+ * the device has no room for that), and a call that finds no room for those
+ * takes fewer, longer splits (at least 1024 tokens, about one workgroup per
+ * CU).  A call whose stream is capturing a graph never allocates: it too takes
+ * the fewer splits where the workspace holds no more, and fails with
+ * GI_ERR_BAD_ARG where it does not hold those either (make one eager call with
+ * the same shape first); once any call has been captured, growth keeps the old
+ * buffers alive until gi_paged_destroy, so captured graphs stay valid. */
 int gi_paged_decode_attention(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                               float *out, const int32_t *block_tables, int max_blocks,
                               const int32_t *seq_lens, int max_seq_len, float scale);
@@ -357,9 +361,10 @@ int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, 
  * [0, start_pos[b] + i + 1).  q, out [batch][chunk_len][num_heads][head_dim]
  * float32.  Launches that leave CUs idle cut the context, as decode does; the
  * handle keeps splits * batch * chunk_len * num_heads * (head_dim + 2) floats
- * for the partials (at most 34 MB on a 256-CU device), grown as needed and kept
- * as decode's; a capturing stream that would need it to grow, or a device
- * without room, keeps the context in one piece.  Replays of captured calls
+ * for the partials, allocated for any later call of the pool (34 MB at head_dim
+ * 128 on a 256-CU device) with the first eager call that cuts; a capturing
+ * stream that finds no room, or a device without any, keeps the context in one
+ * piece.  Replays of captured calls
  * that could overlap other prefill calls of the handle must be serialised. */
 int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len, int num_heads,
                                const float *q, float *out, const int32_t *block_tables,

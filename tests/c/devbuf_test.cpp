@@ -37,9 +37,9 @@ static DevBuffer held(size_t bytes, size_t room) // a buffer of `bytes` and room
     return b;
 }
 
-static int plan(DevBuffer &b, size_t need, size_t lean, bool *use_lean)
+static int plan(DevBuffer &b, size_t need, size_t lean, bool *use_lean, size_t ahead = 0)
 {
-    return devbuf_reserve_plan(b, need, lean, nullptr, "test", use_lean);
+    return devbuf_reserve_plan(b, need, lean, ahead, nullptr, "test", use_lean);
 }
 
 int main()
@@ -83,6 +83,15 @@ int main()
         CHECK(plan(e, 300, 100, &lean) == GI_OK && !lean && e.bytes == 375);
         CHECK(plan(e, 200, 375, &lean) == GI_OK && !lean && fake::mallocs == 1);
         CHECK(plan(e, 0, 0, &lean) == GI_OK && !lean);
+    }
+    { // what later calls can need is allocated with the first growth, where it fits
+        DevBuffer b = held(0, 1000);
+        CHECK(plan(b, 0, 0, &lean, 800) == GI_OK && fake::mallocs == 0);
+        for (size_t need = 50; need <= 800; need += 50)
+            CHECK(plan(b, need, 40, &lean, 800) == GI_OK && !lean && b.bytes == 800 && fake::mallocs == 1);
+        DevBuffer c = held(0, 500);
+        CHECK(plan(c, 300, 100, &lean, 800) == GI_OK && !lean && c.bytes == 300);
+        CHECK(plan(c, 900, 100, &lean, 800) == GI_OK && lean && c.bytes == 300);
     }
     { // a capturing stream never allocates, synchronises or frees
         DevBuffer b = held(200, 1000);
