@@ -1715,8 +1715,10 @@ struct PrefillWork {
         }
     }
 
-    // SPLIT: no column of the workgroup reaches this split's tokens.
-    __device__ __forceinline__ bool empty() const { return SPLIT && t0 >= wg_len; }
+    // SPLIT: no column of the workgroup reaches this split's tokens.  The one
+    // split of a short sequence writes its columns' output in any case (zeros
+    // for queries before position 0, which attend nothing).
+    __device__ __forceinline__ bool empty() const { return SPLIT && t0 >= wg_len && (t0 > 0 || part >= 0); }
 
     // Whether the block at `base` is whole for every column of the workgroup
     // (PAIRED: of this wave's half): all its tokens valid and before the

@@ -105,3 +105,31 @@ def test_prefill_splits_skip_a_bad_page(gi, oracle, dev, kv_type):
         pop.pool.synchronize()
     assert e.value.code == -7
     assert float(rel_err_rows(out[0].cpu().numpy(), want, H, hd).max()) <= TOL
+
+
+# q4_0 pages at head dimension 64 run on the vector kernel, which cuts nothing
+@pytest.mark.parametrize("kv_type,hd", [(0, 64), (0, 128), (1, 64), (1, 128), (2, 64), (2, 128), (3, 128)])
+def test_prefill_splits_queries_before_position_0(gi, oracle, dev, kv_type, hd):
+    """Queries that attend no token get zeros, in a sequence of which every
+    workgroup holds only such queries and in one that crosses position 0,
+    beside a sequence long enough to be cut."""
+    import torch
+    H, kvh, P, starts, chunk = 8, 2, 16, [-300, -20, 1000], 64
+    lens = [max(0, s + chunk) for s in starts]
+    pop = Populated(gi, dev, kv_type, 1, kvh, hd, P, lens, seed=95)
+    bt = pop.block_tables()
+    qd, q = seeded((len(starts), chunk, H * hd), 96, dev)
+    scale = oracle.attn_scale(hd)
+    out = torch.full_like(qd, float("nan"))
+    pop.pool.AttentionGQABatch(out, qd, 0, bt, torch.tensor(starts, dtype=torch.int32, device=dev), H, scale, chunk)
+    pop.pool.synchronize()
+    o = out.cpu().numpy()
+    for i, s in enumerate(starts):
+        skip = min(chunk, max(0, -s))  # queries before position 0
+        assert not o[i, :skip].any(), i
+        if skip == chunk:
+            continue
+        ks, vs = pop.stored(0, i)
+        want = causal64(q[i, skip:], oracle.widen(kv_type, kvh * hd, ks), oracle.widen(kv_type, kvh * hd, vs),
+                        H, kvh, hd, s + skip, scale)
+        assert float(rel_err_rows(o[i, skip:], want, H, hd).max()) <= TOL, i
