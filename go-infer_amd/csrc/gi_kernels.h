@@ -152,6 +152,12 @@ struct PrefillArgs {
 void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
                   int num_cus, int *num_splits, bool *narrow);
 size_t prefill_workspace_bytes(const PrefillArgs &a);
+// Floats of its (maximum, sum) part, in front of the unnormalised outputs,
+// which are read 16 bytes at a time.
+__host__ __device__ __forceinline__ int64_t prefill_ml_floats(int num_splits, int64_t rows)
+{
+    return (2 * num_splits * rows + 3) / 4 * 4;
+}
 // The most that any plan asks for.
 size_t prefill_workspace_ahead(const PoolLayout &L, int num_cus);
 

@@ -1586,7 +1586,7 @@ struct WaveAttn {
         if (part >= 0) {
             const int64_t rows = (int64_t)a.batch * chunk * H;
             float2 *ml = reinterpret_cast<float2 *>(a.ws) + part * rows;
-            float *ow = a.ws + 2 * a.num_splits * rows + part * rows * HD;
+            float *ow = a.ws + prefill_ml_floats(a.num_splits, rows) + part * rows * HD;
 #pragma unroll
             for (int cg = 0; cg < NCG; cg++) {
                 float lt = lsum[cg];
@@ -2498,7 +2498,7 @@ __global__ __launch_bounds__(256) void merge_prefill(PrefillArgs a)
         return;
     const int n = (min(start + qi + 1, mapped) + per - 1) / per;
     const float2 *ml = reinterpret_cast<const float2 *>(a.ws) + row;
-    const float *ow = a.ws + 2 * a.num_splits * rows + row * HD + d;
+    const float *ow = a.ws + prefill_ml_floats(a.num_splits, rows) + row * HD + d;
     float M = -INFINITY;
     for (int s = 0; s < n; s++)
         M = fmaxf(M, ml[s * rows].x);
@@ -2696,13 +2696,15 @@ size_t prefill_workspace_bytes(const PrefillArgs &a)
 {
     if (a.num_splits <= 1)
         return 0;
-    return (size_t)a.num_splits * a.batch * a.chunk_len * a.num_heads * (a.L.head_dim + 2) * sizeof(float);
+    const int64_t rows = (int64_t)a.batch * a.chunk_len * a.num_heads;
+    return (size_t)(prefill_ml_floats(a.num_splits, rows) + a.num_splits * rows * a.L.head_dim) * sizeof(float);
 }
 
 // Split workgroups of 128 columns, at most two per CU (prefill_plan).
 size_t prefill_workspace_ahead(const PoolLayout &L, int num_cus)
 {
-    return (size_t)2 * (num_cus > 0 ? num_cus : 256) * 128 * (L.head_dim + 2) * sizeof(float);
+    const int64_t rows = (int64_t)2 * (num_cus > 0 ? num_cus : 256) * 128; // of all splits
+    return (size_t)(prefill_ml_floats(1, rows) + rows * L.head_dim) * sizeof(float);
 }
 
 hipError_t launch_prefill_mfma(const PrefillArgs &a, hipStream_t st)

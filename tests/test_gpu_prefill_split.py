@@ -133,3 +133,24 @@ def test_prefill_splits_queries_before_position_0(gi, oracle, dev, kv_type, hd):
         want = causal64(q[i, skip:], oracle.widen(kv_type, kvh * hd, ks), oracle.widen(kv_type, kvh * hd, vs),
                         H, kvh, hd, s + skip, scale)
         assert float(rel_err_rows(o[i, skip:], want, H, hd).max()) <= TOL, i
+
+
+# 16 heads per kv head (fp16 pages; the others run on the vector kernel), and
+# an odd number of rows in an odd number of splits, whose (maximum, sum) part
+# is no multiple of 16 bytes
+@pytest.mark.parametrize("kv_type,H,kvh,hd,start,chunk", [
+    (1, 16, 1, 128, 1500, 77), (1, 32, 2, 128, 700, 130), (0, 9, 9, 128, 760, 45), (1, 9, 9, 64, 760, 45),
+    (2, 9, 9, 64, 760, 45), (3, 9, 9, 128, 760, 45)])
+def test_prefill_splits_of_other_head_layouts(gi, oracle, dev, kv_type, H, kvh, hd, start, chunk):
+    import torch
+    pop = Populated(gi, dev, kv_type, 1, kvh, hd, 16, [start + chunk], seed=97)
+    qd, q = seeded((1, chunk, H * hd), 98, dev)
+    scale = oracle.attn_scale(hd)
+    out = torch.full_like(qd, float("nan"))
+    pop.pool.AttentionGQABatch(out, qd, 0, pop.block_tables(), torch.tensor([start], dtype=torch.int32, device=dev),
+                               H, scale, chunk)
+    pop.pool.synchronize()
+    ks, vs = pop.stored(0, 0)
+    want = causal64(q[0], oracle.widen(kv_type, kvh * hd, ks), oracle.widen(kv_type, kvh * hd, vs), H, kvh, hd, start,
+                    scale)
+    assert float(rel_err_rows(out[0].cpu().numpy(), want, H, hd).max()) <= TOL
