@@ -1658,10 +1658,14 @@ __device__ __forceinline__ int split_len(const PoolLayout &L, int len, int n)
 // about the same work; each half then decides alone which blocks it sees
 // whole (wg_full is per half).
 //
-// SPLIT: blockIdx.x holds split * tiles + tile, and the workgroup covers the
-// context tokens [t0, t0 + per) of split_len; everything else stays in
+// SPLIT: blockIdx.z holds split * batch + sequence, and the workgroup covers
+// the context tokens [t0, t0 + per) of split_len; everything else stays in
 // absolute token positions.  part is the split, or -1 if the sequence is
-// short enough for one.
+// short enough for one.  The later splits of short sequences have nothing to
+// do; with the split slowest in the grid their workgroups start behind all
+// others and delay none (split within sequence and kv head: 4 x 128 queries
+// from position 0 under tables of 8192 tokens q8_0 at head dimension 64 17.8 ->
+// 13.2 us, f32 at 128 20.5 -> 18.1).
 template <int P, int NCG, int NW = 4, bool PAIRED = false, bool SPLIT = false>
 struct PrefillWork {
     int wx, kvh, b, tid, lane, w, j, g, start, mapped, col0, wave_len, wg_full, wg_len;
@@ -1672,11 +1676,11 @@ struct PrefillWork {
     __device__ __forceinline__ PrefillWork(const PrefillArgs &a)
     {
         constexpr int WCOLS = 16 * NCG;
-        const int tiles = SPLIT ? gridDim.x / a.num_splits : gridDim.x;
-        const int tile = SPLIT ? blockIdx.x % tiles : blockIdx.x;
-        wx = tiles - 1 - tile; // heaviest (latest-query) workgroups first
+        const int tiles = gridDim.x;
+        wx = tiles - 1 - blockIdx.x; // heaviest (latest-query) workgroups first
         kvh = blockIdx.y;
-        b = blockIdx.z;
+        const int split = SPLIT ? blockIdx.z / a.batch : 0;
+        b = blockIdx.z - split * a.batch;
         tid = threadIdx.x;
         lane = tid & 63;
         w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1705,7 +1709,6 @@ struct PrefillWork {
             atomicOr(a.status, FLAG_BAD_SLOT);
         if (SPLIT) {
             const int len = min(start + chunk, mapped), per = split_len(a.L, len, a.num_splits);
-            const int split = blockIdx.x / tiles;
             t0 = split * per;
             part = per < len ? split : -1;
             const int t1 = t0 + per;
@@ -2583,7 +2586,7 @@ static void launch_lds(const PrefillArgs &a, hipStream_t st)
         return dim3((unsigned)((cols + per_wg - 1) / per_wg), a.L.num_kv_heads, a.batch);
     };
     // one launch of KERNEL<..., SPLIT>, its grid widened by the splits
-#define GI_PGRID(ncg, nw) dim3(grid(ncg, nw).x * a.num_splits, a.L.num_kv_heads, a.batch)
+#define GI_PGRID(ncg, nw) dim3(grid(ncg, nw).x, a.L.num_kv_heads, a.batch * a.num_splits)
 #define GI_PP(KERNEL, ...)                                                                                \
     do {                                                                                                  \
         constexpr int WIDE = HD == 128 ? NCG : 1; /* columns of a wide split, see prefill_plan */         \
@@ -2660,11 +2663,18 @@ static void launch_lds(const PrefillArgs &a, hipStream_t st)
 //  - 1/2 to 2/3 of the CUs: three splits leave less idle than one, of 256
 //    columns where a wave can take them at head dimension 128 (2 x 300 queries
 //    behind 2000, one / three narrow / three wide: fp16 74 / 76 / 65, q8_0
-//    102 / 97 / 83, q4_0 97 / 92 / 76; f32 116 / 112, head dimension 64 fp16
-//    51 / 43 / 44, f32 115 / 90).  Wide splits elsewhere win by a few per
-//    cent at contexts over 3000 and lose more below.
+//    102 / 97 / 83, q4_0 97 / 92 / 76; head dimension 64 fp16 51 / 43 / 44,
+//    f32 115 / 90).  Not f32 pages at head dimension 128 (behind 600 48 / 59,
+//    behind 2000 105 / 98).  Wide splits elsewhere win by a few per cent at
+//    contexts over 3000 and lose more below.
 // The kernels cut each sequence's own context (split_len); the mapped length
-// only bounds the number of pieces.
+// only bounds the number of pieces.  So short contexts under wide tables pay
+// for a merge that has nothing to do: 40 to 300 queries from position 0,
+// tables of their own width / of 8192 tokens, f32 at head dimension 64 8.6 /
+// 11.0 and 20.3 / 22.5 us, fp16 at 128 9.7 / 12.1 and 16.4 / 18.3.  Merging in
+// the launch itself (by the workgroup that ends last) takes that away, but the
+// fence it needs across the XCDs costs every cut context 4 to 10 us (512
+// queries behind 2000 fp16 48.9 -> 59).
 void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, int64_t mapped, int requested,
                   int num_cus, int *num_splits, bool *narrow)
 {
@@ -2681,9 +2691,9 @@ void prefill_plan(const PoolLayout &L, int batch, int chunk_len, int num_heads, 
     *narrow = 16 * two <= 9 * cus;
     int64_t s = (L.kv_type == KV_Q8_0 && L.head_dim == 64 ? 2 * cus : cus) / wgs;
     bool wide = false;
-    if (s == 1 && 2 * wgs > cus && 3 * wgs <= 2 * cus) {
+    if (s == 1 && 2 * wgs > cus && 3 * wgs <= 2 * cus && !(L.kv_type == KV_F32 && L.head_dim == 128)) {
         s = 3;
-        wide = L.head_dim == 128 && L.kv_type != KV_F32;
+        wide = L.head_dim == 128;
     }
     s = std::min(s, mapped / mfma_prefill::kMinSplit);
     if (mapped > mfma_prefill::whole_len(L) && s > 1) {

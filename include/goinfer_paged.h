@@ -364,7 +364,11 @@ int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, 
  * for the partials, allocated for any later call of the pool (34 MB at head_dim
  * 128 on a 256-CU device) with the first eager call that cuts; a capturing
  * stream that finds no room, or a device without any, keeps the context in one
- * piece.  Replays of captured calls
+ * piece.  How many pieces are planned follows max_blocks * page_tokens, since
+ * the lengths are on the device: tables far wider than the context cost a
+ * merge launch that finds nothing to do (about 2.5 us), so pass the blocks in
+ * use where they are known (one sequence's table may be passed with any
+ * max_blocks that covers start_pos + chunk_len).  Replays of captured calls
  * that could overlap other prefill calls of the handle must be serialised. */
 int gi_paged_prefill_attention(gi_paged *h, int layer, int batch, int chunk_len, int num_heads,
                                const float *q, float *out, const int32_t *block_tables,
