@@ -16,8 +16,8 @@ float32 dot products of length cols:
 
 The shapes cover the three product forms: batches of up to 16, larger ones,
 and (F16 / F32 weights, large products) the split-K tiles;
-test_matmul_form_edges takes each at the sizes where its indexing can go
-wrong."""
+test_matmul_form_edges and test_matmul_split_k_edges take each at the sizes
+where its indexing can go wrong."""
 import numpy as np
 import pytest
 
@@ -148,6 +148,32 @@ def test_matmul_form_edges(gi, oracle, dev, t, rows, cols, batch):
     exact = x.astype(np.float64) @ dequant(oracle, t, raw, rows, cols).astype(np.float64).T
     bound = 4 * EPS32 * np.sqrt(cols) * (np.abs(x).astype(np.float64) @ wd.T)
     bound += 2.0**-21 * np.abs(x).max(axis=1, keepdims=True) * wd.sum(axis=1)[None]
+    assert np.isfinite(got).all()
+    assert float((np.abs(got - exact) / bound).max()) <= 1.0
+
+
+# Split-K at its own edges (F16 and F32 weights of 65536 and more 64 x 64 tiles
+# times k-steps): one slice, stored without a reduction, of rows that are no
+# multiple of 4; two slices of 73 and 72 k-steps whose reduction ends in a
+# scalar tail; sixteen slices of 86 and one of 76 over a batch whose last tile
+# has idle waves.
+@pytest.mark.parametrize("t", [0, 1], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,cols,batch,slices", [(4101, 2048, 1000, 1), (4099, 4640, 400, 2), (1000, 43712, 130, 16)])
+def test_matmul_split_k_edges(gi, oracle, dev, t, rows, cols, batch, slices):
+    KS, pad = cols // 32, (batch + 63) // 64 * 64
+    tiles = (rows + 127) // 128 * ((pad + 127) // 128)
+    assert (rows + 63) // 64 * (pad // 64) * KS >= 65536 and min(-(-256 // tiles), KS // 4) == slices
+    rng = np.random.default_rng(rows + cols + batch + t)
+    W = rng.standard_normal((rows, cols), np.float32)
+    x = rng.standard_normal((batch, cols), np.float32)
+    x[batch - 1] *= 1e3
+    raw = oracle.quantize_weights(t, W)
+    got = _run(gi, dev, t, rows, cols, raw, x)
+    wd = dequant(oracle, t, raw, rows, cols).astype(np.float64)
+    exact = x.astype(np.float64) @ wd.T
+    # as in test_matmul_form_edges
+    bound = 4 * EPS32 * np.sqrt(cols) * (np.abs(x).astype(np.float64) @ np.abs(wd).T)
+    bound += 2.0**-21 * np.abs(x).max(axis=1, keepdims=True) * np.abs(wd).sum(axis=1)[None]
     assert np.isfinite(got).all()
     assert float((np.abs(got - exact) / bound).max()) <= 1.0
 
