@@ -316,3 +316,12 @@ def test_rope_decode_step_equals_its_parts(gi, oracle, dev, kv_type, H, kvh, hd,
             assert torch.equal(x, y), i
     good = [i for i in range(B) if i not in bad]
     assert torch.equal(of[good], op[good])
+
+
+@pytest.mark.parametrize("H,kvh,lens", [
+    (16, 1, [90]), (32, 2, [700, 33]), (16, 1, [4000]),  # one split, merged by one wave and by four
+    (64, 4, [40 + i for i in range(70)])])               # four-wave workgroups
+def test_rope_decode_step_of_16_heads_per_kv_head(gi, oracle, dev, H, kvh, lens):
+    """fp16 pages with 16 query heads per kv head have a q operand and a
+    write-back of their own (the hi and lo halves do not share an operand)."""
+    test_rope_decode_step_equals_its_parts(gi, oracle, dev, 1, H, kvh, 128, 16, 128, lens)
