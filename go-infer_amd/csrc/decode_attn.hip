@@ -279,9 +279,10 @@ __global__ __launch_bounds__(NT) void attn_valu(DecodeArgs a)
 // LDS.  Latency bounds it, so a wave's first kMergeAhead partials are
 // requested together with the maxima of all splits: one round trip for up to
 // W * kMergeAhead splits.  W is 1 (four heads per workgroup, no barrier) for
-// up to kMergeAhead splits and 4 above (both also write a step's turned q,
-// DecodeArgs.rope, which every split has read by then): four waves per head on 2 splits of 52
+// up to kMergeAhead splits and 4 above: four waves per head on 2 splits of 52
 // sequences x 32 heads cost 1 us more than one (19.9 against 18.9 us a step).
+// Both also write a step's turned q (DecodeArgs.rope), which every split has
+// read by then.
 constexpr int kMergeAhead = 8;
 
 template <int HD, int W>

@@ -75,10 +75,10 @@ using mfma_ops::u4x8_to_h8;
 enum : int { W_F32 = 0, W_F16 = 1, W_Q4_0 = 2, W_Q8_0 = 8 }; // GGML type ids
 
 
-
-// Activation rows are padded to multiples of 64, the batch side of the
-// 64 x 64 output tile; weight rows to multiples of 128, the row side of the
-// split-K tile (and so of 64 too).
+// Activation rows are padded to multiples of 64, the widest batch side of
+// matmul_reg's tiles and half of matmul_sk's (whose waves past the padding
+// idle); weight rows to multiples of 128, the row side of the split-K tile and
+// a multiple of all others.
 __host__ __device__ __forceinline__ int64_t round_pad(int64_t n) { return (n + 63) / 64 * 64; }
 __host__ __device__ __forceinline__ int64_t weight_rows_pad(int64_t n) { return (n + 127) / 128 * 128; }
 
@@ -403,7 +403,7 @@ __device__ __forceinline__ void static_for(F &&f)
 // for quantised weights the scale multiply-adds beside the products.
 //
 // Per call with split_x, 4096 x 4096: batch 32 Q8_0 34.9 -> 15.4 us, F16 34.5
-// -> 17.1; batch 256 Q8_0 39.3 -> 31.5, F16 33.6 -> 31.5; 8192 x 8192, batch
+// -> 17.1; batch 256 Q8_0 39.0 -> 30.9, F16 33.6 -> 31.5; 8192 x 8192, batch
 // 64, Q8_0: 62.8 -> 42.7.  (Before: 64 x 64 tiles staged through LDS by four
 // waves, one per SIMD, on rows / 64 workgroups; F16 at batch 256 matmul_sk.)
 // Weights four k-steps ahead instead of one (tiles of up to 32 rows): Q8_0,
@@ -613,10 +613,10 @@ void launch_reg(const MatArgs &a, int batch_pad, hipStream_t st)
 // activation halves arrive by direct global->LDS loads two k-steps ahead,
 // through three stages; one barrier per k-step hands a stage from the loads
 // to the products.  The per-CU load volume is 24 KiB per 128 products against
-// 12 KiB per 32 in the 64 x 64 form.  With S > 1 the partial tiles go to a
-// workspace and reduce_splits adds them.  Quantised weights
-// do not take it: their per-block scale multiply-adds need 272 registers here
-// (one wave per SIMD).
+// matmul_reg's 10 to 12 KiB per 32.  With S > 1 the partial tiles go to a
+// workspace and reduce_splits adds them.  Quantised weights do not take it:
+// their per-block scale multiply-adds need 272 registers here (one wave per
+// SIMD).
 
 struct SKArgs {
     MatArgs m;
@@ -626,10 +626,11 @@ struct SKArgs {
     int batch_pad;
 };
 
-// The k-step slices give about kSplitKWorkgroups workgroups, none shorter than kMinSliceSteps
-// k-steps.  The form is taken from kSplitKMinSteps (64 x 64
-// tiles times k-steps) up, where matmul_reg's operand volume per product
-// costs more than the reduction launch here (per call, this / matmul_reg):
+// The k-step slices give about kSplitKWorkgroups workgroups, none shorter than
+// kMinSliceSteps k-steps.  The form is taken from kSplitKMinSteps (64 x 64
+// pieces of the output times k-steps) up, where matmul_reg's operand volume per
+// product costs more than the reduction launch here (per call, this /
+// matmul_reg):
 // 8192 x 8192, batch 256: F16 93 / 101 us, F32 123 / 142; batch 127: 57 / 58,
 // 81 / 88; 4096 x 4096, batch 512: 54 / 56, 69 / 72; batch 256 (below the
 // line): 33.6 / 31.5, 41.8 / 41.2.
@@ -847,8 +848,9 @@ __global__ __launch_bounds__(256) void reduce_splits(const float *__restrict__ p
 // Up to 8 batch rows share one 16-column operand: column b holds row b's hi
 // half, column 8 + b its lo half, and the two sums are added at the end.
 //
-// Batch 1, per call: 4096 x 4096 Q4_0 35.1 -> 5.2 us, F16 32.6 -> 7.6 (4.4 TB/s
-// of weights; an empty kernel called the same way takes 4.2); 8192 x 8192
+// Batch 1, per call: 4096 x 4096 Q4_0 35.1 -> 5.2 us over one matrix again and
+// again and 5.7 in a run of 32 matrices, F16 32.6 -> 7.6 (4.4 TB/s of weights;
+// an empty kernel called the same way takes 4.2); 8192 x 8192
 // Q4_0 63 -> 13.8, F16 59 -> 22.8 (5.9 TB/s).  Batch 16, 4096 x 4096: Q4_0
 // 35.4 -> 9.7, F32 41.8 -> 15.6.  (Before: x padded to 64 rows and split in a
 // launch of its own, then 64 x 64 tiles on 64 workgroups.)  Above 16 rows the

@@ -754,8 +754,8 @@ int gi_paged_rope_decode_step(gi_paged *h, int layer, int batch, int num_heads, 
     if (batch == 0)
         return GI_OK;
     std::lock_guard<std::mutex> g(h->mu);
-    // RoPE and the store go into the decode launch where they fit
-    // (decode_fuses_append, decode_fuses_rope), else into a launch before it
+    // RoPE and the store go into the decode launch (decode_fuses_rope) or into
+    // a launch before it
     return decode_locked(h, layer, batch, num_heads, q, out, block_tables, max_blocks, seq_lens, max_seq_len, scale,
                          nullptr, 0, k, v, q);
 }

@@ -275,7 +275,13 @@ int gi_paged_gather(gi_paged *h, int layer, const int32_t *block_table, int n_to
  * the fewer splits where the workspace holds no more, and fails with
  * GI_ERR_BAD_ARG where it does not hold those either (make one eager call with
  * the same shape first); once any call has been captured, growth keeps the old
- * buffers alive until gi_paged_destroy, so captured graphs stay valid. */
+ * buffers alive until gi_paged_destroy, so captured graphs stay valid.  A plan
+ * of one split (gi_attention_plan.decode_splits) uses no workspace; all others
+ * of a handle share it, so replays of captured split calls (of the steps below
+ * too) that could overlap each other or an eager split call of the handle must
+ * be serialised.  Outputs of different plans agree within rounding: a call
+ * captured before the workspace exists, and one made on a full device, may
+ * differ from the same call made otherwise in the last bits. */
 int gi_paged_decode_attention(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                               float *out, const int32_t *block_tables, int max_blocks,
                               const int32_t *seq_lens, int max_seq_len, float scale);
@@ -298,7 +304,8 @@ int gi_paged_decode_attention(gi_paged *h, int layer, int batch, int num_heads, 
  * first gi_paged_create there).  A stream that is capturing a graph neither
  * waits nor records, so replays of captured calls that could overlap other
  * users of the array on the device (other streams) race: serialise them.
- * Same arguments and results as gi_paged_decode_attention. */
+ * Same arguments as gi_paged_decode_attention and the same results within
+ * rounding (the same bits where the plan's partials fit the array). */
 int gi_paged_decode_attention_noalloc(gi_paged *h, int layer, int batch, int num_heads, const float *q,
                                       float *out, const int32_t *block_tables, int max_blocks,
                                       const int32_t *seq_lens, int max_seq_len, float scale);
@@ -394,7 +401,9 @@ typedef struct gi_attention_plan {
     int decode_split_tokens; /* tokens per split (the last runs to the end) */
     int decode_waves;        /* waves per matrix-core workgroup (4 or 8) */
     int decode_step_fused;   /* gi_paged_decode_step stores the token inside
-                                the decode launch (else an append launch) */
+                                the decode launch (else an append launch);
+                                gi_paged_rope_decode_step follows a rule of
+                                its own, which this does not report */
     int prefill_kernel;      /* 0 vector ALU, 1 matrix core */
     int prefill_fallback;    /* as decode_fallback, for prefill */
 } gi_attention_plan;
