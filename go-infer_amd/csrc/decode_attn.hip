@@ -448,12 +448,14 @@ static void set_plan(const PoolLayout &L, int max_len, int splits, int *split_to
 //    288 pairs: f16 150 -> 125, q4_0 76 -> 57, f32 310 -> 248, q8_0 85 -> 81;
 //    384 pairs, 1500-6500 tokens: f16 157 -> 140, q4_0 87 -> 71, f32 298 ->
 //    268, but q8_0 at 5000 tokens 95 -> 106, which stays unsplit; at 1500
-//    tokens splits lose everywhere;
+//    tokens splits lose everywhere, so only the caller's word for the longest
+//    sequence is taken here, not the width of the tables (40 x 600 tokens under
+//    tables of 4096: f16 23.0 -> 31.2, q4_0 19.0 -> 28.8);
 //  - from two pairs per CU on the launch has enough rounds to even out: 480
 //    and 640 pairs are fastest unsplit.
 constexpr int kDecodeMinSplit = 128;
 
-void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, int num_cus,
+void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, bool bound_only, int num_cus,
                  int *split_tokens, int *num_splits)
 {
     (void)num_heads;
@@ -474,7 +476,7 @@ void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, int
     } else if (pairs < cus) {
         s = single || max_len <= 1024 ? 1 : 2 * cus / pairs;
         min_split = 512;
-    } else if (pairs > cus && pairs < 2 * cus) {
+    } else if (pairs > cus && pairs < 2 * cus && !bound_only) {
         if (pairs * 4 <= 5 * cus && max_len >= 4096)
             s = 5;
         else if (pairs * 16 <= 25 * cus && max_len >= 2560 && L.kv_type != KV_Q8_0)

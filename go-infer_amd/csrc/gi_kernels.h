@@ -99,8 +99,9 @@ bool decode_fuses_rope(const PoolLayout &L, int batch, int num_heads, int reques
                        int split_tokens, int num_splits, int num_cus);
 
 // Picks (split_tokens, num_splits) for a batch whose longest sequence has
-// max_len tokens, so the grid fills the device.
-void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, int num_cus,
+// max_len tokens, so the grid fills the device.  bound_only: max_len is not the
+// caller's word but only what the block tables map.
+void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, bool bound_only, int num_cus,
                  int *split_tokens, int *num_splits);
 
 // The same with longer splits and so less workspace, for callers whose

@@ -586,7 +586,7 @@ static int decode_locked(gi_paged *h, int layer, int batch, int num_heads, const
     const int64_t mapped = (int64_t)max_blocks * h->L.page_tokens;
     const int max_len = (int)(max_seq_len > 0 && max_seq_len < mapped ? max_seq_len
                               : mapped < INT32_MAX ? mapped : INT32_MAX);
-    gi::decode_plan(h->L, batch, num_heads, max_len, h->num_cus, &a.split_tokens, &a.num_splits);
+    gi::decode_plan(h->L, batch, num_heads, max_len, max_seq_len == 0, h->num_cus, &a.split_tokens, &a.num_splits);
     // the workspace first: a call refused here has queued nothing.  Partials
     // that the scratch cannot hold, that a capturing stream cannot allocate or
     // that a full device has no room for: fewer, longer splits may still fit.
@@ -821,7 +821,7 @@ int gi_paged_attention_plan(const gi_paged *h, int batch, int num_heads, int max
     const bool mfma_req = h->decode_kernel != 0;
     r.decode_kernel = gi::decode_kernel_kind(h->L, num_heads, h->decode_kernel);
     r.decode_fallback = mfma_req && r.decode_kernel == 0;
-    gi::decode_plan(h->L, batch, num_heads, max_seq_len > 0 ? max_seq_len : 1, h->num_cus,
+    gi::decode_plan(h->L, batch, num_heads, max_seq_len > 0 ? max_seq_len : 1, false, h->num_cus,
                     &r.decode_split_tokens, &r.decode_splits);
     r.decode_waves = r.decode_kernel == 1 ? gi::decode_waves(h->L, batch, r.decode_splits, h->num_cus) : 0;
     r.decode_step_fused = r.decode_kernel == 1 && gi::decode_fuses_append(h->L, batch, r.decode_splits, h->num_cus);

@@ -260,7 +260,9 @@ int gi_paged_gather(gi_paged *h, int layer, const int32_t *block_table, int n_to
  * means unknown: the longest sequence max_blocks maps) sizes that split
  * plan only: the last split of every sequence runs to its end, so every
  * seq_lens[b] token is attended whatever max_seq_len says (a short hint
- * costs balance, never tokens).  A length below zero or beyond max_blocks *
+ * costs balance, never tokens; one far above the lengths costs splits with
+ * nothing to do, most where batch * num_kv_heads is 1 to 1.6 times the CUs: up
+ * to 10 us a call there).  A length below zero or beyond max_blocks *
  * page_tokens is clamped and reported by gi_synchronize as GI_ERR_BAD_PAGE.
  *
  * Workspace: the handle keeps the partials of split sequences, batch *

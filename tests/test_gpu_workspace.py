@@ -104,3 +104,31 @@ def test_growth_after_a_capture_keeps_the_graph(gi, oracle, dev):
         assert float(rel_err_rows(o2.cpu().numpy(),
                                   oracle.attention_decode(q2h[0], k, v, 2 * H, kvh, hd, n, scale),
                                   2 * H, hd).max()) <= 1e-3, r
+
+
+def test_wide_tables_alone_do_not_split_a_full_device(gi, oracle, dev):
+    """Where (sequence, kv head) pairs fill the CUs 1 to 1.6 times, contexts
+    are cut for a caller that says they are long, not because the tables are
+    wide: without max_seq_len such a call takes no workspace.  Both give the
+    same attention."""
+    import torch
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    H, kvh, hd, P, n, wide = 32, 8, 128, 16, 300, 6000
+    rows = cus * 9 // 8 // kvh
+    pop = Populated(gi, dev, 1, 1, kvh, hd, P, [n], seed=11)
+    bt = torch.zeros(rows, wide // P, dtype=torch.int32, device=dev)
+    bt[:, :pop.max_blocks] = pop.block_tables()
+    sl = torch.full((rows,), n, dtype=torch.int32, device=dev)
+    qd, q = seeded((rows, H * hd), 12, dev)
+    scale = oracle.attn_scale(hd)
+    ks, vs = pop.stored(0, 0)
+    k, v = oracle.widen(1, kvh * hd, ks), oracle.widen(1, kvh * hd, vs)
+    want = oracle.attention_decode(q[rows - 1], k, v, H, kvh, hd, n, scale)
+    out = torch.empty_like(qd)
+    before = _free()
+    for hint, grows in ((0, False), (wide, True)):
+        out.fill_(float("nan"))
+        pop.pool.AttentionGQA(out, qd, 0, bt, sl, H, scale, hint)
+        pop.pool.synchronize()
+        assert (_free() < before) == grows, hint
+        assert float(rel_err_rows(out[rows - 1].cpu().numpy(), want, H, hd).max()) <= 1e-3, hint
