@@ -433,7 +433,11 @@ static void set_plan(const PoolLayout &L, int max_len, int splits, int *split_to
 // CU, rounded up, and at least 1024 tokens per split):
 //  - up to two blocks per wave (four where the pairs themselves use the
 //    CUs), one split: batch 1 x 300 f16 8.6 against 10.0 in splits of 128,
-//    batch 14 x 400-800 (112 pairs) 19.5 against 21.1 in two;
+//    batch 14 x 400-800 (112 pairs) 19.5 against 21.1 in two.  At head
+//    dimension 64 (f32 pages apart) a third round of blocks still costs less
+//    than the merge: batch 4 x 600 f16 9.2 against 9.8, q8_0 10.2 against 11.2
+//    (700: 9.8 / 9.8, 11.7 / 11.2), and f16 with 64 pairs a fourth one: 800
+//    9.9 against 11.0 (900 11.2 / 11.2);
 //  - few (sequence, kv head) pairs: splits of 128 tokens until the CUs are
 //    full.  Batch 1 f16 1000 tokens 16.1 -> 11.1, 6001 18.8 -> 13.5; f32
 //    1000 29.8 -> 13.4; splits of 64 were no faster;
@@ -466,7 +470,10 @@ void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, boo
     const bool single = one_wg_per_cu(L);
     int64_t s = 1;
     int min_split = kDecodeMinSplit;
-    if (pairs < 1 || max_len <= (single ? 256 : pairs * 4 <= cus ? 512 : 1024)) {
+    int whole = single ? 256 : pairs * 4 <= cus ? 512 : 1024;
+    if (L.head_dim == 64 && L.kv_type != KV_F32)
+        whole = max(whole, L.kv_type == KV_F16 && pairs * 8 > cus ? 896 : 640);
+    if (pairs < 1 || max_len <= whole) {
         s = 1;
     } else if (pairs <= cus / 2) {
         s = cus / pairs;

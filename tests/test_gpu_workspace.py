@@ -132,3 +132,15 @@ def test_wide_tables_alone_do_not_split_a_full_device(gi, oracle, dev):
         pop.pool.synchronize()
         assert (_free() < before) == grows, hint
         assert float(rel_err_rows(out[rows - 1].cpu().numpy(), want, H, hd).max()) <= 1e-3, hint
+
+
+def test_short_contexts_at_head_dimension_64_stay_whole(gi, dev):
+    """A third round of 256-token blocks costs less than a merge there."""
+    import torch
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the shapes are worked out for a 256-CU device")
+    for kv_type, batch, whole in ((1, 1, 640), (1, 8, 640), (1, 16, 896), (2, 16, 640), (3, 4, 640), (0, 4, 512)):
+        pool = gi.PagedKVCache(1, 4, 64, 16, 1, kv_type)
+        assert pool.attention_plan(batch, 32, whole)["decode_splits"] == 1, (kv_type, batch)
+        assert pool.attention_plan(batch, 32, whole + 1)["decode_splits"] > 1, (kv_type, batch)
+        pool.close()
