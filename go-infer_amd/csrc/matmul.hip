@@ -574,15 +574,40 @@ __global__ __launch_bounds__(64 * kRegWaves) void matmul_reg(MatArgs a, int batc
 #endif
 }
 
-// Tile shapes: 32 columns to batch 32, else 64; as many rows (16, 32 or 64)
-// as leave about one workgroup per CU.
+// Tile shapes: 32 columns to batch 32, else 64, and the rows (16, 32 or 64)
+// whose rounds of one workgroup per CU cost least: a tile of 64 rows takes 1.6
+// and one of 32 rows 1.2 times as long as one of 16 (4096 x 4096 Q8_0 batch 256
+// 28 us in 256 tiles of 64, batch 128 20 in 256 of 32; 2048 x 2048 17.7, 13.8
+// and 11.9).  By the most rows that still gave each CU a workgroup, 1.5 rounds
+// were common: 2048 x 2048, batch 192, F32 20.5 -> 15.5, Q8_0 18.2 -> 13.5; 4096 x
+// 4096, batch 160, Q8_0 34.1 -> 27.7.
+struct RegTiles {
+    int ct, rt, tiles;
+    RegTiles(int rows, int batch) : ct(batch <= 32 ? 2 : 4)
+    {
+        const int bts = (batch + 16 * ct - 1) / (16 * ct);
+        int64_t best = INT64_MAX;
+        for (const int r : {4, 2, 1}) {
+            const int n = (rows + 16 * r - 1) / (16 * r) * bts;
+            const int64_t cost = (int64_t)rounds(n) * (r == 4 ? 8 : r == 2 ? 6 : 5);
+            if (cost < best) {
+                best = cost;
+                rt = r;
+                tiles = n;
+            }
+        }
+    }
+    static int rounds(int n) { return (n + kRegWorkgroups - 1) / kRegWorkgroups; }
+    // a quarter or more of the last rounds' workgroups missing
+    bool uneven() const { return 4 * (int64_t)tiles <= 3 * (int64_t)rounds(tiles) * kRegWorkgroups; }
+};
+
 template <int WT>
 void launch_reg(const MatArgs &a, int batch_pad, hipStream_t st)
 {
-    const int ct = a.batch <= 32 ? 2 : 4, bts = (a.batch + 16 * ct - 1) / (16 * ct);
-    auto tiles = [&](int rt) { return (a.rows + 16 * rt - 1) / (16 * rt) * bts; };
-    const int rt = tiles(4) >= kRegWorkgroups ? 4 : tiles(2) >= kRegWorkgroups ? 2 : 1;
-    const dim3 grid((unsigned)((tiles(rt) + 7) / 8 * 8)), block(64 * kRegWaves);
+    const RegTiles t(a.rows, a.batch);
+    const int ct = t.ct, rt = t.rt;
+    const dim3 grid((unsigned)((t.tiles + 7) / 8 * 8)), block(64 * kRegWaves);
 #define GI_REG(RT, CT) hipLaunchKernelGGL((matmul_reg<WT, RT, CT>), grid, block, 0, st, a, batch_pad)
     if (ct == 2) {
         if (rt == 4)
@@ -634,7 +659,13 @@ struct SKArgs {
 // 8192 x 8192, batch 256: F16 93 / 101 us, F32 123 / 142; batch 127: 57 / 58,
 // 81 / 88; 4096 x 4096, batch 512: 54 / 56, 69 / 72; batch 256 (below the
 // line): 33.6 / 31.5, 41.8 / 41.2.
+// From a quarter of that up it is taken at batches over 64 where matmul_reg's
+// tiles leave a quarter of the CUs idle (4096 x 4096, batch 160: F16 28.4 / 39,
+// F32 34.4 / 51; batch 320: 40.8 / 52, 60.9 / 70.4; F32 384 73 / 70), and for F32
+// rows of 4096 columns and more, which matmul_reg reads in two planes (batch 65
+// 28.9 / 30.7, 200 40.0 / 40.6; 2048 columns, batch 512: 28.3 / 22.3).
 constexpr int kSplitKWorkgroups = 256, kMinSliceSteps = 4, kSplitKMinSteps = 65536;
+constexpr int kSplitKF32Steps = 128; // 4096 columns
 
 template <int WT>
 __global__ __launch_bounds__(256) void matmul_sk(SKArgs s)
@@ -1197,7 +1228,8 @@ int gi_matmul_batch(gi_weights *w, int batch, const float *x, float *y)
     const size_t nx = (size_t)batch_pad * w->cols * 2;
     const int KS = w->cols / 32;
     const int64_t tiles64 = (int64_t)((w->rows + 63) / 64) * (batch_pad / 64);
-    const bool sk = (w->type == W_F16 || w->type == W_F32) && tiles64 * KS >= kSplitKMinSteps;
+    const bool early = batch > 64 && (RegTiles(w->rows, batch).uneven() || (w->type == W_F32 && KS >= kSplitKF32Steps));
+    const bool sk = (w->type == W_F16 || w->type == W_F32) && tiles64 * KS >= kSplitKMinSteps / (early ? 4 : 1);
     int splits = 1, ks_per = KS;
     if (sk) {
         const int tiles = (rows_pad / 128) * ((batch_pad + 127) / 128);

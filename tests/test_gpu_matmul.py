@@ -152,6 +152,15 @@ def test_matmul_form_edges(gi, oracle, dev, t, rows, cols, batch):
     assert float((np.abs(got - exact) / bound).max()) <= 1.0
 
 
+# Row tiles of 32 by each column width (rows that leave them one round of the
+# 256 workgroups), of 64 where tiles of 32 would take a second round, and a
+# product whose uneven tiles send F16 and F32 weights to the split-K form.
+@pytest.mark.parametrize("t", [0, 1, 2, 8], ids=["f32", "f16", "q4_0", "q8_0"])
+@pytest.mark.parametrize("rows,cols,batch", [(8190, 64, 17), (4090, 96, 70), (2050, 96, 130), (4090, 2752, 130)])
+def test_matmul_row_tiles(gi, oracle, dev, t, rows, cols, batch):
+    test_matmul_form_edges(gi, oracle, dev, t, rows, cols, batch)
+
+
 # Split-K at its own edges (F16 and F32 weights of 65536 and more 64 x 64 tiles
 # times k-steps): one slice, stored without a reduction, of rows that are no
 # multiple of 4; two slices of 73 and 72 k-steps whose reduction ends in a
