@@ -1407,14 +1407,14 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     // token is not ordered with this one.  So a wave whose blocks hold a page
     // that another row writes stores that row's token too: the same bytes as
     // its owner, visible to this wave's own loads once the stores have
-    // completed.  Lane i holds the page that row r0 + i writes (row_page);
-    // the pages of the wave's blocks (own_page, one per 16 tokens) go into a
-    // hash of 1024 bits in LDS, and what it lets through is compared exactly.
-    // The first 64 of both are requested before the first block (row_page
-    // depends on lens, requested with this row's length) and looked at while
-    // the block and q are in flight: +0.5 us for 64 x 1500-3000 q4_0 and q8_0,
-    // nothing for f16 and f32 (after q's loads had returned, 32 compares of
-    // one page each: +1.5 to 2.5).
+    // completed.  Lane i holds the page that row r0 + i writes (row_page), and
+    // is compared with the page of each 16 tokens of the wave's blocks
+    // (own_page).  The first 64 of both are requested before the first block
+    // (row_page depends on lens, requested with this row's length) and
+    // compared in straight-line code while that block and q are in flight: in
+    // the loop over more of them each wait is for every load.  us a step,
+    // without / with: 48 x 1500-6500 q4_0 73 / 74, 32 x 512-4096 f16 62.4 / 61.6,
+    // 2 to 48 x 200 2 to 4 % more (all of it in the loop: 4 to 7 %), 1500 0 to 1.5.
     auto row_page = [&](int r0, int len_) { // of row r0 + lane, whose length is len_
         const int row = min(r0 + lane, a.batch - 1), at = min(max(len_ - 1, 0), a.max_blocks * P - 1);
         return a.block_tables[(int64_t)row * a.max_blocks + at / P];
@@ -1422,7 +1422,37 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     auto own_page = [&](int t) { // of the lane's 16 tokens of the 32 blocks from t
         return bt[min(t + stride * (lane >> 1) + 16 * (lane & 1), t1 - 1) / P];
     };
-    volatile uint32_t *seen = reinterpret_cast<volatile uint32_t *>(s_ml[0][w]);
+    volatile uint32_t *seen = reinterpret_cast<volatile uint32_t *>(s_ml[0][w]); // before the merge uses it
+    // rows of r0 .. r0 + 63 whose page is one of the 32 blocks' from t (groups
+    // past t1 repeat the last page)
+    auto meet = [&](int r0, int len_, int page, int t, int id) -> uint64_t {
+        const int row = r0 + lane, at = len_ - 1, n = min(64, 2 * ((t1 - t + stride - 1) / stride));
+        const bool live = row < a.batch && row != b && at >= 0 && at < a.max_blocks * P &&
+                          (!ROPE || at < a.rope_max_pos) && page >= 0 && page < L.num_pages;
+        uint64_t hit = 0;
+        if (n <= 16) {
+            for (int i = 0; i < n; i += 2)
+#pragma unroll
+                for (int x = 0; x < 2; x++)
+                    hit |= __ballot(page == __builtin_amdgcn_readlane(id, i + x));
+            return hit & __ballot(live);
+        }
+        // more: as bits of a hash of 1024 in LDS, then what it lets through
+        auto bits = [&](int x) { return seen + ((x >> 9) & 1) * (NW * 16) + ((x >> 5) & 15); };
+        if (lane < 32)
+            *bits(lane << 5) = 0;
+        __builtin_amdgcn_wave_barrier();
+        __hip_atomic_fetch_or(bits(id), 1u << (id & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __builtin_amdgcn_wave_barrier();
+        uint64_t may = __ballot(live && (*bits(page) >> (page & 31) & 1));
+        __builtin_amdgcn_wave_barrier();
+        for (; __builtin_expect(may != 0, 0); may &= may - 1) {
+            const int i = __builtin_ctzll(may);
+            if (__ballot(id == __builtin_amdgcn_readlane(page, i)))
+                hit |= 1ull << i;
+        }
+        return hit;
+    };
     int rows_pg = 0, own_pg = 0;
     auto look = [&]() {
         if (rows_meet) {
@@ -1435,39 +1465,18 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     auto share_tokens = [&]() {
         if (!rows_meet)
             return false;
+        uint64_t hit = meet(0, lens, rows_pg, base, own_pg);
+        if (__builtin_expect(hit == 0 && a.batch <= 64 && t1 - base <= 32 * stride, 1))
+            return false;
         bool any = false;
         int len_ = lens, page = rows_pg;
         for (int r0 = 0;;) {
-            const int row = r0 + lane, at = len_ - 1;
-            const bool live = row < a.batch && row != b && at >= 0 && at < a.max_blocks * P &&
-                              (!ROPE || at < a.rope_max_pos) && page >= 0 && page < L.num_pages;
-            uint64_t hit = 0;
-            int id = own_pg;
-            for (int t = base;;) {
-                // the groups' pages as bits of a hash (groups past t1 repeat
-                // the last page), then the exact look at what it lets through
-                auto bits = [&](int x) { return seen + ((x >> 9) & 1) * (NW * 16) + ((x >> 5) & 15); };
-                if (lane < 32)
-                    *bits(lane << 5) = 0;
-                __builtin_amdgcn_wave_barrier();
-                __hip_atomic_fetch_or(bits(id), 1u << (id & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                __builtin_amdgcn_wave_barrier();
-                uint64_t may = __ballot(*bits(page) >> (page & 31) & 1);
-                __builtin_amdgcn_wave_barrier();
-                for (may &= __ballot(live); __builtin_expect(may != 0, 0); may &= may - 1) {
-                    const int i = __builtin_ctzll(may);
-                    if (__ballot(id == __builtin_amdgcn_readlane(page, i)))
-                        hit |= 1ull << i;
-                }
-                t += 32 * stride;
-                if (t >= t1)
-                    break;
-                id = own_page(t);
-            }
+            for (int t = base + (r0 ? 0 : 32 * stride); t < t1; t += 32 * stride)
+                hit |= meet(r0, len_, page, t, own_page(t));
             any |= hit != 0;
             for (; __builtin_expect(hit != 0, 0); hit &= hit - 1) {
                 const int i = __builtin_ctzll(hit);
-                const int pos = __builtin_amdgcn_readlane(at, i);
+                const int pos = __builtin_amdgcn_readlane(len_, i) - 1;
                 const float2 *t = nullptr;
                 if constexpr (ROPE)
                     t = a.rope + (int64_t)pos * (HD / 2);

@@ -11,11 +11,12 @@ pytestmark = pytest.mark.gpu
 
 # H, kvh, hd, P, n, rows: one split and several, eight- and four-wave
 # workgroups, pages whose lines two waves read (64) and that blocks straddle
-# (48), more rows than lanes of a wave, 16 heads per kv head
+# (48), more rows than lanes of a wave, 16 heads per kv head; contexts whose
+# pages go through the hash, and more of them than lanes
 @pytest.mark.parametrize("kv_type", [0, 1, 2, 3], ids=["f32", "f16", "q8_0", "q4_0"])
 @pytest.mark.parametrize("H,kvh,hd,P,n,rows", [
     (32, 8, 128, 16, 45, 5), (32, 8, 128, 32, 700, 4), (32, 4, 64, 64, 100, 3), (16, 2, 64, 16, 20, 70),
-    (32, 8, 128, 16, 30, 40), (16, 1, 128, 48, 200, 6)])
+    (32, 8, 128, 16, 30, 40), (16, 1, 128, 48, 200, 6), (32, 8, 128, 16, 1200, 40), (32, 8, 128, 32, 4200, 52)])
 @pytest.mark.parametrize("rope", [False, True], ids=["step", "rope"])
 def test_rows_of_a_step_see_each_others_tokens(gi, oracle, dev, kv_type, H, kvh, hd, P, n, rows, rope):
     import torch
