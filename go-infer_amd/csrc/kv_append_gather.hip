@@ -600,7 +600,8 @@ __global__ __launch_bounds__(kThreads) void gather_tiles(PoolLayout L, const uin
 }
 
 // Gather one sequence's tokens [0, n_tok) of one layer, element by element:
-// the page sizes and output alignments gather_tiles does not take.
+// the page sizes and output alignments gather_tiles does not take, and short
+// sequences at 4 bytes an element.
 //   widen == 0: stored format, the reference's bytes per token vector
 //               (f32: 4*kv_dim, f16: 2*kv_dim, q8_0: kv_dim/32 blocks of
 //               34 bytes = LE fp16 scale + 32 int8, quant.go:38-41).
@@ -992,10 +993,17 @@ hipError_t launch_gather(const PoolLayout &L, const uint8_t *base, const int32_t
     dim3 grid(grid_for((int64_t)n_tok * per_tok)), block(kThreads);
     uint8_t *ko = (uint8_t *)k_out, *vo = (uint8_t *)v_out;
     // gather_tiles' 16-byte accesses: pages of whole 16-token groups, output
-    // rows on 16-byte (stored quantised blocks: 4-byte) boundaries
+    // rows on 16-byte (stored quantised blocks: 4-byte) boundaries.  Where 4
+    // bytes an element are written, short sequences are too few workgroups of
+    // 32 tokens: element by element below these numbers of elements (us a call,
+    // that / tiles, Llama-3-8B shape: widened fp16 200 tokens 4.6 / 6.6, 600
+    // 5.4 / 7.1, 2000 11.2 / 8.7; widened q8_0 200 4.6 / 5.5, 600 5.9 / 5.8; f32 200
+    // 4.5 / 5.0, 600 5.3 / 5.5, 2000 11.6 / 7.8, TinyLlama shape 2000 5.4 / 4.7).
+    const int64_t tiles_from = !widen && L.kv_type != KV_F32 ? 0 : L.kv_type == KV_F16 ? 1 << 20 : 3 << 17;
     const uintptr_t mask = ((L.kv_type == KV_Q8_0 || L.kv_type == KV_Q4_0) && !widen) ? 3 : 15;
-    if (L.page_tokens % 16 == 0 && (L.head_dim == 64 || L.head_dim == 128) &&
-        (((uintptr_t)k_out | (uintptr_t)v_out) & mask) == 0 && L.num_kv_heads <= 65535) {
+    if ((int64_t)n_tok * kv_dim >= tiles_from && L.page_tokens % 16 == 0 &&
+        (L.head_dim == 64 || L.head_dim == 128) && (((uintptr_t)k_out | (uintptr_t)v_out) & mask) == 0 &&
+        L.num_kv_heads <= 65535) {
         const dim3 tg((unsigned)((n_tok + kGatherTok - 1) / kGatherTok), (unsigned)L.num_kv_heads);
 #define GI_TILES(KT, W)                                                                                            \
     do {                                                                                                           \

@@ -242,3 +242,23 @@ def test_gather_tile_edges(gi, oracle, dev, kv_type, kvh, hd, P):
             want = st[:n] if not widen else oracle.widen(kv_type, kv_dim, st[:n]).view(np.uint8)
             assert np.array_equal(row[shift:shift + n * bytes_per].reshape(n, -1), want.reshape(n, -1)), (widen, shift)
             assert (row[:shift] == 0xA5).all() and (row[shift + n * bytes_per:] == 0xA5).all()
+
+
+@pytest.mark.parametrize("kv_type", [0, 1, 2, 3], ids=["f32", "f16", "q8_0", "q4_0"])
+@pytest.mark.parametrize("kvh,hd,P,lens", [(8, 128, 16, (1024, 1041, 1060)), (4, 64, 48, (4096, 4127)),
+                                           (16, 128, 32, (180, 191, 193, 300, 511, 513))])
+def test_gather_tiles_of_float_elements(gi, oracle, dev, kv_type, kvh, hd, P, lens):
+    """Float32 elements, stored or widened, take the tiles from 393,216 (fp16:
+    1,048,576) elements on: token counts there around their 16-token groups and
+    32-token tiles, and below that."""
+    import torch
+    kv_dim = kvh * hd
+    pop = Populated(gi, dev, kv_type, 1, kvh, hd, P, [max(lens)], seed=19, specials=True)
+    ks, vs = pop.stored(0, 0)
+    t = torch.from_numpy(pop.table(0)).to(dev)
+    for n in lens:
+        for got, st in zip(pop.pool.Get(0, t, n, widen=True), (ks, vs)):
+            want = oracle.widen(kv_type, kv_dim, st[:n])
+            assert np.array_equal(got.cpu().numpy().view(np.uint32), want.view(np.uint32)), n
+        for got, st in zip(pop.pool.Get(0, t, n), (ks, vs)):
+            assert np.array_equal(got.cpu().numpy(), st[:n]), n
