@@ -916,8 +916,11 @@ hipError_t launch_append_at_len(const PoolLayout &L, uint8_t *base, int batch,
 // give.  us a call, rope_append / rows: Llama-3-8B shape fp16 512 tokens 8.5 /
 // 7.7, 1024 13.7 / 10.2, 2048 24.0 / 16.4, f32 2048 31.3 / 17.3, q8_0 300 9.9 /
 // 10.7; TinyLlama shape f32 300 tokens with the attention behind it 24.8 /
-// 25.4, 2048 tokens 13.7 / 8.6.
+// 25.4, 2048 tokens 13.7 / 8.6.  And fp16 and q8_0 chunks from kRopeRowsTok
+// tokens only: Llama-3-70B shape fp16 256 7.1 / 7.7, 512 10.7 / 9.1, q8_0 300
+// 10.4 / 11.4, 512 11.5 / 11.5 (f32 256 7.6 / 6.6, q4_0 9.7 / 8.9).
 constexpr int64_t kRopeRowsMin = 512 * 4096;
+constexpr int kRopeRowsTok = 512;
 
 hipError_t launch_rope_append(const PoolLayout &L, uint8_t *base, int n_tok, const int32_t *block_ids,
                               const int32_t *slots, const int32_t *block_tables, int max_blocks,
@@ -932,7 +935,9 @@ hipError_t launch_rope_append(const PoolLayout &L, uint8_t *base, int n_tok, con
     // a chunk: whole rows, where 16-byte accesses and groups of 4 pairs fit
     const uintptr_t ptrs = (uintptr_t)k | (uintptr_t)v | (uintptr_t)R.q | (uintptr_t)R.q_out | (uintptr_t)R.table;
     const int64_t elems = (int64_t)n_tok * std::max(R.num_heads, 4 * L.num_kv_heads) * L.head_dim;
-    if (!at_len && elems >= kRopeRowsMin && ptrs % 16 == 0 && R.rope_half % 4 == 0 && L.head_dim % 32 == 0 &&
+    const bool enough = elems >= kRopeRowsMin &&
+                        (n_tok >= kRopeRowsTok || L.kv_type == KV_F32 || L.kv_type == KV_Q4_0);
+    if (!at_len && enough && ptrs % 16 == 0 && R.rope_half % 4 == 0 && L.head_dim % 32 == 0 &&
         L.head_dim <= kRowMaxHd) {
         const int per = R.rope_half / 4 + (L.head_dim - 2 * R.rope_half) / 4;
         const int64_t qb = ((int64_t)kRowTok * R.num_heads * per + kThreads - 1) / kThreads;
