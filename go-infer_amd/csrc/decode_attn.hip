@@ -451,7 +451,10 @@ static void set_plan(const PoolLayout &L, int max_len, int splits, int *split_to
 //    half two; 5 or 3 splits even that out on long sequences.  5000 tokens,
 //    288 pairs: f16 150 -> 125, q4_0 76 -> 57, f32 310 -> 248, q8_0 85 -> 81;
 //    384 pairs, 1500-6500 tokens: f16 157 -> 140, q4_0 87 -> 71, f32 298 ->
-//    268, but q8_0 at 5000 tokens 95 -> 106, which stays unsplit; at 1500
+//    268, but q8_0 at 5000 tokens 95 -> 106, which stays unsplit, as does q8_0
+//    from 9/8 pairs per CU (320 pairs, 4200 tokens 0.93 of the speed, 264 1.03);
+//    equal lengths of 2600 to 4000 over 1.25 pairs per CU lose 2 to 5 % on f16
+//    and f32 (q4_0 gains 0 to 9 %), from 4200 on they are even; at 1500
 //    tokens splits lose everywhere, so only the caller's word for the longest
 //    sequence is taken here, not the width of the tables (40 x 600 tokens under
 //    tables of 4096: f16 23.0 -> 31.2, q4_0 19.0 -> 28.8);
@@ -484,9 +487,10 @@ void decode_plan(const PoolLayout &L, int batch, int num_heads, int max_len, boo
         s = single || max_len <= 1024 ? 1 : 2 * cus / pairs;
         min_split = 512;
     } else if (pairs > cus && pairs < 2 * cus && !bound_only) {
-        if (pairs * 4 <= 5 * cus && max_len >= 4096)
+        const bool near = pairs * 4 <= 5 * cus, q8 = L.kv_type == KV_Q8_0;
+        if (near && max_len >= 4096 && (!q8 || pairs * 8 <= 9 * cus))
             s = 5;
-        else if (pairs * 16 <= 25 * cus && max_len >= 2560 && L.kv_type != KV_Q8_0)
+        else if (pairs * 16 <= 25 * cus && !q8 && max_len >= (near || L.kv_type == KV_Q4_0 ? 2560 : 4096))
             s = 3;
     }
     set_plan(L, max_len, (int)min(s, (int64_t)(max_len + min_split - 1) / min_split), split_tokens, num_splits);
